@@ -12,9 +12,10 @@
 // window are wave-uniform and independent of the time tile: they are
 // tabulated once per plan, a block's offsets sit 16 per VGPR, and one trial
 // costs one DPP-broadcast address add for K LDS reads (issued in pairs as
-// ds_read2st64).  The adds are bound by
-// LDS read bandwidth (~128 B/clk/CU), not by HBM, so the storage formats
-// trade LDS bytes per add:
+// ds_read2st64).  These adds are bound by LDS reads, not by HBM, so the
+// storage formats trade LDS bytes per add; the register-window tiles (the
+// defaults of F32 and F16) read a word once per wave instead of once per
+// trial and are bound by instruction issue:
 //   F32  4 B per add: one float per LDS word, staged by direct buffer->LDS
 //        loads (buffer_load_dword ... lds) that use no data VGPRs.
 //   F16  2 B per add: LDS words hold pairs of consecutive samples in two
@@ -274,6 +275,360 @@ struct F32Tile {
     }
   }
 };
+
+// ================================================== register-window tiles
+// Tiles that read each LDS word once per wave and channel instead of once
+// per trial.  A lane owns K = 20 CONSECUTIVE samples, so the words that the
+// wave's MW = 4 trials need of one channel are one window of
+// K + (D[last] - D[first]) FP32 words per lane.  It is read with
+// ds_read_b128 (80-byte lane stride: the 8 lanes of a group cover all 32
+// banks once) into fixed VGPRs, and a trial adds its K words with K plain
+// v_add_f32, which this GPU issues at about 64 T lane-adds/s where
+// v_fma_mix_f32, the packed 16-bit adds and any add in VGPR index mode reach
+// 33-37 T (measured).  Registers cannot be indexed at that rate, so the adds
+// exist once per trial and word offset (4 x 17 blocks of 20 adds, 6.4 KB of
+// code) and the wave jumps from block to block: the plan's table holds, per
+// channel and trial, the offset of the trial's block inside that code.
+//
+// Table entry of a channel and wave, 8 words: d[i] is the code offset of
+// trial i's block, or of a reading stub when trial i needs another window (i
+// = 0 always); e[i] then holds the block's code offset (low half) and the
+// window's LDS byte offset / 16 (high half).  The stubs differ in how many
+// 16-byte reads they make.
+//
+// Bound: instruction issue.  1024 channels x 4096 trials x 2^17 samples, F32:
+// 34.6 T adds/s (18.5 with one LDS read per add), the VALU at 50 % of the 64 T
+// it issues, LDS reads under a third of their rate; one wave issues at most
+// one instruction per about 5 clocks, so 4 waves per SIMD (128 VGPRs) set
+// MW * K + WIN, and K = 20 at MW = 4 the fewest jumps (49 T without staging
+// and tables; MW = 8, K = 12 at 3 waves 41 T).
+//
+// F16 and U8 rows are widened to FP32 in LDS by one pass per channel block
+// (exact; 32 trials share it), so all storage types run the same adds: F16
+// in FP32 channel order, U8 as exact integers (at most 65536 * 255 < 2^24).
+struct WindowCode {
+  static constexpr int MW = 4, K = 20, WAVES = 8;
+  static constexpr int WIN = 36;                  // window words, VGPRs 92..127
+  static constexpr int NV = WIN - K + 1;          // word offsets of a trial
+  static constexpr int BLOCK = 96;                // code bytes per block, per stub
+  static constexpr int STUB = 128, MINREADS = 6, STUBS = 4;
+  static constexpr int STUB0 = MW * NV * BLOCK;   // stubs follow the blocks
+  static constexpr int BYTES = STUB0 + MW * STUBS * STUB;
+  static_assert(STUB0 % STUB == 0 && BYTES < 65536, "code offsets are 16 bits");
+  static_assert(4 * (MINREADS + STUBS - 1) == WIN && 4 * MINREADS >= K + 3, "reads of a window");
+  static_assert(MW == 4 && NV == 17 && BLOCK == 96 && STUBS == 4 && STUB == 128, "add_channel's text");
+  typedef uint32_t u32x8 __attribute__((ext_vector_type(8)));
+  typedef __attribute__((address_space(4))) const u32x8 const_u32x8;
+
+  // The entry of a channel whose trials read from LDS byte offsets
+  // o[0] <= o[1] <= o[2] <= o[3] (a trial stays in the open window while its
+  // words lie inside WIN).
+  __device__ static void entry(const uint32_t o[MW], uint32_t *out) {
+    uint32_t base = 0, rd[MW], idx[MW];
+    int open = -1;
+    for (int i = 0; i < MW; ++i) {
+      rd[i] = 0;
+      if (open < 0 || (o[i] - base) / 4u > (uint32_t)(NV - 1)) {
+        base = o[i] & ~15u;
+        open = i;
+      }
+      idx[i] = (o[i] - base) / 4u;
+      rd[open] = max((uint32_t)MINREADS, (idx[i] + K + 3u) / 4u);
+    }
+    for (int i = 0; i < MW; ++i) {
+      const uint32_t blk = ((uint32_t)i * NV + idx[i]) * BLOCK;
+      out[i] = rd[i] ? (uint32_t)STUB0 + ((uint32_t)i * STUBS + rd[i] - MINREADS) * STUB : blk;
+      out[MW + i] = rd[i] ? blk | ((o[i] & ~15u) >> 4 << 16) : 0u;
+    }
+  }
+
+  // The adds of one channel: window reads, blocks and the jumps between them;
+  // returns the entry at `next`, loaded while the adds run (the scalar loads
+  // share the LDS reads' wait counter, so it is asked for after those came)
+  // (s[96:97]: address of the code, s[98:99]: jump target).  The .org
+  // directives place every block and stub (and fail to assemble where one is
+  // too long).
+#define MDSM_WIN_ADD(i, j) "v_add_f32 %[x" #i "_" #j "], v[92+" #j "+\\v], %[x" #i "_" #j "]\n\t"
+#define MDSM_WIN_ADDS(i)                                                                        \
+  MDSM_WIN_ADD(i, 0) MDSM_WIN_ADD(i, 1) MDSM_WIN_ADD(i, 2) MDSM_WIN_ADD(i, 3) MDSM_WIN_ADD(i, 4) \
+  MDSM_WIN_ADD(i, 5) MDSM_WIN_ADD(i, 6) MDSM_WIN_ADD(i, 7) MDSM_WIN_ADD(i, 8) MDSM_WIN_ADD(i, 9) \
+  MDSM_WIN_ADD(i, 10) MDSM_WIN_ADD(i, 11) MDSM_WIN_ADD(i, 12) MDSM_WIN_ADD(i, 13)               \
+  MDSM_WIN_ADD(i, 14) MDSM_WIN_ADD(i, 15) MDSM_WIN_ADD(i, 16) MDSM_WIN_ADD(i, 17)               \
+  MDSM_WIN_ADD(i, 18) MDSM_WIN_ADD(i, 19)
+#define MDSM_WIN_JUMP(d) \
+  "s_add_u32 s98, s96, " d "\n\ts_addc_u32 s99, s97, 0\n\ts_setpc_b64 s[98:99]\n\t"
+#define MDSM_WIN_BLOCKS(i, next)                                                                \
+  ".irp v,0,1,2,3,4,5,6,7,8,9,10,11,12,13,14,15,16\n\t" MDSM_WIN_ADDS(i) next                   \
+  ".org .Lmdsm_code%=+(" #i "*17+\\v+1)*96\n\t.endr\n\t"
+#define MDSM_WIN_STUB(i, n, reads, more)                                                                 \
+  "s_lshr_b32 s98, %[e" #i "], 16\n\tv_lshl_add_u32 %[av], s98, 4, %[cur]\n\t"                   \
+  ".irp q," reads "\n\tds_read_b128 v[92+4*\\q:95+4*\\q], %[av] offset:16*\\q\n\t.endr\n\t"      \
+  "s_and_b32 s98, %[e" #i "], 0xffff\n\ts_add_u32 s98, s96, s98\n\ts_addc_u32 s99, s97, 0\n\t"   \
+  "s_waitcnt lgkmcnt(0)\n\t" more "s_setpc_b64 s[98:99]\n\t"                                    \
+  ".org .Lmdsm_code%=+4*17*96+(" #i "*4+" #n "+1)*128\n\t"
+#define MDSM_WIN_STUBS(i, more)                                                                 \
+  MDSM_WIN_STUB(i, 0, "0,1,2,3,4,5", more) MDSM_WIN_STUB(i, 1, "0,1,2,3,4,5,6", more)           \
+  MDSM_WIN_STUB(i, 2, "0,1,2,3,4,5,6,7", more) MDSM_WIN_STUB(i, 3, "0,1,2,3,4,5,6,7,8", more)
+#define MDSM_WIN_ACC(i)                                                                         \
+  [x##i##_0] "+v"(acc[i][0]), [x##i##_1] "+v"(acc[i][1]), [x##i##_2] "+v"(acc[i][2]),            \
+      [x##i##_3] "+v"(acc[i][3]), [x##i##_4] "+v"(acc[i][4]), [x##i##_5] "+v"(acc[i][5]),        \
+      [x##i##_6] "+v"(acc[i][6]), [x##i##_7] "+v"(acc[i][7]), [x##i##_8] "+v"(acc[i][8]),        \
+      [x##i##_9] "+v"(acc[i][9]), [x##i##_10] "+v"(acc[i][10]), [x##i##_11] "+v"(acc[i][11]),    \
+      [x##i##_12] "+v"(acc[i][12]), [x##i##_13] "+v"(acc[i][13]), [x##i##_14] "+v"(acc[i][14]),  \
+      [x##i##_15] "+v"(acc[i][15]), [x##i##_16] "+v"(acc[i][16]), [x##i##_17] "+v"(acc[i][17]),  \
+      [x##i##_18] "+v"(acc[i][18]), [x##i##_19] "+v"(acc[i][19])
+  __device__ __forceinline__ static u32x8 add_channel(float (&acc)[MW][K], uint32_t cur, u32x8 t,
+                                                      const_u32x8 *next) {
+    uint32_t av;
+    u32x8 tn;
+    asm volatile(
+        "s_getpc_b64 s[96:97]\n.Lmdsm_pc%=:\n\t"
+        "s_add_u32 s96, s96, .Lmdsm_code%=-.Lmdsm_pc%=\n\ts_addc_u32 s97, s97, 0\n\t"
+        MDSM_WIN_JUMP("%[d0]")
+        ".p2align 7\n.Lmdsm_code%=:\n\t"
+        MDSM_WIN_BLOCKS(0, MDSM_WIN_JUMP("%[d1]"))
+        MDSM_WIN_BLOCKS(1, MDSM_WIN_JUMP("%[d2]"))
+        MDSM_WIN_BLOCKS(2, MDSM_WIN_JUMP("%[d3]"))
+        MDSM_WIN_BLOCKS(3, "s_branch .Lmdsm_end%=\n\t")
+        MDSM_WIN_STUBS(0, "s_load_dwordx8 %[tn], %[next], 0x0\n\t")
+        MDSM_WIN_STUBS(1, "") MDSM_WIN_STUBS(2, "") MDSM_WIN_STUBS(3, "")
+        ".Lmdsm_end%=:\n\ts_waitcnt lgkmcnt(0)"
+        : MDSM_WIN_ACC(0), MDSM_WIN_ACC(1), MDSM_WIN_ACC(2), MDSM_WIN_ACC(3), [av] "=&v"(av),
+          [tn] "=&s"(tn)
+        : [cur] "v"(cur), [next] "s"(next), [d0] "s"(t[0]), [d1] "s"(t[1]), [d2] "s"(t[2]), [d3] "s"(t[3]),
+          [e0] "s"(t[4]), [e1] "s"(t[5]), [e2] "s"(t[6]), [e3] "s"(t[7])
+        : "v92", "v93", "v94", "v95", "v96", "v97", "v98", "v99", "v100", "v101", "v102", "v103",
+          "v104", "v105", "v106", "v107", "v108", "v109", "v110", "v111", "v112", "v113", "v114",
+          "v115", "v116", "v117", "v118", "v119", "v120", "v121", "v122", "v123", "v124", "v125",
+          "v126", "v127", "s96", "s97", "s98", "s99", "scc", "memory");
+    return tn;
+  }
+#undef MDSM_WIN_ACC
+#undef MDSM_WIN_STUBS
+#undef MDSM_WIN_STUB
+#undef MDSM_WIN_BLOCKS
+#undef MDSM_WIN_JUMP
+#undef MDSM_WIN_ADDS
+#undef MDSM_WIN_ADD
+};
+
+template <int MODE>
+struct WindowTile {
+  using W = WindowCode;
+  static constexpr bool PAIRS = false;
+  static constexpr bool IS_F32 = MODE == MDSM_F32, IS_U8 = MODE == MDSM_U8;
+  static constexpr int MW = W::MW, K = W::K, THREADS = 64 * W::WAVES;
+  static constexpr int TT = 64 * K, TD = W::WAVES * MW, CB = IS_F32 ? 6 : 8;
+  // staging (and widening): WPR waves share a row of a block, every wave has RPW rows
+  static constexpr uint32_t WPR = IS_F32 ? 4 : 1, RSTEP = W::WAVES / WPR, RPW = CB / RSTEP;
+  using T = std::conditional_t<IS_F32, float, std::conditional_t<IS_U8, uint8_t, __half>>;
+  static constexpr uint32_t PER = 4u / sizeof(T);  // samples per source dword
+  static uint64_t table_words(uint32_t nchans, uint32_t ndms) {
+    return (uint64_t)((ndms + TD - 1u) / TD) * W::WAVES * (nchans + 1u) * 8u;
+  }
+  static bool fits(uint32_t) { return true; }
+  // FP32 row words: the window of TT + spread samples from an origin that is
+  // a multiple of PER samples; reads end up to 3 words past it
+  static uint32_t row_words(uint32_t spread) { return ((uint32_t)TT + spread + 8u + 63u) & ~63u; }
+  // raw source dwords per row (F16, U8)
+  static __host__ __device__ uint32_t raw_words(uint32_t rw) { return IS_F32 ? rw : (rw / PER + 63u) & ~63u; }
+  // F32: two buffers of rows; F16, U8: raw dwords and widened rows
+  static uint32_t lds_words_per_row(uint32_t rw) { return rw + raw_words(rw); }
+
+  __device__ __forceinline__ static void run(const T *__restrict__ in, uint64_t ld,
+                                             const int32_t *__restrict__ table,
+                                             const int32_t *__restrict__ reltab, uint32_t nchans,
+                                             uint32_t nsamp, uint32_t ndms, uint32_t rw,
+                                             uint32_t cbr, float *__restrict__ out, uint32_t tt,
+                                             uint32_t dt, float *lds) {
+    typedef W::u32x8 u32x8;
+    typedef W::const_u32x8 const_u32x8;
+    typedef __attribute__((address_space(3))) float lds_float;
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = uniform(threadIdx.x >> 6);
+    const uint32_t t0 = tt * TT, d0 = dt * TD;
+    const uint32_t dlast = min(d0 + TD, ndms) - 1u;
+    const uint32_t dw = d0 + wave * MW;
+    const uint32_t rawn = raw_words(rw);
+    // F32: row buffers A and B; F16, U8: widened rows and raw dwords
+    float *const second = lds + cbr * rw;
+    // this wave's first row of a block and its part of the row's 64-dword chunks
+    const uint32_t srow = wave / WPR, part = wave % WPR;
+    const uint32_t voff = 4u * lane + 256u * part;
+    int32_t spos[RPW], slen[RPW];  // first delay and last of the rows the next stage() takes
+    auto prefetch = [&](uint32_t cb) {
+#pragma unroll
+      for (uint32_t i = 0; i < RPW; ++i) {
+        const int32_t *trow = table + (uint64_t)min(cb + srow + RSTEP * i, nchans - 1u) * ndms;
+        spos[i] = trow[d0];
+        slen[i] = trow[dlast];
+      }
+    };
+    auto stage = [&](uint32_t cb, float *b) {
+#pragma unroll
+      for (uint32_t i = 0; i < RPW; ++i) {
+        const uint32_t r = srow + RSTEP * i;
+        if (r >= min(cbr, nchans - cb)) break;
+        const uint32_t g0 = t0 + (uint32_t)spos[i];
+        const uint32_t len = (uint32_t)TT + (uint32_t)(slen[i] - spos[i]) + (g0 & (PER - 1u));
+        const uint32_t w0 = g0 / PER, ldw = (uint32_t)(ld / PER);  // rows < 2 GiB
+        const uint32_t *src = reinterpret_cast<const uint32_t *>(in) + (uint64_t)(cb + r) * ldw + w0;
+        // rows end at the resource's size: dwords past it read as 0 (they only
+        // feed outputs beyond nsamp)
+        const uint32_t avail = 4u * (ldw - min(w0, ldw));
+        const uint64_t a = reinterpret_cast<uint64_t>(src);
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+            reinterpret_cast<void *>(((uint64_t)uniform((uint32_t)(a >> 32)) << 32) | uniform((uint32_t)a)),
+            (short)0, (int)uniform(avail), 0x00020000);
+        const uint32_t nq = (len + 64u * PER - 1u) / (64u * PER);
+        float *dst = b + r * (IS_F32 ? rw : rawn) + 64u * part;
+        // (the immediate offset applies to the LDS address too)
+        uint32_t q = part, vo = voff;
+        for (; q + 3u * WPR < nq; q += 4u * WPR, vo += 1024u * WPR, dst += 256u * WPR) {
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void *)dst, 4, (int)vo, 0, 0, 0);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void *)dst, 4, (int)vo, 0, 256 * (int)WPR, 0);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void *)dst, 4, (int)vo, 0, 512 * (int)WPR, 0);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void *)dst, 4, (int)vo, 0, 768 * (int)WPR, 0);
+        }
+        for (; q < nq; q += WPR, vo += 256u * WPR, dst += 64u * WPR)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void *)dst, 4, (int)vo, 0, 0, 0);
+      }
+    };
+    // FP32 rows from the raw dwords
+    auto widen = [&](uint32_t cb) {
+#pragma unroll
+      for (uint32_t i = 0; i < RPW; ++i) {
+        const uint32_t r = srow + RSTEP * i;
+        if (r >= min(cbr, nchans - cb)) break;
+        const uint32_t *R = reinterpret_cast<const uint32_t *>(second) + r * rawn;
+        float *P = lds + r * rw;
+        for (uint32_t n = 4u * (lane + 64u * part); n < rw; n += 256u * WPR) {
+          float4 v;
+          if constexpr (IS_U8) {
+            const uint32_t x = R[n / 4u];
+            v = make_float4((float)(x & 0xFFu), (float)((x >> 8) & 0xFFu), (float)((x >> 16) & 0xFFu),
+                            (float)(x >> 24));
+          } else {
+            const uint2 x = *reinterpret_cast<const uint2 *>(R + n / 2u);
+            const half2_t a = __builtin_bit_cast(half2_t, x.x), c = __builtin_bit_cast(half2_t, x.y);
+            v = make_float4((float)a.x, (float)a.y, (float)c.x, (float)c.y);
+          }
+          *reinterpret_cast<float4 *>(P + n) = v;
+        }
+      }
+    };
+
+    float acc[MW][K];
+#pragma unroll
+    for (int i = 0; i < MW; ++i)
+#pragma unroll
+      for (int j = 0; j < K; ++j) acc[i][j] = 0.0f;
+
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_float *)lds + (uint32_t)(4 * K) * lane;
+    // the wave's table entries, one per channel (scalar loads)
+    const const_u32x8 *rt =
+        (const const_u32x8 *)(uintptr_t)reltab + ((uint64_t)dt * W::WAVES + wave) * (nchans + 1u);
+    prefetch(0);
+    stage(0, IS_F32 ? lds : second);
+    if (cbr < nchans) prefetch(cbr);
+    u32x8 o = *rt;
+    wait_vmem();
+    __syncthreads();
+    if constexpr (!IS_F32) {
+      widen(0);
+      __syncthreads();
+    }
+    uint32_t k = 0;
+    for (uint32_t cb = 0; cb < nchans; cb += cbr, ++k) {
+      const bool more = cb + cbr < nchans;
+      if (more) {
+        stage(cb + cbr, IS_F32 ? ((k & 1u) ? lds : second) : second);
+        if (cb + 2u * cbr < nchans) prefetch(cb + 2u * cbr);
+      }
+      const uint32_t nc = min(cbr, nchans - cb);
+      const uint32_t cur = lds0 + (IS_F32 ? 4u * ((k & 1u) * cbr * rw) : 0u);
+      for (uint32_t r = 0; r < nc; ++r) {
+        // (with the next channel's entry; one follows the last channel's)
+        ++rt;
+        o = W::add_channel(acc, cur, o, rt);
+      }
+      wait_vmem();
+      __syncthreads();
+      if constexpr (!IS_F32) {
+        if (more) widen(cb + cbr);
+        __syncthreads();
+      }
+    }
+
+    // the lane's 20 consecutive samples become 64-sample rows through the
+    // wave's own 640 words of LDS, half of the lanes at a time
+    float *mine = lds + wave * 640u;
+    const double base = (double)nchans * -4.0;
+#pragma unroll
+    for (int i = 0; i < MW; ++i) {
+      const uint32_t d = dw + (uint32_t)i;
+      if (d >= ndms) break;
+      float *orow = out + (uint64_t)d * nsamp;
+#pragma unroll
+      for (uint32_t h = 0; h < 2u; ++h) {
+        if ((lane >> 5) == h) {
+#pragma unroll
+          for (int j = 0; j < K; j += 4)
+            *reinterpret_cast<float4 *>(mine + K * (lane & 31u) + j) =
+                make_float4(acc[i][j], acc[i][j + 1], acc[i][j + 2], acc[i][j + 3]);
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (uint32_t j = 0; j < 10u; ++j) {
+          const uint32_t t = t0 + 640u * h + lane + 64u * j;
+          float v = mine[lane + 64u * j];
+          if constexpr (IS_U8) v = (float)((double)(uint32_t)v * (8.0 / 255.0) + base);
+          if (t < nsamp) orow[t] = v;
+        }
+        __builtin_amdgcn_wave_barrier();
+      }
+    }
+  }
+};
+
+template <typename T>
+struct IsWindow : std::false_type {};
+template <int MODE>
+struct IsWindow<WindowTile<MODE>> : std::true_type {};
+// Threads per workgroup: four waves, or the window tiles' eight.
+template <typename T>
+constexpr int tile_threads() {
+  if constexpr (IsWindow<T>::value) return T::THREADS;
+  else return 256;
+}
+
+// Table of a window tile: entry ((dt * 8 + wave) * (nchans + 1) + c) for
+// channel c and trials 4 wave .. 4 wave + 3 of DM tile dt, at their samples'
+// byte offsets in the block's FP32 rows (row c % cbr starts at a multiple of
+// PER samples at or below the tile's first delay); entry nchans, which is
+// loaded and not used, repeats the last channel's.
+template <typename Tile>
+__global__ __launch_bounds__(256) void window_table_kernel(const int32_t *__restrict__ table,
+                                                           uint32_t nchans, uint32_t ndms,
+                                                           uint32_t rw, uint32_t cbr,
+                                                           uint64_t entries,
+                                                           int32_t *__restrict__ reltab) {
+  const uint64_t e = (uint64_t)blockIdx.x * 256u + threadIdx.x;
+  if (e >= entries) return;
+  const uint32_t c = min((uint32_t)(e % (nchans + 1u)), nchans - 1u);
+  const uint64_t g = e / (nchans + 1u);
+  const uint32_t wave = (uint32_t)(g % WindowCode::WAVES), dt = (uint32_t)(g / WindowCode::WAVES);
+  const uint32_t d0 = dt * Tile::TD;
+  const int32_t *row = table + (uint64_t)c * ndms;
+  const uint32_t base = (uint32_t)row[d0], skew = base & (Tile::PER - 1u);
+  uint32_t o[WindowCode::MW], w[2 * WindowCode::MW];
+  for (uint32_t i = 0; i < (uint32_t)WindowCode::MW; ++i) {
+    const uint32_t d = min(d0 + wave * WindowCode::MW + i, ndms - 1u);
+    o[i] = 4u * (c % cbr * rw + skew + ((uint32_t)row[d] - base));
+  }
+  WindowCode::entry(o, w);
+  for (int i = 0; i < 2 * WindowCode::MW; ++i) reltab[e * 8u + i] = (int32_t)w[i];
+}
 
 // ============================================================ packed (F16, U8)
 // LDS row of a channel: copy P (words 0..wp-1) then copy Q (words wp..2wp-1).
@@ -614,6 +969,10 @@ struct PairsOf;
 template <int MW, int K2, int CB, int BURST>
 struct PairsOf<PackedTile<MDSM_F16, MW, K2, CB, BURST>> {
   using type = PackedTile<MDSM_F16_PAIRS, MW, K2, CB, BURST / 2>;
+};
+template <>
+struct PairsOf<WindowTile<MDSM_F16>> {
+  using type = PackedTile<MDSM_F16_PAIRS, 12, 4, 4>;
 };
 
 // ================================================ pair-sum rows (F16, U8)
@@ -1071,9 +1430,41 @@ bool xcd_remap_enabled() {
   return on;
 }
 
+// Waves per SIMD the persistent kernel is compiled for: its item loop costs
+// a few VGPRs over the flat kernel, which drops the 12 x 4 and 10 x 4
+// pair-sum tiles from 4 to 3 waves (above 128 VGPRs).  Held at 4 they spill
+// a few dwords and still run faster (32-beam batch, persistent launch: FP16
+// pair sums 1160 against 1240-1266 ms, U8 1076 against 1270-1285 ms); for
+// the 8 x 4 FP16 tile the same hold (6 waves) was slower (1795 against
+// 1705-1725 ms), so the other tiles are left to the compiler.
+template <typename Tile>
+struct PersistWaves {
+  static constexpr int value = 1;
+};
+// Every launch shape of the register-window tiles: their fixed window
+// registers end at v127, which leaves 4 waves per SIMD if nothing is placed
+// above them.
+template <typename Tile>
+struct FlatWaves {
+  static constexpr int value = 1;
+};
+template <int MODE>
+struct FlatWaves<WindowTile<MODE>> {
+  static constexpr int value = 4;
+};
+template <int MODE>
+struct PersistWaves<WindowTile<MODE>> {
+  static constexpr int value = 4;
+};
+template <int MODE, int MW, int K2, int CBP, int NS, int BURST>
+struct PersistWaves<PairSumTile<MODE, MW, K2, CBP, NS, BURST>> {
+  static constexpr int value = 4;
+};
+
 // ================================================================= kernels
 template <typename Tile>
-__global__ __launch_bounds__(256) void dedisp_kernel(const typename Tile::T *__restrict__ in,
+__global__ __launch_bounds__(tile_threads<Tile>()) __attribute__((amdgpu_waves_per_eu(FlatWaves<Tile>::value)))
+void dedisp_kernel(const typename Tile::T *__restrict__ in,
                                                      uint64_t ld,
                                                      const int32_t *__restrict__ table,
                                                      const int32_t *__restrict__ reltab,
@@ -1181,29 +1572,13 @@ __device__ __forceinline__ void run_item(const BeamDesc *__restrict__ beams, con
             uniform(it.dt), lds);
 }
 
-// Waves per SIMD the persistent kernel is compiled for: its item loop costs
-// a few VGPRs over the flat kernel, which drops the 12 x 4 and 10 x 4
-// pair-sum tiles from 4 to 3 waves (above 128 VGPRs).  Held at 4 they spill
-// a few dwords and still run faster (32-beam batch, persistent launch: FP16
-// pair sums 1160 against 1240-1266 ms, U8 1076 against 1270-1285 ms); for
-// the 8 x 4 FP16 tile the same hold (6 waves) was slower (1795 against
-// 1705-1725 ms), so the other tiles are left to the compiler.
-template <typename Tile>
-struct PersistWaves {
-  static constexpr int value = 1;
-};
-template <int MODE, int MW, int K2, int CBP, int NS, int BURST>
-struct PersistWaves<PairSumTile<MODE, MW, K2, CBP, NS, BURST>> {
-  static constexpr int value = 4;
-};
-
 // Persistent multi-beam kernel: resident workgroups pull items from eight
 // queues, one per XCD slot (workgroup b drains queue b % 8, the XCD the
 // dispatcher puts it on), until the queue passes total_items; every wave
 // of every workgroup reaches the exit.  Beams are ordered by the host,
 // largest first.
 template <typename Tile>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PersistWaves<Tile>::value)))
+__global__ __launch_bounds__(tile_threads<Tile>()) __attribute__((amdgpu_waves_per_eu(PersistWaves<Tile>::value)))
 void batch_kernel(const BeamDesc *__restrict__ beams,
                                                     uint32_t nbeams, uint32_t total_items,
                                                     uint32_t cbr, uint32_t *__restrict__ counter) {
@@ -1226,7 +1601,8 @@ void batch_kernel(const BeamDesc *__restrict__ beams,
 // Flat multi-beam kernel: one workgroup per item (workgroup ID = item, so
 // the dispatcher's round-robin puts item g on XCD g % 8).
 template <typename Tile>
-__global__ __launch_bounds__(256) void batch_flat_kernel(const BeamDesc *__restrict__ beams,
+__global__ __launch_bounds__(tile_threads<Tile>()) __attribute__((amdgpu_waves_per_eu(FlatWaves<Tile>::value)))
+void batch_flat_kernel(const BeamDesc *__restrict__ beams,
                                                          uint32_t nbeams, uint32_t cbr) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const BeamItem it = decode_item(beams, nbeams, blockIdx.x);
@@ -1240,7 +1616,7 @@ __global__ __launch_bounds__(256) void batch_flat_kernel(const BeamDesc *__restr
 template <int V>
 struct VariantDef;
 template <> struct VariantDef<1> { using F32 = F32Tile<8, 4, 8>;   using F16 = F16Tile<8, 2, 8>;   using U8 = U8Tile<8, 2, 8>; };
-template <> struct VariantDef<2> { using F32 = F32Tile<16, 4, 4>;  using F16 = F16Tile<16, 2, 4>;  using U8 = U8Tile<16, 2, 4>; };
+template <> struct VariantDef<2> { using F32 = F32Tile<16, 4, 4>;  using F16 = F16Tile<16, 2, 4>;  using U8 = WindowTile<MDSM_U8>; };
 template <> struct VariantDef<3> { using F32 = F32Tile<8, 8, 8>;   using F16 = F16Tile<8, 4, 8>;   using U8 = U8Tile<8, 4, 8>; };
 template <> struct VariantDef<4> { using F32 = F32Tile<16, 8, 4>;  using F16 = F16Tile<16, 4, 4>;  using U8 = U8Tile<16, 4, 4>; };
 template <> struct VariantDef<5> { using F32 = F32Tile<32, 2, 2>;  using F16 = F16Tile<32, 1, 2>;  using U8 = U8Tile<32, 1, 2>; };
@@ -1253,9 +1629,9 @@ template <> struct VariantDef<8> { using F32 = F32Tile<16, 4, 4, 4>; using F16 =
 template <> struct VariantDef<9> { using F32 = F32Tile<8, 8, 4>;    using F16 = F16Tile<8, 4, 4>;   using U8 = U8Tile<8, 4, 4>; };
 template <> struct VariantDef<10> { using F32 = F32Tile<4, 16, 8>;  using F16 = F16Tile<4, 8, 8>;   using U8 = U8Tile<4, 8, 8>; };
 template <> struct VariantDef<11> { using F32 = F32Tile<4, 16, 4>;  using F16 = F16Tile<4, 8, 4>;   using U8 = U8Tile<4, 8, 4>; };
-// more samples per lane at 12 or 16 trials per wave: one address add per
-// 8 or 6 packed adds
-template <> struct VariantDef<12> { using F32 = F32Tile<12, 6, 4>;  using F16 = F16Tile<12, 4, 4>;  using U8 = U8Tile<12, 4, 4>; };
+// register windows (F32 and F16 here, U8 in 2), and 12 or 16 trials per wave
+// with more samples per lane: one address add per 8 or 6 packed adds
+template <> struct VariantDef<12> { using F32 = WindowTile<MDSM_F32>; using F16 = WindowTile<MDSM_F16>; using U8 = U8Tile<12, 4, 4>; };
 template <> struct VariantDef<13> { using F32 = F32Tile<16, 6, 4>;  using F16 = F16Tile<16, 3, 4>;  using U8 = U8Tile<16, 3, 4>; };
 // 16 trials per wave over 8-channel blocks: half the barriers per add
 template <> struct VariantDef<14> { using F32 = F32Tile<16, 4, 8>;  using F16 = F16Tile<16, 2, 8>;  using U8 = U8Tile<16, 2, 8>; };
@@ -1334,15 +1710,22 @@ int with_tile(int dtype, int variant, Fn &&fn) {
   return MDSM_ERR_ARG;
 }
 
+// LDS of a workgroup: 64 KB, or 80 KB for the window tiles (their registers
+// leave two workgroups of eight waves per CU, which has 160 KB).
+template <typename Tile>
+constexpr uint64_t tile_lds() {
+  return IsWindow<Tile>::value ? 80 * 1024 : 64 * 1024;
+}
+
 // Channels staged per block: the tile's CB, reduced while the block's LDS
-// (two buffers, plus raw staging for U8) exceeds 64 KB (160 KB per CU); even
+// (two buffers, plus raw staging for U8) exceeds tile_lds (160 KB per CU); even
 // for F16_PAIRS, whose channel pairs must not straddle two blocks.
 template <typename Tile>
 uint32_t stage_channels(uint32_t rw) {
   const uint64_t per = Tile::lds_words_per_row(rw) * sizeof(float);
   const uint64_t step = Tile::PAIRS ? 2 : 1;
   uint64_t n = (uint64_t)Tile::CB;
-  while (n > step && n * per > 64 * 1024) n -= step;
+  while (n > step && n * per > tile_lds<Tile>()) n -= step;
   if (n * per > 160 * 1024) return 0;
   return (uint32_t)n;
 }
@@ -1354,14 +1737,19 @@ int num_variants(int dtype) {
                                                        : kNumVariants;
 }
 
-// Untuned defaults, the fastest shapes measured at 1024 channels x 4096
-// trials: F16_PAIRS and U8 prefer the pair-sum shapes (20, 22), which take
-// only surveys with few delay differences per channel pair and DM tile, and
-// fall back to the fastest shape that takes every survey (15, 2).
+// Untuned defaults.  F32 and F16 take the register-window tile, which was
+// the fastest shape of every survey tried: 1024 channels x 4096 trials x 2^17
+// samples 15.9 ms against 29.7 (F32, shape 8) and 15.1 against 21.9 (F16,
+// shape 15); delay slopes from 0.1 to 24 samples per trial 1.5 to 2.5 times
+// (418 MHz, step 0.5: 5.7 against 14.2 ms); 64 channels 1.6 times; 64 trials x
+// 8192 samples, too few tiles for the chip, level.  F16_PAIRS and U8 prefer
+// the pair-sum shapes (20, 22), which take only surveys with few delay
+// differences per channel pair and DM tile, and fall back to a shape that
+// takes every survey whose delay spread it can stage.
 int preferred_variant(int dtype) {
   switch (dtype) {
-    case MDSM_F32: return 8;
-    case MDSM_F16: return 15;
+    case MDSM_F32: return 12;
+    case MDSM_F16: return 12;
     case MDSM_F16_PAIRS: return 20;
     default: return 22;
   }
@@ -1369,9 +1757,9 @@ int preferred_variant(int dtype) {
 
 int fallback_variant(int dtype) {
   switch (dtype) {
-    case MDSM_F16_PAIRS: return 15;
+    case MDSM_F32: return 8;
     case MDSM_U8: return 2;
-    default: return preferred_variant(dtype);
+    default: return 15;
   }
 }
 
@@ -1439,11 +1827,16 @@ uint64_t trial_offset_words(int dtype, int variant, uint32_t nchans, uint32_t nd
   uint64_t n = 0;
   with_tile(dtype, variant, [&](auto *tp) {
     using Tile = std::remove_pointer_t<decltype(tp)>;
+    if constexpr (IsWindow<Tile>::value) {
+      n = Tile::table_words(nchans, ndms);
+      return MDSM_OK;
+    } else {
     const uint64_t n_dtiles = (ndms + Tile::TD - 1) / Tile::TD;
     const uint64_t nblocks = cbr ? (nchans + cbr - 1) / cbr : 0;
     n = n_dtiles * nblocks * 4u * Tile::Rel::WORDS;
     if constexpr (IsPairSum<Tile>::value) n += n_dtiles * nblocks * (uint64_t)(Tile::CB / 2) * 2u;
     return MDSM_OK;
+    }
   });
   return n;
 }
@@ -1462,6 +1855,10 @@ int launch_trial_offsets(int dtype, int variant, const int32_t *table, uint32_t 
       const uint64_t nrel = (uint64_t)((ndms + Tile::TD - 1) / Tile::TD) * nblocks * 4u * Tile::Rel::WORDS;
       hipLaunchKernelGGL(pairsum_offset_kernel<Tile>, dim3((uint32_t)grid), dim3(256), 0, s, table,
                          nchans, ndms, rw, cbr, nblocks, nrel, total, reltab);
+    } else if constexpr (IsWindow<Tile>::value) {
+      const uint64_t entries = total / 8u;
+      hipLaunchKernelGGL(window_table_kernel<Tile>, dim3((uint32_t)((entries + 255u) / 256u)), dim3(256),
+                         0, s, table, nchans, ndms, rw, cbr, entries, reltab);
     } else {
       hipLaunchKernelGGL(trial_offset_kernel<Tile>, dim3((uint32_t)grid), dim3(256), 0, s, table,
                          nchans, ndms, rw, cbr, nblocks, total, reltab);
@@ -1488,7 +1885,7 @@ int launch_dedisperse(int dtype, int variant, const void *in, uint64_t ld, const
     const uint32_t cbr = stage_channels<Tile>(rw);
     MDSM_REQUIRE(cbr >= 1, MDSM_ERR_ARG, "delay spread too large for LDS staging (%u words)", rw);
     const size_t lds = (size_t)cbr * Tile::lds_words_per_row(rw) * sizeof(float);
-    hipLaunchKernelGGL(dedisp_kernel<Tile>, dim3((uint32_t)blocks), dim3(256), lds, s,
+    hipLaunchKernelGGL(dedisp_kernel<Tile>, dim3((uint32_t)blocks), dim3(tile_threads<Tile>()), lds, s,
                        reinterpret_cast<const typename Tile::T *>(in), ld, table, reltab, nchans,
                        nsamp, ndms, rw, cbr, n_dtiles, n_ttiles, remap, out);
     MDSM_HIP(hipGetLastError());
@@ -1514,7 +1911,7 @@ int launch_batch_flat(int dtype, int variant, const BeamDesc *d_beams, uint32_t 
     const uint32_t cbr = stage_channels<Tile>(max_rw);
     MDSM_REQUIRE(cbr >= 1, MDSM_ERR_ARG, "delay spread too large for LDS staging");
     const size_t lds = (size_t)cbr * Tile::lds_words_per_row(max_rw) * sizeof(float);
-    hipLaunchKernelGGL(batch_flat_kernel<Tile>, dim3(total_items), dim3(256), lds, s, d_beams,
+    hipLaunchKernelGGL(batch_flat_kernel<Tile>, dim3(total_items), dim3(tile_threads<Tile>()), lds, s, d_beams,
                        nbeams, cbr);
     MDSM_HIP(hipGetLastError());
     return MDSM_OK;
@@ -1533,14 +1930,14 @@ int launch_batch_dedisperse(int dtype, int variant, const BeamDesc *d_beams, uin
     if (grid <= 0) {
       // persistent: as many workgroups as can be resident at once
       int per_cu = 0, dev = 0, cus = 0;
-      MDSM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, batch_kernel<Tile>, 256, lds));
+      MDSM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, batch_kernel<Tile>, tile_threads<Tile>(), lds));
       MDSM_HIP(hipGetDevice(&dev));
       MDSM_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
       grid = std::max(1, per_cu) * std::max(1, cus);
     }
     // every one of the eight queues needs workers: a multiple of 8, at least 8
     grid = std::max(8, (grid + 7) / 8 * 8);
-    hipLaunchKernelGGL(batch_kernel<Tile>, dim3(grid), dim3(256), lds, s, d_beams, nbeams,
+    hipLaunchKernelGGL(batch_kernel<Tile>, dim3(grid), dim3(tile_threads<Tile>()), lds, s, d_beams, nbeams,
                        total_items, cbr, d_counter);
     MDSM_HIP(hipGetLastError());
     return MDSM_OK;
