@@ -336,6 +336,74 @@ __device__ __forceinline__ double from_next_lane(double x) {
   return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
 
+__device__ __forceinline__ float from_next_lane(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x130, 0xF, 0xF, true));
+}
+
+// FP32 screen of a wave's runs: true in lanes that may hold a sample passing
+// the FP64 test at some level.  The levels are the same sums in FP32; with
+// E >= |x| over a level's window of w samples, the FP32 sum lies within
+// 6 * 2^-24 w E of the FP64 one, and the FP64 test needs
+// S >= w m + thresh sd sqrt(w) (1 - 2^-40), whose FP32 form is off by less
+// than 8 * 2^-24 of its terms; slack covers both twice over.  The compare is
+// written so that a NaN or an overflow on either side passes.
+__device__ __forceinline__ bool screen_runs(const float (&x)[DW_R], double m, double sd, int nwidths,
+                                            float thresh) {
+  const float mf = (float)m, sdf = (float)sd;
+  bool pass = !(sdf > 1e-30f && sdf < 1e30f);
+  float v[DW_R], e = 0.0f;
+#pragma unroll
+  for (int i = 0; i < DW_R; ++i) {
+    v[i] = x[i];
+    e = fmaxf(e, fabsf(x[i]));
+  }
+  auto test = [&](int k, float sqrtw) {
+    const float w = (float)(1 << k);
+    const float a = w * mf, b = thresh * sqrtw * sdf;
+    const float bound = a + b - ((fabsf(a) + b) * 0x1p-20f + w * e * 0x1p-21f);
+    float mx = v[0];
+#pragma unroll
+    for (int i = 1; i < DW_R; ++i) mx = fmaxf(mx, v[i]);
+    pass |= !(mx < bound);
+  };
+  test(0, 1.0f);
+#pragma unroll
+  for (int k = 1; k < 7; ++k) {
+    if (k >= nwidths) break;
+    const int h = 1 << (k - 1);
+    // e covers the lanes a level-k window reaches: 1 on (k <= 4), 2, 4
+    if (k == 1 || k == 5) e = fmaxf(e, from_next_lane(e));
+    if (k == 6) e = fmaxf(e, from_next_lane(from_next_lane(e)));
+    if (h < DW_R) {
+      float nx[DW_R / 2];
+#pragma unroll
+      for (int j = 0; j < DW_R / 2; ++j)
+        if (j < h) nx[j] = from_next_lane(v[j]);
+#pragma unroll
+      for (int i = 0; i < DW_R; ++i) v[i] = v[i] + (i + h < DW_R ? v[i + h] : nx[i + h - DW_R]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < DW_R; ++i) {
+        const float n1 = from_next_lane(v[i]);
+        v[i] = v[i] + (h == DW_R ? n1 : from_next_lane(n1));
+      }
+    }
+    constexpr float kSqrt[7] = {1.0f, 1.41421356f, 2.0f, 2.82842712f, 4.0f, 5.65685425f, 8.0f};
+    test(k, kSqrt[k]);
+  }
+  return pass && sd > 0.0;
+}
+
+// SCREEN: the FP64 levels run only in waves where the FP32 screen finds a
+// lane that may pass.  The screen costs half of the FP64 levels (FP32 adds
+// issue at twice the rate, one DPP move instead of two), so it pays while
+// most waves hold no candidate: launch_detect takes it from a threshold of
+// 4 on (noise passes in about one wave in ten there, in one of 10^5 at 6);
+// at 3 nearly every wave does.  4096 rows of 2^17 samples at 6 sigma: 400 us
+// (5.4 TB/s read), 617 us with FP64 levels and 4-byte loads everywhere.  One
+// reservation per wave instead of one per sample position matters where
+// candidates are many: at 3 sigma (4.2 million) 6.4 ms, 35 ms before.
+template <bool SCREEN>
 __global__ __launch_bounds__(NT) void detect_wave_kernel(
     const float *__restrict__ x, uint32_t nsamp, uint32_t L, uint32_t nb,
     const double *__restrict__ mean, const double *__restrict__ stdv, int nwidths, double thresh,
@@ -345,23 +413,33 @@ __global__ __launch_bounds__(NT) void detect_wave_kernel(
   const uint64_t seg0 = ((uint64_t)blockIdx.x * (NT / 64) + (threadIdx.x >> 6)) * DW_SEG;
   if (seg0 >= nsamp) return;  // whole wave; this kernel has no barriers
   const uint64_t t0 = seg0 + (uint64_t)DW_R * lane;
-  // the row through a buffer resource bounded to nsamp floats: samples past
-  // the row end read as 0 (they only feed levels that run past nsamp)
   const float *row = x + (uint64_t)d * nsamp;
-  const __amdgpu_buffer_rsrc_t rs =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(row), (short)0, (int)(4u * nsamp), 0x00020000);
-  double v[DW_R];
-  const int byte0 = (int)min(t0, (uint64_t)nsamp) * 4;
-  // one range-checked dword per sample (no branch on the row end: the
-  // hardware returns 0 past num_records)
+  float xf[DW_R];
+  if (seg0 + 64u * DW_R <= nsamp) {
+    // four 16-byte loads per lane (any 4-byte alignment)
 #pragma unroll
-  for (int i = 0; i < DW_R; ++i)
-    v[i] = (double)__builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, byte0 + 4 * i, 0, 0));
-
+    for (int i = 0; i < DW_R; i += 4) {
+      const float4u q = *reinterpret_cast<const float4u *>(row + t0 + i);
+      xf[i] = q[0], xf[i + 1] = q[1], xf[i + 2] = q[2], xf[i + 3] = q[3];
+    }
+  } else {
+    // the row's end through a buffer resource bounded to nsamp floats:
+    // samples past it read as 0 (they only feed levels that run past nsamp)
+    const __amdgpu_buffer_rsrc_t rs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(row), (short)0, (int)(4u * nsamp), 0x00020000);
+    const int byte0 = (int)min(t0, (uint64_t)nsamp) * 4;
+#pragma unroll
+    for (int i = 0; i < DW_R; ++i)
+      xf[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, byte0 + 4 * i, 0, 0));
+  }
   // the run's block statistics and per-level bounds (see detect_kernel for
   // the pass bound a >= lim * den)
   const uint32_t b = (uint32_t)(min(t0, (uint64_t)nsamp - 1u) / L);
   const double m = mean[(uint64_t)d * nb + b], sd = stdv[(uint64_t)d * nb + b];
+  if (SCREEN && __ballot(screen_runs(xf, m, sd, nwidths, (float)thresh)) == 0ull) return;
+  double v[DW_R];
+#pragma unroll
+  for (int i = 0; i < DW_R; ++i) v[i] = (double)xf[i];
   const bool live = sd > 0.0;
   const double lim = thresh > 0.0 ? thresh * (1.0 - 0x1p-40) : -INFINITY;
   // samples of the run whose level-k window ends inside the row: i < n_in_k
@@ -430,13 +508,25 @@ __global__ __launch_bounds__(NT) void detect_wave_kernel(
     }
     test_level(k);
   }
+  // one reservation for the wave's candidates, then each sample's in lane order
   const bool own = lane < (uint32_t)DW_LANES;
+  auto level = [&](int i) { return i < 8 ? (bk >> (4 * i)) & 15u : (bk2 >> (4 * (i - 8))) & 15u; };
+  auto hit = [&](int i) { return own && level(i) < 8u && best[i] >= thresh; };
+  uint32_t total = 0;
+#pragma unroll
+  for (int i = 0; i < DW_R; ++i) total += (uint32_t)__popcll(__ballot(hit(i)));
+  if (total == 0) return;
+  uint32_t base = 0;
+  if (lane == 0) base = atomicAdd(count, total);
+  base = __shfl(base, 0);
 #pragma unroll
   for (int i = 0; i < DW_R; ++i) {
-    const uint32_t k = i < 8 ? (bk >> (4 * i)) & 15u : (bk2 >> (4 * (i - 8))) & 15u;
-    const bool hit = own && k < 8u && best[i] >= thresh;
-    mdsm_cand_t cand{(int32_t)d, (int32_t)(t0 + (uint64_t)i), (int32_t)k, (float)best[i]};
-    emit(hit, cand, cands, cap, count);
+    const bool h = hit(i);
+    const unsigned long long mask = __ballot(h);
+    const uint32_t idx = base + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
+    if (h && idx < cap)
+      cands[idx] = mdsm_cand_t{(int32_t)d, (int32_t)(t0 + (uint64_t)i), (int32_t)level(i), (float)best[i]};
+    base += (uint32_t)__popcll(mask);
   }
 }
 
@@ -810,8 +900,13 @@ int launch_detect(const float *x, uint32_t nrows, uint32_t nsamp, uint32_t L, co
     // register-resident form: four waves of DW_SEG samples per workgroup
     const uint64_t per_wg = (uint64_t)DW_SEG * (NT / 64);
     const uint32_t nwg = (uint32_t)(((uint64_t)nsamp + per_wg - 1u) / per_wg);
-    hipLaunchKernelGGL(detect_wave_kernel, dim3(nwg, nrows), dim3(NT), 0, s, x, nsamp, L, nb, mean,
-                       stdv, nwidths, thresh, cands, cap, count);
+    const bool screen = thresh >= 4.0 && thresh < 1e6;
+    if (screen)
+      hipLaunchKernelGGL(detect_wave_kernel<true>, dim3(nwg, nrows), dim3(NT), 0, s, x, nsamp, L, nb, mean,
+                         stdv, nwidths, thresh, cands, cap, count);
+    else
+      hipLaunchKernelGGL(detect_wave_kernel<false>, dim3(nwg, nrows), dim3(NT), 0, s, x, nsamp, L, nb, mean,
+                         stdv, nwidths, thresh, cands, cap, count);
     MDSM_HIP(hipGetLastError());
     return MDSM_OK;
   }
