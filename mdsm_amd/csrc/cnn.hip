@@ -1,12 +1,12 @@
 // cnn.hip -- BF16 MFMA kernels of the event-triage CNN (forward, backward,
 // optimiser).
 //
-// Every product of the network (3x3 convolutions as implicit GEMMs,
-// their weight and input gradients, the two linear layers) runs through one
-// GEMM kernel, C[m][n] = sum_k A(m,k) B(k,n), with BF16 operands, FP32
-// accumulation on v_mfma_f32_16x16x16_bf16, and operand loaders that read
-// dense strided matrices or gather im2col windows straight from NHWC
-// activations (no im2col buffer):
+// The 3x3 convolutions run as implicit products on
+// v_mfma_f32_16x16x16_bf16 with BF16 operands and FP32 accumulation, each
+// fused with what follows or precedes it (forward with bias, ReLU and pool;
+// the first layer's weight gradient with the pool's backward), reading NHWC
+// activations without an im2col buffer.  The two linear layers run through
+// one GEMM kernel, C[m][n] = sum_k A(m,k) B(k,n):
 //
 //   tile 64 (m) x 64 (n) x 32 (k), 256 threads = 4 waves in 2 x 2, each wave
 //   a 32 x 32 block = 2 x 2 MFMA 16x16 tiles.  A is staged as As[m][k] and B
@@ -19,9 +19,8 @@
 //   epilogue_kernel sums in slice order (deterministic), adds the bias,
 //   applies ReLU or a ReLU mask and stores FP32 and/or BF16.
 //
-// Element-wise kernels: ReLU + 2x2 max pool (argmax and mask byte), its
-// backward, per-channel bias gradients, softmax cross-entropy, Adam, NCHW ->
-// NHWC input transpose.  BF16 conversion is round-to-nearest-even.
+// Element-wise kernels: backward of the pool with the bias gradients, softmax
+// cross-entropy, Adam, NCHW -> NHWC input transpose, parameter layouts.  BF16 conversion is round-to-nearest-even.
 #include <hip/hip_runtime.h>
 
 #include "cnn_internal.h"
@@ -83,73 +82,6 @@ struct Dense {  // (r, c) at p[r*sr + c*sc]
     }
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = k + e < kend ? q[e * sr] : (uint16_t)0;
-  }
-};
-
-// im2col view of NHWC x[B][H][W][C]: (pixel, k) with k = (ky*3 + kx)*C + c
-// reads x at (h + ky - 1, w + kx - 1); flipped, at (h - ky + 1, w - kx + 1).
-template <bool FLIP>
-struct Im2col {
-  const uint16_t *p;
-  int H, W, C;
-  __device__ __forceinline__ uint16_t elem(int b, int h, int w, int k) const {
-    const int kk = k / C, c = k - kk * C;
-    const int ky = kk / 3, kx = kk - 3 * ky;
-    const int hh = FLIP ? h - ky + 1 : h + ky - 1, ww = FLIP ? w - kx + 1 : w + kx - 1;
-    if (hh < 0 || hh >= H || ww < 0 || ww >= W) return 0;
-    return p[(int64_t)((b * H + hh) * W + ww) * C + c];
-  }
-  // one pixel, 8 consecutive k: with C a multiple of 8 they share (ky, kx)
-  // and are 8 consecutive channels, one aligned 16-byte load
-  __device__ __forceinline__ void fetchA(int64_t m, int64_t k, int64_t kend, uint16_t v[8]) const {
-    const int pix = (int)m, kk0 = (int)k;
-    const int w = pix % W, bh = pix / W, h = bh % H, b = bh / H;
-    if ((C & 7) == 0 && k + 8 <= kend) {
-      const int kk = kk0 / C, c = kk0 - kk * C;
-      const int ky = kk / 3, kx = kk - 3 * ky;
-      const int hh = FLIP ? h - ky + 1 : h + ky - 1, ww = FLIP ? w - kx + 1 : w + kx - 1;
-      if (hh < 0 || hh >= H || ww < 0 || ww >= W) {
-        zero8(v);
-      } else {
-        load8(p + (int64_t)((b * H + hh) * W + ww) * C + c, v);
-      }
-      return;
-    }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = k + e < kend ? elem(b, h, w, kk0 + e) : (uint16_t)0;
-  }
-  // 8 consecutive pixels, one k: stepped through (w, h, b) without division
-  __device__ __forceinline__ void fetchB(int64_t n, int64_t k, int64_t kend, uint16_t v[8]) const {
-    int pix = (int)k;
-    int w = pix % W, bh = pix / W, h = bh % H, b = bh / H;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      v[e] = k + e < kend ? elem(b, h, w, (int)n) : (uint16_t)0;
-      if (++w == W) {
-        w = 0;
-        if (++h == H) {
-          h = 0;
-          ++b;
-        }
-      }
-    }
-  }
-};
-
-// weights w[co][(ky*3+kx)*Ci + ci] seen as (k = (ky*3+kx)*Co + co, n = ci)
-struct WFlip {
-  const uint16_t *p;
-  int Ci, Co;
-  __device__ __forceinline__ void fetchB(int64_t n, int64_t k, int64_t kend, uint16_t v[8]) const {
-    int kk = (int)k / Co, co = (int)k - kk * Co;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      v[e] = k + e < kend ? p[(int64_t)co * 9 * Ci + kk * Ci + (int)n] : (uint16_t)0;
-      if (++co == Co) {
-        co = 0;
-        ++kk;
-      }
-    }
   }
 };
 
@@ -231,8 +163,18 @@ __global__ void epilogue_kernel(const float *__restrict__ part, int splits, int6
   const int64_t MN = M * N;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < MN;
        i += (int64_t)gridDim.x * blockDim.x) {
+    // slices in order, 16 loads ahead of their adds (one at a time, 128
+    // slices of 16384 values took 31 us; 9 us so)
     float v = part[i];
-    for (int z = 1; z < splits; ++z) v += part[(int64_t)z * MN + i];
+    int z = 1;
+    for (; z + 16 <= splits; z += 16) {
+      float t[16];
+#pragma unroll
+      for (int u = 0; u < 16; ++u) t[u] = part[(int64_t)(z + u) * MN + i];
+#pragma unroll
+      for (int u = 0; u < 16; ++u) v += t[u];
+    }
+    for (; z < splits; ++z) v += part[(int64_t)z * MN + i];
     if (bias) v += bias[i % N];
     if (out_f32) out_f32[i] = v;
     if (mask && !(mask[i] > 0.f)) v = 0.f;
@@ -241,56 +183,480 @@ __global__ void epilogue_kernel(const float *__restrict__ part, int splits, int6
   }
 }
 
-// z[B][H][W][C] + bias -> ReLU -> 2x2 max pool -> a[B][H/2][W/2][C] (BF16),
-// idx = argmax (0..3, first maximum) | 4 when the maximum is positive
-__global__ void relu_pool_kernel(const float *__restrict__ z, const float *__restrict__ bias,
-                                 int64_t B, int H, int W, int C, uint16_t *__restrict__ a,
-                                 uint8_t *__restrict__ idx) {
+// ------------------------------------------------------------ convolutions
+// Walks NHWC pixels: (b, h, w) of a linear index, stepped without division.
+struct Pixel {
+  int w, h;
+  int64_t b;
+  __device__ __forceinline__ void set(int64_t i, int H, int W) {
+    const int64_t bh = i / W;
+    w = (int)(i - bh * W);
+    b = bh / H;
+    h = (int)(bh - b * H);
+  }
+  __device__ __forceinline__ void advance(int n, int H, int W) {
+    for (w += n; w >= W; w -= W)
+      if (++h == H) {
+        h = 0;
+        ++b;
+      }
+  }
+};
+
+__device__ __forceinline__ bf16x4 load4(const uint16_t *p) { return *reinterpret_cast<const bf16x4 *>(p); }
+
+// 3x3 convolution (pad 1) + bias + ReLU + 2x2 max pool in one pass, NHWC BF16
+// in and out, FP32 accumulation on v_mfma_f32_16x16x16_bf16 over
+// k = (ky*3 + kx)*CI + ci in order.
+//   A (16 x 16): rows are 4 pooled pixels x the 4 positions of their window,
+//   so a lane's four results of one output channel (D rows 4*(lane/16)+r) are
+//   one pool window and bias, ReLU and maximum need no exchange; a lane's
+//   operand is one 8-byte load of 4 channels (two 4-byte loads for CI = 2),
+//   straight from the activations (each is read 9 times, from L1/L2).
+//   B: the layer's weights, held in registers for the wave's whole run of
+//   tiles; NB output-channel tiles per wave.
+// a[pooled][CO] = BF16 of the maximum, idx = argmax (0..3, first maximum) | 4
+// when the maximum is positive.  Storing the FP32 pre-activations and pooling
+// them in a second pass moved 8 bytes per pixel and channel: 256 snippets of
+// 64 x 256, three layers: 320 + 117 + 57 us, now 46 + 44 + 41.  Bound by the
+// activation loads (9 per element, L1 and L2).
+template <int CI, int CO, int NB>
+__global__ __launch_bounds__(NT) void conv_pool_kernel(const uint16_t *__restrict__ x,
+                                                       const uint16_t *__restrict__ wt,
+                                                       const float *__restrict__ bias, int64_t P, int H,
+                                                       int W, int run, uint16_t *__restrict__ a,
+                                                       uint8_t *__restrict__ idx) {
+  constexpr int KC = (9 * CI + 15) / 16;  // 16-deep steps
+  const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
   const int Ho = H / 2, Wo = W / 2;
-  const int64_t n = B * Ho * Wo * C;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int c = (int)(i % C);
-    int64_t r = i / C;
-    const int wo = (int)(r % Wo);
-    r /= Wo;
-    const int ho = (int)(r % Ho);
-    const int64_t b = r / Ho;
-    float best = -1.f;
-    int arg = 0;
+  const int n0 = blockIdx.y * NB * 16;
+  bf16x4 bw[KC][NB];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      float v = z[((b * H + 2 * ho + (k >> 1)) * W + 2 * wo + (k & 1)) * C + c] + bias[c];
-      v = v > 0.f ? v : 0.f;
-      if (v > best) {
-        best = v;
-        arg = k;
+  for (int c = 0; c < KC; ++c)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      const uint16_t *q = wt + (int64_t)(n0 + 16 * j + n) * (9 * CI) + 16 * c + 4 * g;
+      if constexpr (CI == 2) {  // rows of 18, 4-byte aligned
+        const int k = 16 * c + 4 * g;
+        const uint32_t lo = k < 18 ? *reinterpret_cast<const uint32_t *>(q) : 0u;
+        const uint32_t hi = k + 2 < 18 ? *reinterpret_cast<const uint32_t *>(q + 2) : 0u;
+        bw[c][j] = __builtin_bit_cast(bf16x4, ((uint64_t)hi << 32) | lo);
+      } else {
+        bw[c][j] = load4(q);
       }
     }
-    a[i] = to_bf16(best);
-    idx[i] = (uint8_t)(arg | (best > 0.f ? 4 : 0));
+  float bs[NB];
+#pragma unroll
+  for (int j = 0; j < NB; ++j) bs[j] = bias[n0 + 16 * j + n];
+  const int64_t wave = (int64_t)blockIdx.x * (NT / 64) + (threadIdx.x >> 6);
+  int64_t p = wave * run * 4;  // first pooled pixel of the wave's run
+  const int64_t pend = p + (int64_t)run * 4 < P ? p + (int64_t)run * 4 : P;
+  if (p >= pend) return;
+  // this lane's A row: pooled pixel p + n/4, window position n%4
+  Pixel px;
+  px.set(p + (n >> 2) < P ? p + (n >> 2) : P - 1, Ho, Wo);
+  for (; p < pend; p += 4) {
+    const int h = 2 * px.h + ((n >> 1) & 1), w = 2 * px.w + (n & 1);
+    const uint16_t *q = x + ((px.b * H + h) * W + w) * CI;
+    auto tap = [&](int t, bool &ok) {  // address of the tap's pixel, itself when outside
+      const int ky = t / 3, kx = t - 3 * ky;
+      ok = (ky != 0 || h > 0) && (ky != 2 || h < H - 1) && (kx != 0 || w > 0) && (kx != 2 || w < W - 1);
+      return q + (ok ? ((ky - 1) * W + (kx - 1)) * CI : 0);
+    };
+    f32x4 acc[NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (CI == 2) {
+      // step 0: taps 2g and 2g + 1; step 1: tap 8 (g = 0), zeros
+      uint32_t v[2];
+      const int ty = (2 * g) / 3, tx = 2 * g - 3 * ty, uy = (2 * g + 1) / 3, ux = 2 * g + 1 - 3 * uy;
+      const int dy[2] = {ty - 1, uy - 1}, dx[2] = {tx - 1, ux - 1};
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const int hh = h + dy[e], ww = w + dx[e];
+        const bool ok = hh >= 0 && hh < H && ww >= 0 && ww < W;
+        const uint32_t u = *reinterpret_cast<const uint32_t *>(q + (ok ? (dy[e] * W + dx[e]) * 2 : 0));
+        v[e] = ok ? u : 0u;
+      }
+      const bool ok8 = g == 0 && h < H - 1 && w < W - 1;
+      const uint32_t u8 = *reinterpret_cast<const uint32_t *>(q + (ok8 ? (W + 1) * 2 : 0));
+      const bf16x4 a0 = __builtin_bit_cast(bf16x4, ((uint64_t)v[1] << 32) | v[0]);
+      const bf16x4 a1 = __builtin_bit_cast(bf16x4, (uint64_t)(ok8 ? u8 : 0u));
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a0, bw[0][j], acc[j], 0, 0, 0);
+        acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a1, bw[1][j], acc[j], 0, 0, 0);
+      }
+    } else {
+      bf16x4 av[KC];
+#pragma unroll
+      for (int c = 0; c < KC; ++c) {
+        bool ok;
+        const uint16_t *s = tap(c * 16 / CI, ok);
+        av[c] = load4(s + c * 16 % CI + 4 * g);
+        if (!ok) av[c] = bf16x4{0, 0, 0, 0};
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int c = 0; c < KC; ++c)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+          acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av[c], bw[c][j], acc[j], 0, 0, 0);
+    }
+    if (p + g < P) {
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        float best = -1.f;
+        int arg = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          float v = acc[j][k] + bs[j];
+          v = v > 0.f ? v : 0.f;
+          if (v > best) {
+            best = v;
+            arg = k;
+          }
+        }
+        const int64_t o = (p + g) * CO + n0 + 16 * j + n;
+        a[o] = to_bf16(best);
+        idx[o] = (uint8_t)(arg | (best > 0.f ? 4 : 0));
+      }
+    }
+    px.advance(4, Ho, Wo);
+    if (p + 4 + (n >> 2) >= P) px.set(P - 1, Ho, Wo);  // rows past the end repeat the last pixel
   }
 }
 
-// da[B][H/2][W/2][C] (FP32) -> dz[B][H][W][C] (BF16): the gradient goes to
-// the argmax when it was positive, zeros elsewhere
-__global__ void pool_bwd_kernel(const float *__restrict__ da, const uint8_t *__restrict__ idx,
-                                int64_t B, int H, int W, int C, uint16_t *__restrict__ dz) {
-  const int Ho = H / 2, Wo = W / 2;
-  const int64_t n = B * Ho * Wo * C;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int c = (int)(i % C);
-    int64_t r = i / C;
-    const int wo = (int)(r % Wo);
-    r /= Wo;
-    const int ho = (int)(r % Ho);
-    const int64_t b = r / Ho;
-    const uint8_t q = idx[i];
-    const uint16_t g = (q & 4) ? to_bf16(da[i]) : (uint16_t)0;
+// Input gradient of a 3x3 convolution: dx[pix][ci] = sum over
+// k = (ky*3 + kx)*CO + co, in order, of dz[pix moved back by the tap][co] *
+// w[co][tap][ci], FP32.  As the forward kernel, with 16 consecutive pixels as
+// rows; wf: the weights as [ci][(ky*3 + kx)*CO + co] (weights_flip_kernel).
+// Bound by its gradient loads; every input-channel tile in one wave reads
+// them once (64 -> 32 channels, 256 snippets: 98 us, 158 with a wave per
+// tile; 32 -> 16: 78 us, 148 as an im2col product).
+template <int CO, int CI, int NB>
+__global__ __launch_bounds__(NT) void conv_dx_kernel(const uint16_t *__restrict__ dz,
+                                                     const uint16_t *__restrict__ wf, int64_t P, int H,
+                                                     int W, int run, float *__restrict__ dx) {
+  constexpr int KC = 9 * CO / 16;
+  const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.y * NB * 16;
+  bf16x4 bw[KC][NB];
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
-      dz[((b * H + 2 * ho + (k >> 1)) * W + 2 * wo + (k & 1)) * C + c] = (k == (q & 3)) ? g : (uint16_t)0;
+  for (int c = 0; c < KC; ++c)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) bw[c][j] = load4(wf + (int64_t)(n0 + 16 * j + n) * (9 * CO) + 16 * c + 4 * g);
+  const int64_t wave = (int64_t)blockIdx.x * (NT / 64) + (threadIdx.x >> 6);
+  int64_t p = wave * run * 16;
+  const int64_t pend = p + (int64_t)run * 16 < P ? p + (int64_t)run * 16 : P;
+  if (p >= pend) return;
+  Pixel px;
+  px.set(p + n < P ? p + n : P - 1, H, W);
+  for (; p < pend; p += 16) {
+    const uint16_t *q = dz + ((px.b * H + px.h) * W + px.w) * CO;
+    f32x4 acc[NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // the loads of HALF steps are issued together ahead of their products
+    constexpr int HALF = KC > 18 ? KC / 2 : KC;
+#pragma unroll
+    for (int c0 = 0; c0 < KC; c0 += HALF) {
+      bf16x4 av[HALF];
+#pragma unroll
+      for (int c = 0; c < HALF; ++c) {
+        const int t = (c0 + c) / (CO / 16), cc = (c0 + c) % (CO / 16);
+        const int ky = t / 3, kx = t - 3 * ky;  // reads (h - ky + 1, w - kx + 1)
+        const bool ok = (ky != 2 || px.h > 0) && (ky != 0 || px.h < H - 1) && (kx != 2 || px.w > 0) &&
+                        (kx != 0 || px.w < W - 1);
+        av[c] = load4(q + (ok ? ((1 - ky) * W + (1 - kx)) * CO : 0) + 16 * cc + 4 * g);
+        if (!ok) av[c] = bf16x4{0, 0, 0, 0};
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int c = 0; c < HALF; ++c)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+          acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av[c], bw[c0 + c][j], acc[j], 0, 0, 0);
+    }
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int64_t o = p + 4 * g + r;
+        if (o < P) dx[o * CI + n0 + 16 * j + n] = acc[j][r];
+      }
+    px.advance(16, H, W);
+    if (p + 16 + n >= P) px.set(P - 1, H, W);
+  }
+}
+
+// w[co][tap*CI + ci] -> wf[ci][tap*CO + co]
+__global__ void weights_flip_kernel(const uint16_t *__restrict__ w, int CI, int CO, uint16_t *__restrict__ wf) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= 9 * CI * CO) return;
+  const int ci = i / (9 * CO), r = i - ci * 9 * CO, t = r / CO, co = r - t * CO;
+  wf[i] = w[co * 9 * CI + t * CI + ci];
+}
+
+// Weight gradient of a 3x3 convolution, dw[co][tap*CI + ci] = sum over pixels
+// of dz[pix][co] * x[pix moved by the tap][ci]: a product with the pixels as
+// the reduction, so both operands need 4 consecutive pixels of one channel
+// per lane while the activations are stored channel by channel of a pixel.
+// A workgroup stages WR rows x WC columns of dz and of x (with a border) in
+// LDS and its lanes gather the pixels with 2-byte reads; the three taps of a
+// kernel row share one window of 6 pixels.  The pixel pitch is 8 bytes more
+// than the channels take, which spreads the four 16-lane groups (4 pixels
+// apart) over the banks.  A wave owns CT output-channel tiles x 9*CI/16
+// column tiles (72 accumulator registers); with CO > 16 CT the waves split the
+// output channels, and otherwise the workgroup's pixels (their sums are added
+// in LDS).  Each workgroup writes one partial; sum_rows_kernel adds them.
+// Bound by the 2-byte LDS reads: 256 snippets 73 + 5 us (32 channels) and 46
+// + 13 us (64), 377 and 187 as split im2col products.
+constexpr int WR = 2, WC = 64;
+template <int CI, int CO, int CT>
+__global__ __launch_bounds__(NT) void conv_dw_kernel(const uint16_t *__restrict__ dz,
+                                                     const uint16_t *__restrict__ x, int64_t B, int H,
+                                                     int W, float *__restrict__ part) {
+  constexpr int PZ = CO + 4, PX = CI + 4;      // pixel pitch (elements)
+  constexpr int NTILE = 9 * CI / 16, CS = CO / (16 * CT);  // column tiles; waves over co
+  constexpr int KS = (NT / 64) / CS;           // waves over pixels
+  constexpr int XW = WC + 2;
+  __shared__ __align__(16) uint16_t sz[WR * WC * PZ];
+  __shared__ __align__(16) uint16_t sx[(WR + 2) * XW * PX];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 15, g = lane >> 4;
+  const int ws = wave % CS, kw = wave / CS;
+  f32x4 acc[CT][NTILE];
+#pragma unroll
+  for (int i = 0; i < CT; ++i)
+#pragma unroll
+    for (int j = 0; j < NTILE; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int nh = (H + WR - 1) / WR, nw = (W + WC - 1) / WC;
+  const int64_t items = B * nh * nw;
+  for (int64_t it = blockIdx.x; it < items; it += gridDim.x) {
+    const int iw = (int)(it % nw);
+    const int64_t r0 = it / nw;
+    const int ih = (int)(r0 % nh);
+    const int64_t b = r0 / nh;
+    const int h0 = ih * WR, w0 = iw * WC;
+    __syncthreads();
+    for (int i = threadIdx.x; i < WR * WC * (CO / 4); i += NT) {
+      const int c = i % (CO / 4), q = i / (CO / 4), ww = q % WC, hh = q / WC;
+      uint2 v = make_uint2(0u, 0u);
+      if (h0 + hh < H && w0 + ww < W)
+        v = *reinterpret_cast<const uint2 *>(dz + ((b * H + h0 + hh) * W + w0 + ww) * CO + 4 * c);
+      *reinterpret_cast<uint2 *>(sz + (hh * WC + ww) * PZ + 4 * c) = v;
+    }
+    for (int i = threadIdx.x; i < (WR + 2) * XW * (CI / 4); i += NT) {
+      const int c = i % (CI / 4), q = i / (CI / 4), ww = q % XW, hh = q / XW;
+      const int hs = h0 + hh - 1, wsrc = w0 + ww - 1;
+      uint2 v = make_uint2(0u, 0u);
+      if (hs >= 0 && hs < H && wsrc >= 0 && wsrc < W)
+        v = *reinterpret_cast<const uint2 *>(x + ((b * H + hs) * W + wsrc) * CI + 4 * c);
+      *reinterpret_cast<uint2 *>(sx + (hh * XW + ww) * PX + 4 * c) = v;
+    }
+    __syncthreads();
+    for (int ks = kw; ks < WR * WC / 16; ks += KS) {
+      const int hh = ks / (WC / 16), wb = (ks % (WC / 16)) * 16 + 4 * g;  // this lane's first pixel
+      bf16x4 av[CT];
+#pragma unroll
+      for (int i = 0; i < CT; ++i) {
+        const uint16_t *q = sz + (hh * WC + wb) * PZ + (ws * CT + i) * 16 + n;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) av[i][e] = (short)q[e * PZ];
+      }
+#pragma unroll
+      for (int ky = 0; ky < 3; ++ky)
+#pragma unroll
+        for (int cc = 0; cc < CI / 16; ++cc) {
+          const uint16_t *q = sx + ((hh + ky) * XW + wb) * PX + 16 * cc + n;
+          short v[6];
+#pragma unroll
+          for (int e = 0; e < 6; ++e) v[e] = (short)q[e * PX];
+#pragma unroll
+          for (int kx = 0; kx < 3; ++kx) {
+            const bf16x4 bv = {v[kx], v[kx + 1], v[kx + 2], v[kx + 3]};
+            const int j = (ky * 3 + kx) * (CI / 16) + cc;
+#pragma unroll
+            for (int i = 0; i < CT; ++i)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av[i], bv, acc[i][j], 0, 0, 0);
+          }
+        }
+    }
+  }
+  // D: column n = (tap, ci) of tile j, rows 4g + r = co of tile i
+  float *o = part + (int64_t)blockIdx.x * (CO * 9 * CI);
+  auto at = [&](int i, int j, int r) { return ((ws * CT + i) * 16 + 4 * g + r) * 9 * CI + 16 * j + n; };
+  if constexpr (KS == 1) {
+#pragma unroll
+    for (int i = 0; i < CT; ++i)
+#pragma unroll
+      for (int j = 0; j < NTILE; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[at(i, j, r)] = acc[i][j][r];
+  } else {
+    __shared__ float sum[KS == 1 ? 1 : CO * 9 * CI];
+    for (int w = 0; w < KS; ++w) {
+      __syncthreads();
+      if (kw == w) {
+#pragma unroll
+        for (int i = 0; i < CT; ++i)
+#pragma unroll
+          for (int j = 0; j < NTILE; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              float *q = sum + at(i, j, r);
+              *q = w ? *q + acc[i][j][r] : acc[i][j][r];
+            }
+      }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < CO * 9 * CI; i += NT) o[i] = sum[i];
+  }
+}
+
+// First layer (2 input channels, no input gradient): weight and bias gradients
+// straight from the pooled gradient.  Only the argmax pixel of a pool window
+// has a gradient, so each (pooled pixel, output channel) is 18 multiply-adds
+// with the 3x3 neighbourhood of that pixel, and neither the full-resolution
+// gradient (134 MB for 256 snippets) nor a product over all pixels is formed.
+// Thread t: channel t % 16, every 16th pooled pixel of a row chunk whose
+// input pixels (both channels in one word) are staged with a border in LDS.
+// Products of BF16 values, FP32 sums; part[block][288 weights, 16 biases].
+// 256 snippets: 75 us, against 670 for the pool's backward, its column sums
+// and the product over all pixels.
+constexpr int W1C = 128;  // pooled columns per chunk
+__global__ __launch_bounds__(NT) void conv1_dw_kernel(const float *__restrict__ da,
+                                                      const uint8_t *__restrict__ idx,
+                                                      const uint32_t *__restrict__ x, int64_t B, int H,
+                                                      int W, float *__restrict__ part) {
+  constexpr int XW = 2 * W1C + 2;
+  __shared__ uint32_t sx[4 * XW];
+  __shared__ float red[4][16][19];
+  const int co = threadIdx.x & 15, slot = threadIdx.x >> 4;
+  const int Ho = H / 2, Wo = W / 2, nc = (Wo + W1C - 1) / W1C;
+  float acc[18], bsum = 0.f;
+#pragma unroll
+  for (int k = 0; k < 18; ++k) acc[k] = 0.f;
+  const int64_t items = B * Ho * nc;
+  for (int64_t it = blockIdx.x; it < items; it += gridDim.x) {
+    const int ic = (int)(it % nc);
+    const int64_t bh = it / nc;  // b * Ho + ho
+    const int ho = (int)(bh % Ho);
+    const int64_t b = bh / Ho;
+    const int c0 = ic * W1C, cols = Wo - c0 < W1C ? Wo - c0 : W1C;
+    __syncthreads();
+    for (int i = threadIdx.x; i < 4 * XW; i += NT) {
+      const int hh = i / XW, ww = i - hh * XW;
+      const int h = 2 * ho - 1 + hh, w = 2 * c0 - 1 + ww;
+      sx[i] = (h >= 0 && h < H && w >= 0 && w < W) ? x[(b * H + h) * W + w] : 0u;
+    }
+    __syncthreads();
+    for (int c = slot; c < cols; c += 16) {
+      const int64_t o = (bh * Wo + c0 + c) * 16 + co;
+      const uint8_t q = idx[o];
+      const float gr = (q & 4) ? from_bf16(to_bf16(da[o])) : 0.f;
+      const uint32_t *s = sx + ((q >> 1) & 1) * XW + 2 * c + (q & 1);
+      bsum += gr;
+#pragma unroll
+      for (int t = 0; t < 9; ++t) {
+        const uint32_t v = s[(t / 3) * XW + t % 3];
+        acc[2 * t] = __builtin_fmaf(gr, __uint_as_float(v << 16), acc[2 * t]);
+        acc[2 * t + 1] = __builtin_fmaf(gr, __uint_as_float(v & 0xFFFF0000u), acc[2 * t + 1]);
+      }
+    }
+  }
+  // lanes 16 and 32 apart hold the same channel, then the four waves
+#pragma unroll
+  for (int k = 0; k < 19; ++k) {
+    float v = k < 18 ? acc[k] : bsum;
+    v += __shfl_xor(v, 16);
+    v += __shfl_xor(v, 32);
+    if ((threadIdx.x & 63) < 16) red[threadIdx.x >> 6][co][k] = v;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < 16 * 19; i += NT) {
+    const int c = i / 19, k = i - c * 19;
+    const float v = (red[0][c][k] + red[1][c][k]) + (red[2][c][k] + red[3][c][k]);
+    part[(int64_t)blockIdx.x * 304 + (k < 18 ? c * 18 + k : 288 + c)] = v;
+  }
+}
+
+// Backward of ReLU + pool with the bias gradient: da[B][H/2][W/2][C] (FP32)
+// -> dz[B][H][W][C] (BF16, the gradient at the argmax when it was positive,
+// zeros elsewhere) and per-workgroup sums of the BF16 gradients per channel.
+// A thread takes 8 channels of a pooled pixel (16-byte stores).
+template <int C>
+__global__ __launch_bounds__(NT) void pool_bwd_kernel(const float *__restrict__ da,
+                                                      const uint8_t *__restrict__ idx, int64_t P, int H,
+                                                      int W, uint16_t *__restrict__ dz,
+                                                      float *__restrict__ part) {
+  constexpr int G = C / 8;  // channel groups
+  __shared__ float s[NT * 8];
+  const int Ho = H / 2, Wo = W / 2;
+  const int cg = threadIdx.x % G;
+  float sum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  for (int64_t p = (int64_t)blockIdx.x * (NT / G) + threadIdx.x / G; p < P;
+       p += (int64_t)gridDim.x * (NT / G)) {
+    const float4 v0 = *reinterpret_cast<const float4 *>(da + p * C + 8 * cg);
+    const float4 v1 = *reinterpret_cast<const float4 *>(da + p * C + 8 * cg + 4);
+    const uint2 qq = *reinterpret_cast<const uint2 *>(idx + p * C + 8 * cg);
+    const float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+    uint32_t gr[8], q[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      q[e] = ((e < 4 ? qq.x : qq.y) >> (8 * (e & 3))) & 7u;
+      gr[e] = (q[e] & 4u) ? (uint32_t)to_bf16(v[e]) : 0u;
+      sum[e] += from_bf16((uint16_t)gr[e]);
+    }
+    const int64_t bh = p / Wo;
+    const int wo = (int)(p - bh * Wo);
+    const int64_t b = bh / Ho;
+    const int ho = (int)(bh - b * Ho);
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; ++k) {
+      uint32_t o[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        o[e] = ((q[2 * e] & 3u) == k ? gr[2 * e] : 0u) | ((q[2 * e + 1] & 3u) == k ? gr[2 * e + 1] << 16 : 0u);
+      *reinterpret_cast<uint4 *>(dz + ((b * H + 2 * ho + (k >> 1)) * W + 2 * wo + (k & 1)) * C + 8 * cg) =
+          make_uint4(o[0], o[1], o[2], o[3]);
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) s[(threadIdx.x / G) * C + 8 * cg + e] = sum[e];
+  __syncthreads();
+  for (int c = threadIdx.x; c < C; c += NT) {
+    float v = 0.f;
+    for (int r = 0; r < NT / G; ++r) v += s[r * C + c];
+    part[(int64_t)blockIdx.x * C + c] = v;
+  }
+}
+
+// out[j] = sum over rows of part[row][j]: 16 columns per workgroup, 16 rows at
+// a time, 8 loads in flight per thread
+__global__ __launch_bounds__(NT) void sum_rows_kernel(const float *__restrict__ part, int rows, int n,
+                                                      float *__restrict__ out) {
+  __shared__ float s[16][17];
+  const int c = threadIdx.x & 15, r0 = threadIdx.x >> 4;
+  const int j = blockIdx.x * 16 + c;
+  float v = 0.f;
+  if (j < n) {
+    int r = r0;
+    for (; r + 7 * 16 < rows; r += 8 * 16) {
+      float t[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) t[u] = part[(int64_t)(r + 16 * u) * n + j];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v += t[u];
+    }
+    for (; r < rows; r += 16) v += part[(int64_t)r * n + j];
+  }
+  s[r0][c] = v;
+  __syncthreads();
+  if (r0 == 0 && j < n) {
+    float t = 0.f;
+    for (int r = 0; r < 16; ++r) t += s[r][c];
+    out[j] = t;
   }
 }
 
@@ -378,19 +744,41 @@ __global__ void to_bf16_kernel(const float *__restrict__ x, uint16_t *__restrict
     y[i] = to_bf16(x[i]);
 }
 
-// x[B][C][H][W] -> y[B][H][W][C]
-__global__ void nchw_to_nhwc_kernel(const uint16_t *__restrict__ x, int64_t B, int C, int H, int W,
-                                    uint16_t *__restrict__ y) {
-  const int64_t n = B * C * H * W;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
+// x[B][2][HW] -> y[B][HW][2], four pixels per thread (HW is a multiple of 64)
+__global__ void nchw2_to_nhwc_kernel(const uint16_t *__restrict__ x, int64_t n4, int64_t HW4,
+                                     uint16_t *__restrict__ y) {
+  typedef uint16_t u16x4 __attribute__((ext_vector_type(4), aligned(2)));
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n4;
        i += (int64_t)gridDim.x * blockDim.x) {
-    const int c = (int)(i % C);
-    int64_t r = i / C;
-    const int w = (int)(r % W);
-    r /= W;
-    const int h = (int)(r % H);
-    const int64_t b = r / H;
-    y[i] = x[((b * C + c) * H + h) * W + w];
+    const int64_t b = i / HW4, r = i - b * HW4;
+    const uint16_t *p = x + (b * 2 * HW4 + r) * 4;
+    const u16x4 u = *reinterpret_cast<const u16x4 *>(p), v = *reinterpret_cast<const u16x4 *>(p + HW4 * 4);
+    reinterpret_cast<uint4 *>(y)[i] =
+        make_uint4(u[0] | (uint32_t)v[0] << 16, u[1] | (uint32_t)v[1] << 16, u[2] | (uint32_t)v[2] << 16,
+                   u[3] | (uint32_t)v[3] << 16);
+  }
+}
+
+// Parameters or gradients from the device layout to the canonical one: conv
+// weights [co][ci][tap] from [co][tap][ci] and fc1 columns [c][y][x] from
+// [y][x][c].  Segments: L.w[k] and L.fw1 as offsets, everything else in place.
+__global__ void canonical_kernel(const float *__restrict__ src, CanonicalLayout L, float *__restrict__ out) {
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < L.n;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    int64_t j = i;
+    for (int k = 0; k < 3; ++k) {
+      const int64_t r = i - L.w[k];
+      if (r >= 0 && r < (int64_t)9 * L.ci[k] * L.co[k]) {
+        const int t = (int)(r % 9), ci = (int)(r / 9 % L.ci[k]);
+        j = L.w[k] + r / (9 * L.ci[k]) * 9 * L.ci[k] + t * L.ci[k] + ci;
+      }
+    }
+    const int64_t r = i - L.fw1;
+    if (r >= 0 && r < (int64_t)L.fin * L.hid) {
+      const int64_t o = r / L.fin, e = r - o * L.fin;
+      j = L.fw1 + o * L.fin + e % L.pix * L.chan + e / L.pix;
+    }
+    out[i] = src[j];
   }
 }
 
@@ -425,47 +813,100 @@ int gemm_dense(const uint16_t *a, int64_t asr, int64_t asc, const uint16_t *b, i
   return gemm(Dense{a, asr, asc}, Dense{b, bsr, bsc}, M, N, K, splits, C, s);
 }
 
-int conv_forward(const uint16_t *x, int64_t B, int H, int W, int Ci, const uint16_t *w, int Co,
-                 float *z, hipStream_t s) {
-  // z[pix][co] = sum_k im2col(x)[pix][k] * w[co][k]
-  return gemm(Im2col<false>{x, H, W, Ci}, Dense{w, 1, (int64_t)9 * Ci}, B * H * W, Co,
-              (int64_t)9 * Ci, 1, z, s);
+namespace {
+
+// tiles per wave: runs of up to `most` while 4096 waves remain
+int run_of(int64_t tiles, int most) {
+  const int64_t r = tiles / 4096;
+  return (int)(r < 1 ? 1 : (r > most ? most : r));
 }
 
-int conv_weight_grad(const uint16_t *dz, const uint16_t *x, int64_t B, int H, int W, int Ci, int Co,
-                     int splits, float *part, hipStream_t s) {
-  // dw[co][k] = sum_pix dz[pix][co] * im2col(x)[pix][k]
-  return gemm(Dense{dz, 1, Co}, Im2col<false>{x, H, W, Ci}, Co, (int64_t)9 * Ci, B * H * W, splits,
-              part, s);
+int sum_rows(const float *part, int rows, int n, float *out, hipStream_t s) {
+  hipLaunchKernelGGL(sum_rows_kernel, dim3((n + 15) / 16), dim3(NT), 0, s, part, rows, n, out);
+  MDSM_HIP(hipGetLastError());
+  return MDSM_OK;
 }
 
-int conv_input_grad(const uint16_t *dz, int64_t B, int H, int W, int Ci, int Co, const uint16_t *w,
-                    float *dx, hipStream_t s) {
-  // dx[pix][ci] = sum_{ky,kx,co} dz[pix shifted back][co] * w[co][ky,kx,ci]
-  return gemm(Im2col<true>{dz, H, W, Co}, WFlip{w, Ci, Co}, B * H * W, Ci, (int64_t)9 * Co, 1, dx,
-              s);
+}  // namespace
+
+int conv_pool(int layer, const uint16_t *x, int64_t B, int H, int W, const uint16_t *w, const float *bias,
+              uint16_t *a, uint8_t *idx, hipStream_t s) {
+  const int64_t P = B * (H / 2) * (W / 2), tiles = (P + 3) / 4;
+  const int run = run_of(tiles, 8);
+  const unsigned gx = (unsigned)((tiles + (int64_t)run * 4 - 1) / ((int64_t)run * 4));
+  switch (layer) {
+    case 0: hipLaunchKernelGGL((conv_pool_kernel<2, 16, 1>), dim3(gx, 1), dim3(NT), 0, s, x, w, bias, P, H, W, run, a, idx); break;
+    case 1: hipLaunchKernelGGL((conv_pool_kernel<16, 32, 2>), dim3(gx, 1), dim3(NT), 0, s, x, w, bias, P, H, W, run, a, idx); break;
+    default:
+      // all four output tiles in one wave read the activations once (256
+      // snippets of 64 x 256: 41 us, 53 with two waves of two tiles); with
+      // few tiles the second wave is worth more (24 snippets: 12 against 13)
+      if (tiles >= 8192)
+        hipLaunchKernelGGL((conv_pool_kernel<32, 64, 4>), dim3(gx, 1), dim3(NT), 0, s, x, w, bias, P, H, W, run, a, idx);
+      else
+        hipLaunchKernelGGL((conv_pool_kernel<32, 64, 2>), dim3(gx, 2), dim3(NT), 0, s, x, w, bias, P, H, W, run, a, idx);
+      break;
+  }
+  MDSM_HIP(hipGetLastError());
+  return MDSM_OK;
+}
+
+int conv_dx(int layer, const uint16_t *dz, int64_t B, int H, int W, const uint16_t *w, uint16_t *wf, float *dx,
+            hipStream_t s) {
+  const int CI = layer == 1 ? 16 : 32, CO = 2 * CI;
+  hipLaunchKernelGGL(weights_flip_kernel, dim3((9 * CI * CO + NT - 1) / NT), dim3(NT), 0, s, w, CI, CO, wf);
+  MDSM_HIP(hipGetLastError());
+  const int64_t P = B * H * W, tiles = (P + 15) / 16;
+  const int run = run_of(tiles, 8);
+  const unsigned gx = (unsigned)((tiles + (int64_t)run * 4 - 1) / ((int64_t)run * 4));
+  if (layer == 1) hipLaunchKernelGGL((conv_dx_kernel<32, 16, 1>), dim3(gx, 1), dim3(NT), 0, s, dz, wf, P, H, W, run, dx);
+  else hipLaunchKernelGGL((conv_dx_kernel<64, 32, 2>), dim3(gx, 1), dim3(NT), 0, s, dz, wf, P, H, W, run, dx);
+  MDSM_HIP(hipGetLastError());
+  return MDSM_OK;
+}
+
+int64_t conv_dw_floats() { return (int64_t)DW_BLOCKS * 64 * 288; }
+
+int conv_dw(int layer, const uint16_t *dz, const uint16_t *x, int64_t B, int H, int W, float *part, float *dw,
+            hipStream_t s) {
+  const int64_t items = B * ((H + WR - 1) / WR) * ((W + WC - 1) / WC);
+  const int blocks = (int)(items < DW_BLOCKS ? items : DW_BLOCKS);
+  if (layer == 1) hipLaunchKernelGGL((conv_dw_kernel<16, 32, 2>), dim3(blocks), dim3(NT), 0, s, dz, x, B, H, W, part);
+  else hipLaunchKernelGGL((conv_dw_kernel<32, 64, 1>), dim3(blocks), dim3(NT), 0, s, dz, x, B, H, W, part);
+  MDSM_HIP(hipGetLastError());
+  return sum_rows(part, blocks, layer == 1 ? 32 * 144 : 64 * 288, dw, s);
+}
+
+int conv1_dw(const float *da, const uint8_t *idx, const uint16_t *x, int64_t B, int H, int W, float *part,
+             float *dwb, hipStream_t s) {
+  const int64_t items = B * (H / 2) * ((W / 2 + W1C - 1) / W1C);
+  const int blocks = (int)(items < 1024 ? items : 1024);
+  hipLaunchKernelGGL(conv1_dw_kernel, dim3(blocks), dim3(NT), 0, s, da, idx,
+                     reinterpret_cast<const uint32_t *>(x), B, H, W, part);
+  MDSM_HIP(hipGetLastError());
+  return sum_rows(part, blocks, 304, dwb, s);
+}
+
+int pool_backward(const float *da, const uint8_t *idx, int64_t B, int H, int W, int C, uint16_t *dz, float *part,
+                  float *db, hipStream_t s) {
+  const int64_t P = B * (H / 2) * (W / 2), per = NT / (C / 8), want = (P + per - 1) / per;
+  const int blocks = (int)(want < 1024 ? want : 1024);
+  if (C == 32) hipLaunchKernelGGL(pool_bwd_kernel<32>, dim3(blocks), dim3(NT), 0, s, da, idx, P, H, W, dz, part);
+  else hipLaunchKernelGGL(pool_bwd_kernel<64>, dim3(blocks), dim3(NT), 0, s, da, idx, P, H, W, dz, part);
+  MDSM_HIP(hipGetLastError());
+  return sum_rows(part, blocks, C, db, s);
+}
+
+int to_canonical(const float *src, const CanonicalLayout &L, float *out, hipStream_t s) {
+  hipLaunchKernelGGL(canonical_kernel, dim3(grid1d(L.n)), dim3(NT), 0, s, src, L, out);
+  MDSM_HIP(hipGetLastError());
+  return MDSM_OK;
 }
 
 int epilogue(const float *part, int splits, int64_t M, int64_t N, const float *bias, float *out_f32,
              const float *mask, int relu, uint16_t *out_bf16, hipStream_t s) {
   hipLaunchKernelGGL(epilogue_kernel, dim3(grid1d(M * N)), dim3(NT), 0, s, part, splits, M, N, bias,
                      out_f32, mask, relu, out_bf16);
-  MDSM_HIP(hipGetLastError());
-  return MDSM_OK;
-}
-
-int relu_pool(const float *z, const float *bias, int64_t B, int H, int W, int C, uint16_t *a,
-              uint8_t *idx, hipStream_t s) {
-  hipLaunchKernelGGL(relu_pool_kernel, dim3(grid1d(B * (H / 2) * (W / 2) * C)), dim3(NT), 0, s, z,
-                     bias, B, H, W, C, a, idx);
-  MDSM_HIP(hipGetLastError());
-  return MDSM_OK;
-}
-
-int pool_backward(const float *da, const uint8_t *idx, int64_t B, int H, int W, int C, uint16_t *dz,
-                  hipStream_t s) {
-  hipLaunchKernelGGL(pool_bwd_kernel, dim3(grid1d(B * (H / 2) * (W / 2) * C)), dim3(NT), 0, s, da,
-                     idx, B, H, W, C, dz);
   MDSM_HIP(hipGetLastError());
   return MDSM_OK;
 }
@@ -506,9 +947,9 @@ int to_bf16(const float *x, uint16_t *y, int64_t n, hipStream_t s) {
   return MDSM_OK;
 }
 
-int nchw_to_nhwc(const uint16_t *x, int64_t B, int C, int H, int W, uint16_t *y, hipStream_t s) {
-  hipLaunchKernelGGL(nchw_to_nhwc_kernel, dim3(grid1d(B * C * H * W)), dim3(NT), 0, s, x, B, C, H,
-                     W, y);
+int nchw2_to_nhwc(const uint16_t *x, int64_t B, int64_t HW, uint16_t *y, hipStream_t s) {
+  const int64_t n4 = B * HW / 4;
+  hipLaunchKernelGGL(nchw2_to_nhwc_kernel, dim3(grid1d(n4)), dim3(NT), 0, s, x, n4, HW / 4, y);
   MDSM_HIP(hipGetLastError());
   return MDSM_OK;
 }

@@ -63,9 +63,9 @@ struct mdsm_cnn_s {
   uint16_t *pb = nullptr;
   uint16_t *x = nullptr, *a[4] = {nullptr, nullptr, nullptr, nullptr};
   uint8_t *idx[3] = {nullptr, nullptr, nullptr};
-  float *z = nullptr, *z4 = nullptr, *logits = nullptr, *dA = nullptr, *part = nullptr;
+  float *canon = nullptr, *z4 = nullptr, *logits = nullptr, *dA = nullptr, *part = nullptr;
   float *cpart = nullptr, *loss = nullptr;
-  uint16_t *h = nullptr, *dl = nullptr, *dh = nullptr, *dZ = nullptr;
+  uint16_t *h = nullptr, *dl = nullptr, *dh = nullptr, *dZ = nullptr, *wf = nullptr;
   int64_t part_floats = 0;
   int last_batch = 0;
   int step = 0;
@@ -133,16 +133,16 @@ extern "C" int mdsm_cnn_create(int height, int width, int max_batch, mdsm_cnn *o
   need(NCLS, HID, B);          // fc2 weight grad
   need(B, HID, NCLS);          // fc2 input grad
   need(HID, n->L.fin, B);      // fc1 weight grad
-  for (int k = 0; k < 3; ++k)  // conv weight grads
-    need(CH[k + 1], 9 * CH[k], B * (HW >> (2 * k)));
+  pf = std::max(pf, cnn::conv_dw_floats());
   n->part_floats = pf;
   bool ok = dalloc(n, &n->p, n->L.n) && dalloc(n, &n->g, n->L.n) && dalloc(n, &n->m, n->L.n) &&
             dalloc(n, &n->v, n->L.n) && dalloc(n, &n->pb, n->L.n) && dalloc(n, &n->x, B * HW * 2) &&
-            dalloc(n, &n->z, B * HW * 16) && dalloc(n, &n->z4, B * HID) &&
+            dalloc(n, &n->canon, n->L.n) && dalloc(n, &n->wf, 64 * 288) &&
+            dalloc(n, &n->z4, B * HID) &&
             dalloc(n, &n->logits, B * NCLS) && dalloc(n, &n->dA, B * HW * 4) &&
-            dalloc(n, &n->part, pf) && dalloc(n, &n->cpart, 1024 * 64) && dalloc(n, &n->loss, 1) &&
+            dalloc(n, &n->part, pf) && dalloc(n, &n->cpart, 1024 * 304) && dalloc(n, &n->loss, 1) &&
             dalloc(n, &n->h, B * HID) && dalloc(n, &n->dl, B * NCLS) && dalloc(n, &n->dh, B * HID) &&
-            dalloc(n, &n->dZ, B * HW * 16);
+            dalloc(n, &n->dZ, B * HW * 8);
   for (int k = 0; k < 3 && ok; ++k) {
     const int64_t cnt = B * (HW >> (2 * (k + 1))) * CH[k + 1];
     ok = dalloc(n, &n->a[k + 1], cnt) && dalloc(n, &n->idx[k], cnt);
@@ -192,13 +192,27 @@ extern "C" int mdsm_cnn_set_params(mdsm_cnn n, const float *host) {
   return rc;
 }
 
+// (the layouts are exchanged on the device: one pass and one copy instead of
+// a copy, an index map and a gather on the host)
 static int get_canonical(mdsm_cnn n, const float *dsrc, float *host) {
   MDSM_REQUIRE(n && host, MDSM_ERR_ARG, "null argument");
-  std::vector<float> dev(n->L.n);
+  const Layout &L = n->L;
+  cnn::CanonicalLayout c{};
+  for (int k = 0; k < 3; ++k) {
+    c.w[k] = L.w[k];
+    c.ci[k] = CH[k];
+    c.co[k] = CH[k + 1];
+  }
+  c.fw1 = L.fw1;
+  c.n = L.n;
+  c.fin = L.fin;
+  c.hid = HID;
+  c.pix = (n->H / 8) * (n->W / 8);
+  c.chan = CH[3];
   MDSM_HIP(hipDeviceSynchronize());
-  MDSM_HIP(hipMemcpy(dev.data(), dsrc, n->L.n * 4, hipMemcpyDeviceToHost));
-  const auto map = device_index(n);
-  for (int64_t i = 0; i < n->L.n; ++i) host[i] = dev[map[i]];
+  const int rc = cnn::to_canonical(dsrc, c, n->canon, nullptr);
+  if (rc != MDSM_OK) return rc;
+  MDSM_HIP(hipMemcpy(host, n->canon, L.n * 4, hipMemcpyDeviceToHost));
   return MDSM_OK;
 }
 
@@ -229,12 +243,10 @@ extern "C" int mdsm_cnn_forward(mdsm_cnn n, const uint16_t *d_x, uint32_t batch,
   hipStream_t s = as_stream(stream);
   const int64_t B = batch;
   const Layout &L = n->L;
-  int rc = cnn::nchw_to_nhwc(d_x, B, 2, n->H, n->W, n->x, s);
-  for (int k = 0; k < 3 && rc == MDSM_OK; ++k) {
-    const int Hk = n->H >> k, Wk = n->W >> k;
-    rc = cnn::conv_forward(n->a[k], B, Hk, Wk, CH[k], n->pb + L.w[k], CH[k + 1], n->z, s);
-    if (rc == MDSM_OK) rc = cnn::relu_pool(n->z, n->p + L.b[k], B, Hk, Wk, CH[k + 1], n->a[k + 1], n->idx[k], s);
-  }
+  int rc = cnn::nchw2_to_nhwc(d_x, B, (int64_t)n->H * n->W, n->x, s);
+  for (int k = 0; k < 3 && rc == MDSM_OK; ++k)
+    rc = cnn::conv_pool(k, n->a[k], B, n->H >> k, n->W >> k, n->pb + L.w[k], n->p + L.b[k], n->a[k + 1],
+                        n->idx[k], s);
   if (rc == MDSM_OK) {  // fc1: z4 = a3 fw1^T + fb1, h = relu(z4)
     const int sp = choose_splits(B, HID, L.fin);
     rc = cnn::gemm_dense(n->a[3], L.fin, 1, n->pb + L.fw1, 1, L.fin, B, HID, L.fin, sp, n->part, s);
@@ -284,19 +296,13 @@ extern "C" int mdsm_cnn_backward(mdsm_cnn n, const int32_t *d_labels, uint32_t b
   if (rc == MDSM_OK) rc = cnn::column_sums(n->dh, B, HID, n->cpart, 1024, n->g + L.fb1, s);
   if (rc == MDSM_OK) rc = cnn::gemm_dense(n->dh, HID, 1, n->pb + L.fw1, L.fin, 1, B, L.fin, HID, 1, n->dA, s);
   // conv stack, top down: dA holds the gradient of the layer's pooled output
-  for (int k = 2; k >= 0 && rc == MDSM_OK; --k) {
-    const int Hk = n->H >> k, Wk = n->W >> k, Ci = CH[k], Co = CH[k + 1];
-    const int64_t P = B * Hk * Wk;
-    rc = cnn::pool_backward(n->dA, n->idx[k], B, Hk, Wk, Co, n->dZ, s);
-    if (rc == MDSM_OK) rc = cnn::column_sums(n->dZ, P, Co, n->cpart, 1024, n->g + L.b[k], s);
-    if (rc == MDSM_OK) {
-      const int sp = choose_splits(Co, 9 * Ci, P);
-      rc = cnn::conv_weight_grad(n->dZ, n->a[k], B, Hk, Wk, Ci, Co, sp, n->part, s);
-      if (rc == MDSM_OK)
-        rc = cnn::epilogue(n->part, cnn::splits_used(P, sp), Co, 9 * Ci, nullptr, n->g + L.w[k], nullptr, 0, nullptr, s);
-    }
-    if (rc == MDSM_OK && k > 0) rc = cnn::conv_input_grad(n->dZ, B, Hk, Wk, Ci, Co, n->pb + L.w[k], n->dA, s);
+  for (int k = 2; k >= 1 && rc == MDSM_OK; --k) {
+    const int Hk = n->H >> k, Wk = n->W >> k;
+    rc = cnn::pool_backward(n->dA, n->idx[k], B, Hk, Wk, CH[k + 1], n->dZ, n->cpart, n->g + L.b[k], s);
+    if (rc == MDSM_OK) rc = cnn::conv_dw(k, n->dZ, n->a[k], B, Hk, Wk, n->part, n->g + L.w[k], s);
+    if (rc == MDSM_OK) rc = cnn::conv_dx(k, n->dZ, B, Hk, Wk, n->pb + L.w[k], n->wf, n->dA, s);
   }
+  if (rc == MDSM_OK) rc = cnn::conv1_dw(n->dA, n->idx[0], n->x, B, n->H, n->W, n->cpart, n->g + L.w[0], s);
   return rc;
 }
 
