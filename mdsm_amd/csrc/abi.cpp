@@ -293,14 +293,28 @@ static bool variant_fits(const mdsm_plan_s *p, int v) {
 static int default_variant(const mdsm_plan_s *p) {
   const int pref = preferred_variant(p->dtype);
   if (variant_fits(p, pref)) return pref;
-  const int fb = fallback_variant(p->dtype);
-  if (variant_fits(p, fb)) return fb;
-  for (int v = 1; v < (int)p->row_words.size(); ++v)
+  for (int n = 0, fb; (fb = fallback_variant(p->dtype, n)) != 0; ++n)
+    if (variant_fits(p, fb)) return fb;
+  for (int v = 1; v <= num_variants(p->dtype); ++v)
     if (variant_fits(p, v)) return v;
   return pref;
 }
 
 static int plan_variant(const mdsm_plan_s *p) { return p->variant ? p->variant : default_variant(p); }
+
+// What a dedisperse call launches: the variant that was set or tuned, or the
+// form of the default variant that suits the survey's size.
+static int plan_shape(const mdsm_plan_s *p) {
+  if (p->variant) {
+    const int narrow = variant_fits(p, p->variant) ? 0 : narrow_variant(p->dtype, p->variant);
+    return narrow && variant_fits(p, narrow) ? narrow : p->variant;
+  }
+  const int v = default_variant(p);
+  if (!variant_fits(p, v)) return v;  // refused there
+  std::vector<bool> fits(p->row_words.size());
+  for (int i = 1; i < (int)fits.size(); ++i) fits[i] = variant_fits(p, i);
+  return untuned_shape(p->dtype, v, fits, p->s.ndms, p->s.nsamp);
+}
 
 extern "C" int mdsm_plan_create(const mdsm_survey_t *s, int in_dtype, mdsm_plan *plan) {
   MDSM_REQUIRE(plan, MDSM_ERR_ARG, "null plan");
@@ -316,7 +330,7 @@ extern "C" int mdsm_plan_create(const mdsm_survey_t *s, int in_dtype, mdsm_plan 
     delete p;
     return rc;
   }
-  const int nv = num_variants(in_dtype);
+  const int nv = num_shapes(in_dtype);
   p->row_words.assign(nv + 1, 0);
   p->d_rel.assign(nv + 1, nullptr);
   for (int v = 1; v <= nv; ++v) {
@@ -381,7 +395,7 @@ extern "C" int mdsm_plan_set_variant(mdsm_plan plan, int variant) {
   plan->variant = variant;
   // build the variant's trial-offset table now, so that dedisperse calls
   // (and graphs captured from them) allocate nothing
-  const int v = plan_variant(plan);
+  const int v = plan_shape(plan);
   if (variant_fits(plan, v)) {
     const int rc = ensure_trial_offsets(plan, v, nullptr);
     if (rc != MDSM_OK) return rc;
@@ -401,9 +415,9 @@ extern "C" int mdsm_plan_variant_channels(mdsm_plan plan, int variant, uint32_t 
   MDSM_REQUIRE(plan && channels, MDSM_ERR_ARG, "null argument");
   MDSM_REQUIRE(variant >= 1 && variant <= num_variants(plan->dtype), MDSM_ERR_ARG,
                "variant %d out of range", variant);
-  *channels = variant_fits(plan, variant)
-                  ? stage_channels(plan->dtype, variant, plan->row_words[variant])
-                  : 0u;
+  int v = variant;
+  if (!variant_fits(plan, v) && narrow_variant(plan->dtype, v)) v = narrow_variant(plan->dtype, v);
+  *channels = variant_fits(plan, v) ? stage_channels(plan->dtype, v, plan->row_words[v]) : 0u;
   return MDSM_OK;
 }
 
@@ -424,7 +438,7 @@ extern "C" int mdsm_dedisperse(mdsm_plan plan, const void *d_in, uint64_t ld, fl
                input_alignment(plan->dtype));
   MDSM_REQUIRE(ld / input_alignment(plan->dtype) < (1ull << 29), MDSM_ERR_ARG,
                "input rows must be shorter than 2 GiB");
-  const int v = plan_variant(plan);
+  const int v = plan_shape(plan);
   const int rc = ensure_trial_offsets(plan, v, as_stream(stream));
   if (rc != MDSM_OK) return rc;
   return launch_dedisperse(plan->dtype, v, d_in, ld, plan->d_table, plan->d_rel[v], plan->s.nchans,
@@ -444,8 +458,9 @@ int plan_time_variants(mdsm_plan plan, const void *d_in, uint64_t ld, float *d_o
   const int nv = num_variants(plan->dtype);
   const int keep = plan->variant;
   t.assign(nv + 1, -1.0f);
-  for (int v = 1; v <= nv; ++v) {
+  for (int v = 0; v <= nv; ++v) {
     plan->variant = v;
+    if (v == 0 && plan_shape(plan) == plan_variant(plan)) continue;  // timed by its number
     if (mdsm_dedisperse(plan, d_in, ld, d_out, s) != MDSM_OK) continue;  // warm-up / LDS fit
     float vms = -1.0f;
     for (int rep = 0; rep < 3; ++rep) {
@@ -488,9 +503,11 @@ extern "C" int mdsm_plan_autotune(mdsm_plan plan, const void *d_in, uint64_t ld,
   if (rc != MDSM_OK) return rc;
   const int best = pick_variant(plan->dtype, t);
   MDSM_REQUIRE(best > 0, MDSM_ERR_ARG, "no tile variant fits this survey");
-  plan->variant = best;
-  if (best_variant) *best_variant = best;
-  if (best_ms) *best_ms = t[best];
+  // t[0]: the untuned plan, where it launches no numbered shape
+  const bool untuned = t[0] >= 0.0f && t[0] <= t[best];
+  plan->variant = untuned ? 0 : best;
+  if (best_variant) *best_variant = plan_variant(plan);
+  if (best_ms) *best_ms = t[untuned ? 0 : best];
   return MDSM_OK;
 }
 

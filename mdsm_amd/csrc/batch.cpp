@@ -72,11 +72,31 @@ static int batch_variant(const mdsm_batch_s *b) {
   auto fits = [&](int v) { return batch_fits(b, v); };
   const int pref = preferred_variant(b->dtype);
   if (fits(pref)) return pref;
-  const int fb = fallback_variant(b->dtype);
-  if (fits(fb)) return fb;
+  for (int n = 0, fb; (fb = fallback_variant(b->dtype, n)) != 0; ++n)
+    if (fits(fb)) return fb;
   for (int v = 1; v <= num_variants(b->dtype); ++v)
     if (fits(v)) return v;
   return pref;
+}
+
+// The shape a launch uses: the variant that was set or tuned, or the eight-wave
+// form of the default by the rounds of all beams' tiles (as untuned_shape).
+static int batch_shape(const mdsm_batch_s *b) {
+  const int v = batch_variant(b);
+  const int narrow = narrow_variant(b->dtype, v);
+  if (!narrow || !batch_fits(b, narrow)) return v;
+  if (b->variant) return batch_fits(b, v) ? v : narrow;
+  auto cost = [&](int shape) {
+    const TileShape sh = variant_shape(b->dtype, shape);
+    double tiles = 0.0, work = 0.0;
+    for (const auto &s : b->beams) {
+      const double n = (double)((s.nsamp + sh.tt() - 1) / sh.tt()) * ((s.ndms + sh.td() - 1) / sh.td());
+      tiles += n;
+      work += n * s.nchans;
+    }
+    return tile_rounds(b->dtype, shape, tiles) * (work / tiles);
+  };
+  return cost(narrow) < cost(v) ? narrow : v;
 }
 
 static void free_batch(mdsm_batch_s *b) {
@@ -105,7 +125,7 @@ extern "C" int mdsm_batch_create(const mdsm_survey_t *beams, uint32_t nbeams, in
   b->h_tables.resize(nbeams);
   b->d_tables.assign(nbeams, nullptr);
   b->row_words.resize(nbeams);
-  const int nv = num_variants(in_dtype);
+  const int nv = num_shapes(in_dtype);
   b->d_rel.assign(nbeams, std::vector<int32_t *>(nv + 1, nullptr));
   for (uint32_t i = 0; i < nbeams; ++i) {
     int rc = build_delay_table(&beams[i], b->h_tables[i], &b->maxshift[i]);
@@ -262,7 +282,7 @@ extern "C" int mdsm_batch_bind(mdsm_batch batch, const void *const *d_in, const 
                                float *const *d_out) {
   MDSM_REQUIRE(batch && d_in && ld && d_out, MDSM_ERR_ARG, "null argument");
   const uint32_t nb = (uint32_t)batch->beams.size();
-  const int v = batch_variant(batch);
+  const int v = batch_shape(batch);
   const TileShape sh = variant_shape(batch->dtype, v);
   batch->h_desc.resize(nb);
   uint64_t items = 0;

@@ -2,7 +2,7 @@
 //
 // out[d][t] = sum_{c=0}^{C-1} in[c][t + D[c][d]]   (FP32 accumulation, channel order)
 //
-// Design (MI355X).  A workgroup of 4 wave64s owns a tile of TD = 4*MW DM
+// Design (MI355X), tiles that read a word per add.  A workgroup of 4 wave64s owns a tile of TD = 4*MW DM
 // trials x TT time samples; every wave owns MW consecutive trials and every
 // lane a few samples spaced 64 (FP32) or 128 (packed pairs) apart.  Channels
 // are processed in blocks: each block's input windows [t0 + D[c][d0],
@@ -13,9 +13,9 @@
 // tabulated once per plan, a block's offsets sit 16 per VGPR, and one trial
 // costs one DPP-broadcast address add for K LDS reads (issued in pairs as
 // ds_read2st64).  These adds are bound by LDS reads, not by HBM, so the
-// storage formats trade LDS bytes per add; the register-window tiles (the
-// defaults of F32 and F16) read a word once per wave instead of once per
-// trial and are bound by instruction issue:
+// storage formats trade LDS bytes per add.  The register-window tiles (the
+// defaults of every storage type) read a word once per wave instead of once
+// per trial and are bound by instruction issue.  The word-per-add formats:
 //   F32  4 B per add: one float per LDS word, staged by direct buffer->LDS
 //        loads (buffer_load_dword ... lds) that use no data VGPRs.
 //   F16  2 B per add: LDS words hold pairs of consecutive samples in two
@@ -49,6 +49,7 @@
 #include <hip/hip_fp16.h>
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "internal.h"
@@ -297,17 +298,17 @@ struct F32Tile {
 // 16-byte reads they make.
 //
 // Bound: instruction issue.  1024 channels x 4096 trials x 2^17 samples, F32:
-// 34.6 T adds/s (18.5 with one LDS read per add), the VALU at 50 % of the 64 T
-// it issues, LDS reads under a third of their rate; one wave issues at most
+// 40.5 T adds/s (18.5 with one LDS read per add), the VALU at two thirds of the
+// 64 T it issues, LDS reads under half of their rate; one wave issues at most
 // one instruction per about 5 clocks, so 4 waves per SIMD (128 VGPRs) set
 // MW * K + WIN, and K = 20 at MW = 4 the fewest jumps (49 T without staging
 // and tables; MW = 8, K = 12 at 3 waves 41 T).
 //
 // F16 and U8 rows are widened to FP32 in LDS by one pass per channel block
-// (exact; 32 trials share it), so all storage types run the same adds: F16
+// (exact; all trials of the tile share it), so all storage types run the same adds: F16
 // in FP32 channel order, U8 as exact integers (at most 65536 * 255 < 2^24).
 struct WindowCode {
-  static constexpr int MW = 4, K = 20, WAVES = 8;
+  static constexpr int MW = 4, K = 20;
   static constexpr int WIN = 36;                  // window words, VGPRs 92..127
   static constexpr int NV = WIN - K + 1;          // word offsets of a trial
   static constexpr int BLOCK = 96;                // code bytes per block, per stub
@@ -410,21 +411,62 @@ struct WindowCode {
 #undef MDSM_WIN_JUMP
 #undef MDSM_WIN_ADDS
 #undef MDSM_WIN_ADD
+
+  // The wave's sums to out: a lane's 20 consecutive samples become 64-sample
+  // rows through the wave's own 640 words of LDS, half of the lanes at a time.
+  template <bool IS_U8>
+  __device__ __forceinline__ static void store(const float (&acc)[MW][K], float *lds, uint32_t wave,
+                                               uint32_t lane, float *__restrict__ out, uint32_t nsamp,
+                                               uint32_t ndms, uint32_t dw, uint32_t t0, uint32_t nchans) {
+    float *mine = lds + wave * 640u;
+    const double base = (double)nchans * -4.0;
+#pragma unroll
+    for (int i = 0; i < MW; ++i) {
+      const uint32_t d = dw + (uint32_t)i;
+      if (d >= ndms) break;
+      float *orow = out + (uint64_t)d * nsamp;
+#pragma unroll
+      for (uint32_t h = 0; h < 2u; ++h) {
+        if ((lane >> 5) == h) {
+#pragma unroll
+          for (int j = 0; j < K; j += 4)
+            *reinterpret_cast<float4 *>(mine + K * (lane & 31u) + j) =
+                make_float4(acc[i][j], acc[i][j + 1], acc[i][j + 2], acc[i][j + 3]);
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (uint32_t j = 0; j < 10u; ++j) {
+          const uint32_t t = t0 + 640u * h + lane + 64u * j;
+          float v = mine[lane + 64u * j];
+          if constexpr (IS_U8) v = (float)((double)(uint32_t)v * (8.0 / 255.0) + base);
+          if (t < nsamp) orow[t] = v;
+        }
+        __builtin_amdgcn_wave_barrier();
+      }
+    }
+  }
 };
 
-template <int MODE>
+//
+// A workgroup is NW waves: 16 (64 trials, all 160 KB of a CU's LDS) stage and
+// widen a row for twice the trials and meet at half the barriers per add of 8
+// (32 trials, 80 KB): F32 40.5 against 34.6 T adds/s, F16 37.7 against 36.5,
+// U8 38.3 against 37.5.  8 pads surveys of few trials less.
+template <int MODE, int NW>
 struct WindowTile {
   using W = WindowCode;
   static constexpr bool PAIRS = false;
   static constexpr bool IS_F32 = MODE == MDSM_F32, IS_U8 = MODE == MDSM_U8;
-  static constexpr int MW = W::MW, K = W::K, THREADS = 64 * W::WAVES;
-  static constexpr int TT = 64 * K, TD = W::WAVES * MW, CB = IS_F32 ? 6 : 8;
-  // staging (and widening): WPR waves share a row of a block, every wave has RPW rows
-  static constexpr uint32_t WPR = IS_F32 ? 4 : 1, RSTEP = W::WAVES / WPR, RPW = CB / RSTEP;
+  static constexpr int MW = W::MW, K = W::K, WAVES = NW, THREADS = 64 * NW;
+  static constexpr int TT = 64 * K, TD = NW * MW;
+  static constexpr int CB = NW == 8 ? (IS_F32 ? 6 : 8) : (IS_F32 ? 12 : 16);
+  // staging (and widening): WPR waves share a row of a block, every wave has
+  // up to RPW rows
+  static constexpr uint32_t WPR = NW == 8 && IS_F32 ? 4 : 1, RSTEP = NW / WPR, RPW = (CB + RSTEP - 1) / RSTEP;
   using T = std::conditional_t<IS_F32, float, std::conditional_t<IS_U8, uint8_t, __half>>;
   static constexpr uint32_t PER = 4u / sizeof(T);  // samples per source dword
   static uint64_t table_words(uint32_t nchans, uint32_t ndms) {
-    return (uint64_t)((ndms + TD - 1u) / TD) * W::WAVES * (nchans + 1u) * 8u;
+    return (uint64_t)((ndms + TD - 1u) / TD) * NW * (nchans + 1u) * 8u;
   }
   static bool fits(uint32_t) { return true; }
   // FP32 row words: the window of TT + spread samples from an origin that is
@@ -527,7 +569,7 @@ struct WindowTile {
     const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_float *)lds + (uint32_t)(4 * K) * lane;
     // the wave's table entries, one per channel (scalar loads)
     const const_u32x8 *rt =
-        (const const_u32x8 *)(uintptr_t)reltab + ((uint64_t)dt * W::WAVES + wave) * (nchans + 1u);
+        (const const_u32x8 *)(uintptr_t)reltab + ((uint64_t)dt * NW + wave) * (nchans + 1u);
     prefetch(0);
     stage(0, IS_F32 ? lds : second);
     if (cbr < nchans) prefetch(cbr);
@@ -560,41 +602,14 @@ struct WindowTile {
       }
     }
 
-    // the lane's 20 consecutive samples become 64-sample rows through the
-    // wave's own 640 words of LDS, half of the lanes at a time
-    float *mine = lds + wave * 640u;
-    const double base = (double)nchans * -4.0;
-#pragma unroll
-    for (int i = 0; i < MW; ++i) {
-      const uint32_t d = dw + (uint32_t)i;
-      if (d >= ndms) break;
-      float *orow = out + (uint64_t)d * nsamp;
-#pragma unroll
-      for (uint32_t h = 0; h < 2u; ++h) {
-        if ((lane >> 5) == h) {
-#pragma unroll
-          for (int j = 0; j < K; j += 4)
-            *reinterpret_cast<float4 *>(mine + K * (lane & 31u) + j) =
-                make_float4(acc[i][j], acc[i][j + 1], acc[i][j + 2], acc[i][j + 3]);
-        }
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (uint32_t j = 0; j < 10u; ++j) {
-          const uint32_t t = t0 + 640u * h + lane + 64u * j;
-          float v = mine[lane + 64u * j];
-          if constexpr (IS_U8) v = (float)((double)(uint32_t)v * (8.0 / 255.0) + base);
-          if (t < nsamp) orow[t] = v;
-        }
-        __builtin_amdgcn_wave_barrier();
-      }
-    }
+    W::store<IS_U8>(acc, lds, wave, lane, out, nsamp, ndms, dw, t0, nchans);
   }
 };
 
 template <typename T>
 struct IsWindow : std::false_type {};
-template <int MODE>
-struct IsWindow<WindowTile<MODE>> : std::true_type {};
+template <int MODE, int NW>
+struct IsWindow<WindowTile<MODE, NW>> : std::true_type {};
 // Threads per workgroup: four waves, or the window tiles' eight.
 template <typename T>
 constexpr int tile_threads() {
@@ -602,7 +617,7 @@ constexpr int tile_threads() {
   else return 256;
 }
 
-// Table of a window tile: entry ((dt * 8 + wave) * (nchans + 1) + c) for
+// Table of a window tile: entry ((dt * WAVES + wave) * (nchans + 1) + c) for
 // channel c and trials 4 wave .. 4 wave + 3 of DM tile dt, at their samples'
 // byte offsets in the block's FP32 rows (row c % cbr starts at a multiple of
 // PER samples at or below the tile's first delay); entry nchans, which is
@@ -617,7 +632,7 @@ __global__ __launch_bounds__(256) void window_table_kernel(const int32_t *__rest
   if (e >= entries) return;
   const uint32_t c = min((uint32_t)(e % (nchans + 1u)), nchans - 1u);
   const uint64_t g = e / (nchans + 1u);
-  const uint32_t wave = (uint32_t)(g % WindowCode::WAVES), dt = (uint32_t)(g / WindowCode::WAVES);
+  const uint32_t wave = (uint32_t)(g % Tile::WAVES), dt = (uint32_t)(g / Tile::WAVES);
   const uint32_t d0 = dt * Tile::TD;
   const int32_t *row = table + (uint64_t)c * ndms;
   const uint32_t base = (uint32_t)row[d0], skew = base & (Tile::PER - 1u);
@@ -970,8 +985,8 @@ template <int MW, int K2, int CB, int BURST>
 struct PairsOf<PackedTile<MDSM_F16, MW, K2, CB, BURST>> {
   using type = PackedTile<MDSM_F16_PAIRS, MW, K2, CB, BURST / 2>;
 };
-template <>
-struct PairsOf<WindowTile<MDSM_F16>> {
+template <int NW>
+struct PairsOf<WindowTile<MDSM_F16, NW>> {
   using type = PackedTile<MDSM_F16_PAIRS, 12, 4, 4>;
 };
 
@@ -1355,6 +1370,254 @@ struct IsPairSum : std::false_type {};
 template <int MODE, int MW, int K2, int CBP, int NS, int BURST>
 struct IsPairSum<PairSumTile<MODE, MW, K2, CBP, NS, BURST>> : std::true_type {};
 
+// Register windows over pair-sum rows: the sum rows S_j of each channel pair,
+// built in LDS as FP32 (F16_PAIRS: the FP16-rounded pair sums widened, U8: the
+// exact sums), are read by WindowCode's adds, so one v_add_f32 adds two
+// channels.  Trials of one wave that differ in j or run out of a window read
+// another one (1.9 windows and 12 reads per wave and pair at 1024 channels
+// and a DM step of 0.2, against one and 7 for single channels).  Results are
+// those of the other pair-sum shapes.  1024 channels x 4096 trials x 2^17
+// samples: U8 12.1 ms (45.6 T adds/s; 14.9 with shape 20), F16_PAIRS 12.4
+// (44.5; 14.1).  With eight waves the twelve barriers per LDS fill are shared
+// by half the trials: 33 T.
+template <int MODE, int NW>
+struct WindowPairTile {
+  using W = WindowCode;
+  static constexpr bool PAIRS = true;
+  static constexpr bool IS_U8 = MODE == MDSM_U8;
+  static constexpr int MW = W::MW, K = W::K, WAVES = NW, THREADS = 64 * NW;
+  static constexpr int TT = 64 * K, TD = NW * MW, CB = NW == 8 ? 6 : 12, CBP = CB / 2, NSUM = 3;
+  using T = std::conditional_t<IS_U8, uint8_t, __half>;
+  static constexpr uint32_t PER = 4u / sizeof(T);  // samples per source dword, origin of a window
+  // staging: WPR waves share a row of a block, every wave has up to RPW rows;
+  // building: 512 threads take a pair (four samples each), every 512 of the
+  // workgroup every NG-th pair
+  static constexpr uint32_t WPR = NW == 8 ? 4 : 1, RSTEP = NW / WPR, RPW = (CB + RSTEP - 1) / RSTEP;
+  static constexpr uint32_t NG = THREADS / 512, PPG = CBP / NG;
+  static bool fits(uint32_t) { return true; }
+  static uint32_t row_words(uint32_t spread) { return ((uint32_t)TT + spread + 16u + 63u) & ~63u; }
+  // raw dwords per channel: the samples of a sum row and 8 more (shifts)
+  static __host__ __device__ uint32_t raw_words(uint32_t rw) { return (rw / PER + 4u + 63u) & ~63u; }
+  static uint32_t lds_words_per_row(uint32_t rw) { return raw_words(rw) + (uint32_t)NSUM * rw / 2u; }
+  static uint64_t table_entries(uint32_t nchans, uint32_t ndms) {
+    return (uint64_t)((ndms + TD - 1u) / TD) * NW * ((nchans + 1u) / 2u + 1u);
+  }
+  // 8 words per entry, then {dmin, n} per DM tile and pair
+  static uint64_t table_words(uint32_t nchans, uint32_t ndms) {
+    return 8u * table_entries(nchans, ndms) +
+           2u * (uint64_t)((ndms + TD - 1u) / TD) * ((nchans + 1u) / 2u);
+  }
+
+  __device__ __forceinline__ static void run(const T *__restrict__ in, uint64_t ld,
+                                             const int32_t *__restrict__ table,
+                                             const int32_t *__restrict__ reltab, uint32_t nchans,
+                                             uint32_t nsamp, uint32_t ndms, uint32_t rw,
+                                             uint32_t cbr, float *__restrict__ out, uint32_t tt,
+                                             uint32_t dt, float *lds) {
+    typedef W::u32x8 u32x8;
+    typedef W::const_u32x8 const_u32x8;
+    typedef __attribute__((address_space(3))) float lds_float;
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = uniform(threadIdx.x >> 6);
+    const uint32_t t0 = tt * TT, d0 = dt * TD;
+    const uint32_t dw = d0 + wave * MW;
+    const uint32_t rawn = raw_words(rw);
+    const uint32_t npairs = (nchans + 1u) / 2u, n_dtiles = (ndms + TD - 1u) / TD;
+    typedef __attribute__((address_space(4))) const int32_t const_i32;  // scalar loads
+    const const_i32 *dtab = (const const_i32 *)(uintptr_t)reltab +
+                            8u * ((uint64_t)n_dtiles * NW * (npairs + 1u)) + 2u * (uint64_t)dt * npairs;
+    const const_i32 *ctable = (const const_i32 *)(uintptr_t)table;
+    // LDS: cbr / 2 pairs of NSUM sum rows, then cbr raw windows
+    uint32_t *const raw = reinterpret_cast<uint32_t *>(lds) + (cbr / 2u) * (uint32_t)NSUM * rw;
+    const uint32_t srow = wave / WPR, part = wave % WPR;
+    // window starts of the rows the next stage() takes
+    uint32_t gpre[RPW];
+    auto prefetch = [&](uint32_t cb) {
+#pragma unroll
+      for (uint32_t i = 0; i < RPW; ++i) {
+        const uint32_t c = min(cb + srow + RSTEP * i, nchans - 1u), c0 = c & ~1u;
+        const uint32_t g = t0 + (uint32_t)ctable[(uint64_t)c0 * ndms + d0];
+        gpre[i] = (c & 1u) ? (g & ~(PER - 1u)) + (uint32_t)dtab[c0] : g;
+      }
+    };
+    auto stage = [&](uint32_t cb) {
+#pragma unroll
+      for (uint32_t i = 0; i < RPW; ++i) {
+        const uint32_t r = srow + RSTEP * i;
+        if (r >= min(cbr, nchans - cb)) break;
+        const uint32_t w0 = gpre[i] / PER, ldw = (uint32_t)(ld / PER);  // rows < 2 GiB
+        const uint32_t *src = reinterpret_cast<const uint32_t *>(in) + (uint64_t)(cb + r) * ldw + w0;
+        const uint32_t avail = 4u * (ldw - min(w0, ldw));  // dwords past the row read as 0
+        const uint64_t a = reinterpret_cast<uint64_t>(src);
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+            reinterpret_cast<void *>(((uint64_t)uniform((uint32_t)(a >> 32)) << 32) | uniform((uint32_t)a)),
+            (short)0, (int)uniform(avail), 0x00020000);
+        uint32_t *dst = raw + r * rawn + 64u * part;
+        uint32_t vo = 4u * (threadIdx.x & 63u) + 256u * part;
+        asm volatile("" : "+v"(vo));
+        for (uint32_t q = part; 64u * q < rawn; q += WPR, vo += 256u * WPR, dst += 64u * WPR)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void *)dst, 4, (int)vo, 0, 0, 0);
+      }
+    };
+    // the block's pairs: dmin's part below the window origin's grid, and the
+    // number of sum rows (0: no such pair)
+    const uint32_t grp = wave / 8u;
+    uint32_t frac[PPG], nrow[PPG];
+    auto pairs_of = [&](uint32_t cb) {
+      const uint32_t np = (min(cbr, nchans - cb) + 1u) / 2u;
+#pragma unroll
+      for (uint32_t i = 0; i < PPG; ++i) {
+        const uint32_t p = grp + NG * i, q = min(cb / 2u + p, npairs - 1u);
+        frac[i] = (uint32_t)dtab[2u * q] & (PER - 1u);
+        nrow[i] = p < np ? (uint32_t)dtab[2u * q + 1u] : 0u;
+      }
+    };
+    // S_j[n .. n+3] = x0[n ..] + x1[n + SH ..], SH = j + frac; a pair without
+    // its second channel adds 0.  The reads of all pairs are issued together.
+    // (n0 is opaque, so that no address is kept in registers over the adds)
+    auto build = [&](uint32_t cb) {
+      const bool odd = cb + cbr >= nchans && (nchans & 1u);  // the block's last pair is one channel
+      const uint32_t last = (min(cbr, nchans - cb) - 1u) / 2u;
+      uint32_t n0 = 4u * (threadIdx.x & 511u);
+      asm volatile("" : "+v"(n0));
+      for (uint32_t n = n0; n < rw; n += 2048u) {
+        uint32_t x[PPG][2], z[PPG][4];
+#pragma unroll
+        for (uint32_t i = 0; i < PPG; ++i) {
+          const uint32_t *R0 = raw + 2u * min(grp + NG * i, last) * rawn, *R1 = R0 + rawn;
+          if constexpr (IS_U8) {
+            x[i][0] = R0[n / 4u];
+            z[i][0] = R1[n / 4u], z[i][1] = R1[n / 4u + 1u], z[i][2] = R1[n / 4u + 2u];
+          } else {
+            const uint2 a = *reinterpret_cast<const uint2 *>(R0 + n / 2u);
+            const uint2 c = *reinterpret_cast<const uint2 *>(R1 + n / 2u);
+            const uint2 e = *reinterpret_cast<const uint2 *>(R1 + n / 2u + 2u);
+            x[i][0] = a.x, x[i][1] = a.y;
+            z[i][0] = c.x, z[i][1] = c.y, z[i][2] = e.x, z[i][3] = e.y;
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (uint32_t i = 0; i < PPG; ++i) {
+          float *S = lds + (grp + NG * i) * NSUM * rw;
+          if (odd && grp + NG * i == last) z[i][0] = z[i][1] = z[i][2] = z[i][3] = 0u;
+          uint32_t y[3];  // U8: bytes n + frac .., F16: halves n + frac ..
+          if constexpr (IS_U8) {
+            y[0] = __builtin_amdgcn_alignbyte(z[i][1], z[i][0], frac[i]);
+            y[1] = __builtin_amdgcn_alignbyte(z[i][2], z[i][1], frac[i]);
+          } else {
+            y[0] = __builtin_amdgcn_alignbit(z[i][1], z[i][0], 16u * frac[i]);
+            y[1] = __builtin_amdgcn_alignbit(z[i][2], z[i][1], 16u * frac[i]);
+            y[2] = __builtin_amdgcn_alignbit(z[i][3], z[i][2], 16u * frac[i]);
+          }
+#pragma unroll
+          for (int j = 0; j < NSUM; ++j) {
+            if ((uint32_t)j >= nrow[i]) break;
+            float4 v;
+            if constexpr (IS_U8) {
+              const uint32_t a = x[i][0], c = __builtin_amdgcn_alignbyte(y[1], y[0], (uint32_t)j);
+              v = make_float4((float)((a & 0xFFu) + (c & 0xFFu)), (float)(((a >> 8) & 0xFFu) + ((c >> 8) & 0xFFu)),
+                              (float)(((a >> 16) & 0xFFu) + ((c >> 16) & 0xFFu)), (float)((a >> 24) + (c >> 24)));
+            } else {
+              const uint32_t a = j == 1 ? __builtin_amdgcn_alignbit(y[1], y[0], 16) : y[j / 2];
+              const uint32_t c = j == 1 ? __builtin_amdgcn_alignbit(y[2], y[1], 16) : y[j / 2 + 1];
+              const half2_t s0 = __builtin_bit_cast(half2_t, x[i][0]) + __builtin_bit_cast(half2_t, a);
+              const half2_t s1 = __builtin_bit_cast(half2_t, x[i][1]) + __builtin_bit_cast(half2_t, c);
+              v = make_float4((float)s0.x, (float)s0.y, (float)s1.x, (float)s1.y);
+            }
+            *reinterpret_cast<float4 *>(S + j * rw + n) = v;
+          }
+        }
+      }
+    };
+
+    float acc[MW][K];
+#pragma unroll
+    for (int i = 0; i < MW; ++i)
+#pragma unroll
+      for (int j = 0; j < K; ++j) acc[i][j] = 0.0f;
+
+    const uint32_t cur = (uint32_t)(uintptr_t)(lds_float *)lds + (uint32_t)(4 * K) * lane;
+    const const_u32x8 *rt =
+        (const const_u32x8 *)(uintptr_t)reltab + ((uint64_t)dt * NW + wave) * (npairs + 1u);
+    prefetch(0);
+    stage(0);
+    pairs_of(0);
+    if (cbr < nchans) prefetch(cbr);
+    u32x8 o = *rt;
+    wait_vmem();
+    __syncthreads();
+    build(0);
+    __syncthreads();
+    for (uint32_t cb = 0; cb < nchans; cb += cbr) {
+      const bool more = cb + cbr < nchans;
+      if (more) {
+        stage(cb + cbr);
+        pairs_of(cb + cbr);
+        if (cb + 2u * cbr < nchans) prefetch(cb + 2u * cbr);
+      }
+      const uint32_t np = (min(cbr, nchans - cb) + 1u) / 2u;
+      for (uint32_t p = 0; p < np; ++p) {
+        ++rt;
+        o = W::add_channel(acc, cur, o, rt);
+      }
+      wait_vmem();
+      __syncthreads();
+      if (more) build(cb + cbr);
+      __syncthreads();
+    }
+    W::store<IS_U8>(acc, lds, wave, lane, out, nsamp, ndms, dw, t0, nchans);
+  }
+};
+
+template <typename T>
+struct IsWindowPair : std::false_type {};
+template <int MODE, int NW>
+struct IsWindowPair<WindowPairTile<MODE, NW>> : std::true_type {};
+template <int MODE, int NW>
+struct IsWindow<WindowPairTile<MODE, NW>> : std::true_type {};
+
+// Table of a window pair-sum tile (layout at table_words): entry ((dt * WAVES +
+// wave) * (npairs + 1) + p), and {dmin, n} of pair p in DM tile dt.  A pair
+// without its second channel sums with zero: dmin 0, n 1.
+template <typename Tile>
+__global__ __launch_bounds__(256) void window_pair_table_kernel(const int32_t *__restrict__ table,
+                                                                uint32_t nchans, uint32_t ndms,
+                                                                uint32_t rw, uint32_t cbr,
+                                                                uint64_t entries,
+                                                                int32_t *__restrict__ reltab) {
+  const uint64_t e = (uint64_t)blockIdx.x * 256u + threadIdx.x;
+  if (e >= entries) return;
+  const uint32_t npairs = (nchans + 1u) / 2u;
+  const uint32_t p = min((uint32_t)(e % (npairs + 1u)), npairs - 1u);
+  const uint64_t g = e / (npairs + 1u);
+  const uint32_t wave = (uint32_t)(g % Tile::WAVES), dt = (uint32_t)(g / Tile::WAVES);
+  const uint32_t d0 = dt * Tile::TD, dl = min(d0 + (uint32_t)Tile::TD, ndms) - 1u;
+  const uint32_t c0 = 2u * p;
+  const bool solo = c0 + 1u >= nchans;
+  const int32_t *r0 = table + (uint64_t)c0 * ndms, *r1 = solo ? r0 : r0 + ndms;
+  int32_t dmin = r1[d0] - r0[d0], dmax = dmin;
+  for (uint32_t d = d0 + 1u; d <= dl; ++d) {
+    const int32_t v = r1[d] - r0[d];
+    dmin = min(dmin, v);
+    dmax = max(dmax, v);
+  }
+  const uint32_t base = (uint32_t)r0[d0], skew = base & (Tile::PER - 1u);
+  uint32_t o[WindowCode::MW], w[2 * WindowCode::MW];
+  for (uint32_t i = 0; i < (uint32_t)WindowCode::MW; ++i) {
+    const uint32_t d = min(d0 + wave * WindowCode::MW + i, ndms - 1u);
+    const uint32_t j = min((uint32_t)(r1[d] - r0[d] - dmin), (uint32_t)Tile::NSUM - 1u);
+    o[i] = 4u * ((p % (cbr / 2u) * Tile::NSUM + j) * rw + skew + ((uint32_t)r0[d] - base));
+  }
+  WindowCode::entry(o, w);
+  for (int i = 0; i < 2 * WindowCode::MW; ++i) reltab[e * 8u + i] = (int32_t)w[i];
+  if (wave == 0) {
+    int32_t *t = reltab + entries * 8u + 2u * ((uint64_t)dt * npairs + p);
+    t[0] = dmin;
+    t[1] = dmax - dmin + 1;
+  }
+}
+
 // Trial offsets and {dmin, n} of a pair-sum tile (layout above): entry e <
 // nrel is ((dt * nblocks + k) * 4 + w) * WORDS + idx with (p, i) =
 // divmod(idx, MW); the byte offset of trial dw + i of pair p inside the sum
@@ -1448,12 +1711,20 @@ template <typename Tile>
 struct FlatWaves {
   static constexpr int value = 1;
 };
-template <int MODE>
-struct FlatWaves<WindowTile<MODE>> {
+template <int MODE, int NW>
+struct FlatWaves<WindowTile<MODE, NW>> {
   static constexpr int value = 4;
 };
-template <int MODE>
-struct PersistWaves<WindowTile<MODE>> {
+template <int MODE, int NW>
+struct PersistWaves<WindowTile<MODE, NW>> {
+  static constexpr int value = 4;
+};
+template <int MODE, int NW>
+struct FlatWaves<WindowPairTile<MODE, NW>> {
+  static constexpr int value = 4;
+};
+template <int MODE, int NW>
+struct PersistWaves<WindowPairTile<MODE, NW>> {
   static constexpr int value = 4;
 };
 template <int MODE, int MW, int K2, int CBP, int NS, int BURST>
@@ -1616,7 +1887,7 @@ void batch_flat_kernel(const BeamDesc *__restrict__ beams,
 template <int V>
 struct VariantDef;
 template <> struct VariantDef<1> { using F32 = F32Tile<8, 4, 8>;   using F16 = F16Tile<8, 2, 8>;   using U8 = U8Tile<8, 2, 8>; };
-template <> struct VariantDef<2> { using F32 = F32Tile<16, 4, 4>;  using F16 = F16Tile<16, 2, 4>;  using U8 = WindowTile<MDSM_U8>; };
+template <> struct VariantDef<2> { using F32 = F32Tile<16, 4, 4>;  using F16 = F16Tile<16, 2, 4>;  using U8 = WindowTile<MDSM_U8, 16>; };
 template <> struct VariantDef<3> { using F32 = F32Tile<8, 8, 8>;   using F16 = F16Tile<8, 4, 8>;   using U8 = U8Tile<8, 4, 8>; };
 template <> struct VariantDef<4> { using F32 = F32Tile<16, 8, 4>;  using F16 = F16Tile<16, 4, 4>;  using U8 = U8Tile<16, 4, 4>; };
 template <> struct VariantDef<5> { using F32 = F32Tile<32, 2, 2>;  using F16 = F16Tile<32, 1, 2>;  using U8 = U8Tile<32, 1, 2>; };
@@ -1629,9 +1900,9 @@ template <> struct VariantDef<8> { using F32 = F32Tile<16, 4, 4, 4>; using F16 =
 template <> struct VariantDef<9> { using F32 = F32Tile<8, 8, 4>;    using F16 = F16Tile<8, 4, 4>;   using U8 = U8Tile<8, 4, 4>; };
 template <> struct VariantDef<10> { using F32 = F32Tile<4, 16, 8>;  using F16 = F16Tile<4, 8, 8>;   using U8 = U8Tile<4, 8, 8>; };
 template <> struct VariantDef<11> { using F32 = F32Tile<4, 16, 4>;  using F16 = F16Tile<4, 8, 4>;   using U8 = U8Tile<4, 8, 4>; };
-// register windows (F32 and F16 here, U8 in 2), and 12 or 16 trials per wave
+// register windows (F32 and F16 here, U8 in 2); 12 or 16 trials per wave
 // with more samples per lane: one address add per 8 or 6 packed adds
-template <> struct VariantDef<12> { using F32 = WindowTile<MDSM_F32>; using F16 = WindowTile<MDSM_F16>; using U8 = U8Tile<12, 4, 4>; };
+template <> struct VariantDef<12> { using F32 = WindowTile<MDSM_F32, 16>; using F16 = WindowTile<MDSM_F16, 16>; using U8 = U8Tile<12, 4, 4>; };
 template <> struct VariantDef<13> { using F32 = F32Tile<16, 6, 4>;  using F16 = F16Tile<16, 3, 4>;  using U8 = U8Tile<16, 3, 4>; };
 // 16 trials per wave over 8-channel blocks: half the barriers per add
 template <> struct VariantDef<14> { using F32 = F32Tile<16, 4, 8>;  using F16 = F16Tile<16, 2, 8>;  using U8 = U8Tile<16, 2, 8>; };
@@ -1646,12 +1917,16 @@ template <> struct PairSumDef<16> { template <int M> using type = PairSumTile<M,
 template <> struct PairSumDef<17> { template <int M> using type = PairSumTile<M, 12, 4, 2, 3>; };
 template <> struct PairSumDef<18> { template <int M> using type = PairSumTile<M, 12, 2, 2, 3>; };
 template <> struct PairSumDef<19> { template <int M> using type = PairSumTile<M, 16, 3, 2, 4>; };
-// 17 with the reads of 2 or 3 trials issued ahead of their adds
+// 17, and 10 trials per wave, with the reads of 2 trials issued ahead of their adds
 template <> struct PairSumDef<20> { template <int M> using type = PairSumTile<M, 12, 4, 2, 3, 2>; };
-template <> struct PairSumDef<21> { template <int M> using type = PairSumTile<M, 12, 4, 2, 3, 3>; };
-// 10 trials x 4 pairs with grouped reads: 4 waves per SIMD for U8 (126 VGPRs)
-template <> struct PairSumDef<22> { template <int M> using type = PairSumTile<M, 10, 4, 2, 3, 2>; };
+template <> struct PairSumDef<21> { template <int M> using type = PairSumTile<M, 10, 4, 2, 3, 2>; };
+// register windows over FP32 sum rows
+template <> struct PairSumDef<22> { template <int M> using type = WindowPairTile<M, 16>; };
 constexpr int kNumPairSumVariants = 7;
+// Eight-wave forms of the register-window shapes (narrow_variant), numbered
+// after the public ones: 16 for F32 and F16; 23 (pair sums) and 24 for U8, 23
+// for F16_PAIRS.
+constexpr int narrow_shapes(int dtype) { return dtype == MDSM_U8 ? 2 : 1; }
 
 template <typename V, typename Fn>
 int pick_dtype(int dtype, Fn &&fn) {
@@ -1706,15 +1981,24 @@ int with_tile(int dtype, int variant, Fn &&fn) {
       case 22: return fn((PairSumDef<22>::type<MDSM_U8> *)nullptr);
     }
   }
+  if (variant == num_variants(dtype) + 1) {
+    if (dtype == MDSM_F32) return fn((WindowTile<MDSM_F32, 8> *)nullptr);
+    if (dtype == MDSM_F16) return fn((WindowTile<MDSM_F16, 8> *)nullptr);
+    if (dtype == MDSM_U8) return fn((WindowPairTile<MDSM_U8, 8> *)nullptr);
+    if (dtype == MDSM_F16_PAIRS) return fn((WindowPairTile<MDSM_F16_PAIRS, 8> *)nullptr);
+  }
+  if (variant == num_variants(dtype) + 2 && dtype == MDSM_U8) return fn((WindowTile<MDSM_U8, 8> *)nullptr);
   set_error("unknown dedispersion variant %d", variant);
   return MDSM_ERR_ARG;
 }
 
-// LDS of a workgroup: 64 KB, or 80 KB for the window tiles (their registers
-// leave two workgroups of eight waves per CU, which has 160 KB).
+// LDS of a workgroup: 64 KB; window tiles, whose registers leave 16 waves per
+// CU, take its 160 KB in one workgroup of 16 waves or two of eight.
 template <typename Tile>
 constexpr uint64_t tile_lds() {
-  return IsWindow<Tile>::value ? 80 * 1024 : 64 * 1024;
+  // (256 bytes spare for static LDS)
+  if constexpr (IsWindow<Tile>::value) return (Tile::WAVES == 8 ? 80 : 160) * 1024 - 256;
+  else return 64 * 1024;
 }
 
 // Channels staged per block: the tile's CB, reduced while the block's LDS
@@ -1739,28 +2023,89 @@ int num_variants(int dtype) {
 
 // Untuned defaults.  F32 and F16 take the register-window tile, which was
 // the fastest shape of every survey tried: 1024 channels x 4096 trials x 2^17
-// samples 15.9 ms against 29.7 (F32, shape 8) and 15.1 against 21.9 (F16,
-// shape 15); delay slopes from 0.1 to 24 samples per trial 1.5 to 2.5 times
-// (418 MHz, step 0.5: 5.7 against 14.2 ms); 64 channels 1.6 times; 64 trials x
-// 8192 samples, too few tiles for the chip, level.  F16_PAIRS and U8 prefer
-// the pair-sum shapes (20, 22), which take only surveys with few delay
-// differences per channel pair and DM tile, and fall back to a shape that
-// takes every survey whose delay spread it can stage.
+// samples 13.5 ms against 29.7 (F32, shape 8) and 14.6 against 21.9 (F16,
+// shape 15); delay slopes from 0.1 to 24 samples per trial 1.5 to 2.5 times;
+// 64 channels 1.6 times.  F16_PAIRS and U8 prefer the register windows over
+// pair sums (12.4 ms against 14.1, 12.1 against 14.9 of the other pair-sum
+// shapes), which take only surveys with few delay differences per channel pair
+// and DM tile, and fall back to shapes that take more of them, the last one
+// every survey whose delay spread it can stage.
 int preferred_variant(int dtype) {
   switch (dtype) {
     case MDSM_F32: return 12;
     case MDSM_F16: return 12;
-    case MDSM_F16_PAIRS: return 20;
     default: return 22;
   }
 }
 
-int fallback_variant(int dtype) {
+// Surveys whose delay differences suit DM tiles of fewer trials than 64 take
+// the pair-sum shapes of 40 (U8: 36 against 33 T adds/s of shape 2) or 48, 40
+// and 32 trials (F16_PAIRS: 36, 33 and 31 against 25 of shape 15; 256 channels
+// x 1920 trials x 81920 samples).
+int fallback_variant(int dtype, int n) {
   switch (dtype) {
-    case MDSM_F32: return 8;
-    case MDSM_U8: return 2;
-    default: return 15;
+    case MDSM_F32: return n == 0 ? 8 : 0;
+    case MDSM_F16: return n == 0 ? 15 : 0;
+    case MDSM_U8: return n == 0 ? 21 : (n == 1 ? 2 : 0);
+    default: return n == 0 ? 20 : (n == 1 ? 21 : (n == 2 ? 16 : (n == 3 ? 15 : 0)));
   }
+}
+
+int num_shapes(int dtype) { return num_variants(dtype) + narrow_shapes(dtype); }
+
+int narrow_variant(int dtype, int variant) {
+  const int nv = num_variants(dtype);
+  switch (dtype) {
+    case MDSM_F32:
+    case MDSM_F16: return variant == 12 ? nv + 1 : 0;
+    case MDSM_U8: return variant == 22 ? nv + 1 : (variant == 2 ? nv + 2 : 0);
+    default: return variant == 22 ? nv + 1 : 0;
+  }
+}
+
+// Estimated time of a launch's tiles, for the shapes that untuned launches
+// choose between: every CU runs one (16 waves) or two workgroups of a shape at
+// a time, so tiles take whole rounds of 256 or 512, each at the shape's full
+// rate; a last round of up to 256 of two per CU, three quarters of one.  T
+// adds/s measured at 512 to 1024 channels, 1920 trials x 81920 samples; eight
+// waves per workgroup 1.04 to 1.36 times as long per add.
+double tile_rounds(int dtype, int shape, double tiles) {
+  const int nv = num_variants(dtype);
+  const bool pair_windows = shape == 22 || (shape == nv + 1 && (dtype == MDSM_U8 || dtype == MDSM_F16_PAIRS));
+  const double wide = dtype == MDSM_F32 ? 39.0 : (pair_windows ? 42.0 : 36.5);
+  double rate, slots = 512.0;
+  if (shape > nv) {
+    rate = wide / (pair_windows ? 1.36 : (dtype == MDSM_F32 ? 1.17 : 1.04));
+  } else if (shape == 20 || shape == 21) {
+    rate = dtype == MDSM_U8 ? 36.5 : 37.5;
+  } else {
+    rate = wide;
+    slots = 256.0;
+  }
+  const TileShape sh = variant_shape(dtype, shape);
+  double rounds = ceil(tiles / slots);
+  if (slots > 256.0 && tiles <= slots * rounds - 256.0) rounds -= 0.25;
+  return rounds * slots * sh.td() * sh.tt() / rate;
+}
+
+// The shape an untuned plan launches for its tile variant `nominal`.
+//   Eight waves instead of 16, or a pair-sum shape of smaller tiles instead of
+//   the pair windows: by the tiles' rounds (32 trials x 600000 samples x 512
+//   channels F32: 399 against 598 us; 856 channels x 1222 trials x 15994
+//   samples U8, 260 tiles of 16 waves: 540 against 766 us).
+// `fits` holds the shapes that take the survey.
+int untuned_shape(int dtype, int nominal, const std::vector<bool> &fits, uint32_t ndms, uint32_t nsamp) {
+  auto cost = [&](int shape) {
+    const TileShape sh = variant_shape(dtype, shape);
+    return tile_rounds(dtype, shape, ((double)((ndms + sh.td() - 1) / sh.td())) * ((nsamp + sh.tt() - 1) / sh.tt()));
+  };
+  int best = nominal;
+  const int narrow = narrow_variant(dtype, nominal);
+  if (!narrow) return nominal;
+  const int small = nominal == 22 ? (dtype == MDSM_U8 ? 21 : 20) : narrow;
+  for (int shape : {narrow, small})
+    if (fits[shape] && cost(shape) < cost(best)) best = shape;
+  return best;
 }
 
 TileShape variant_shape(int dtype, int variant) {
@@ -1801,7 +2146,7 @@ uint32_t lds_row_words(int dtype, int variant, uint32_t spread, const int32_t *t
   with_tile(dtype, variant, [&](auto *tp) {
     using Tile = std::remove_pointer_t<decltype(tp)>;
     rw = Tile::fits(spread) ? Tile::row_words(spread) : 0u;
-    if constexpr (IsPairSum<Tile>::value) {
+    if constexpr (IsPairSum<Tile>::value || IsWindowPair<Tile>::value) {
       if (!pairsum_accepts(table, nchans, ndms, Tile::TD, Tile::NSUM)) rw = 0;
     }
     return MDSM_OK;
@@ -1855,6 +2200,11 @@ int launch_trial_offsets(int dtype, int variant, const int32_t *table, uint32_t 
       const uint64_t nrel = (uint64_t)((ndms + Tile::TD - 1) / Tile::TD) * nblocks * 4u * Tile::Rel::WORDS;
       hipLaunchKernelGGL(pairsum_offset_kernel<Tile>, dim3((uint32_t)grid), dim3(256), 0, s, table,
                          nchans, ndms, rw, cbr, nblocks, nrel, total, reltab);
+    } else if constexpr (IsWindowPair<Tile>::value) {
+      MDSM_REQUIRE(cbr % 2u == 0u, MDSM_ERR_ARG, "pair-sum tiles stage whole channel pairs");
+      const uint64_t entries = Tile::table_entries(nchans, ndms);
+      hipLaunchKernelGGL(window_pair_table_kernel<Tile>, dim3((uint32_t)((entries + 255u) / 256u)),
+                         dim3(256), 0, s, table, nchans, ndms, rw, cbr, entries, reltab);
     } else if constexpr (IsWindow<Tile>::value) {
       const uint64_t entries = total / 8u;
       hipLaunchKernelGGL(window_table_kernel<Tile>, dim3((uint32_t)((entries + 255u) / 256u)), dim3(256),

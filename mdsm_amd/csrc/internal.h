@@ -73,9 +73,19 @@ int build_delay_table(const mdsm_survey_t *s, std::vector<int32_t> &table, uint3
 // Untuned default tile variant per storage type (the fastest measured on a
 // 1024-channel, 4096-trial beam).
 int preferred_variant(int dtype);
-// The shape an untuned plan takes when the preferred one does not take the
-// survey (F16_PAIRS, U8: the fastest shape that takes every survey).
-int fallback_variant(int dtype);
+// The shapes an untuned plan tries, n = 0, 1, .. (0: no more), when the
+// preferred one does not take the survey; after them the first one that does.
+int fallback_variant(int dtype, int n);
+// Launch shapes: the public tile variants 1..num_variants, two more that
+// untuned plans and batches choose by size (narrow_variant: the eight-wave form
+// of a 16-wave variant, 0 if it has none; its DM tiles of half the trials also
+// take surveys that a variant set by number cannot stage).
+int num_shapes(int dtype);
+int narrow_variant(int dtype, int variant);
+// Estimated time of a number of tiles of a register-window or pair-sum shape.
+double tile_rounds(int dtype, int shape, double tiles);
+// The shape an untuned plan launches where its tile variant is `nominal`.
+int untuned_shape(int dtype, int nominal, const std::vector<bool> &fits, uint32_t ndms, uint32_t nsamp);
 // Channels staged per LDS block for a tile variant and row width (0: does not fit).
 uint32_t stage_channels(int dtype, int variant, uint32_t row_words);
 // Words of a variant's trial-offset table, and the kernel that fills it
