@@ -258,8 +258,8 @@ struct mdsm_plan_s {
 static int ensure_trial_offsets(mdsm_plan_s *p, int v, hipStream_t s) {
   if (p->d_rel[v]) return MDSM_OK;
   const uint32_t rw = p->row_words[v];
-  const uint32_t cbr = stage_channels(p->dtype, v, rw);
-  MDSM_REQUIRE(rw > 0 && cbr > 0, MDSM_ERR_ARG,
+  const uint32_t cbr = v == kDirectShape ? 0u : stage_channels(p->dtype, v, rw);
+  MDSM_REQUIRE(v == kDirectShape || (rw > 0 && cbr > 0), MDSM_ERR_ARG,
                "delay spread too large for tile variant %d (choose another variant)", v);
   const uint64_t words = trial_offset_words(p->dtype, v, p->s.nchans, p->s.ndms, cbr);
   int32_t *d = nullptr;
@@ -396,7 +396,7 @@ extern "C" int mdsm_plan_set_variant(mdsm_plan plan, int variant) {
   // build the variant's trial-offset table now, so that dedisperse calls
   // (and graphs captured from them) allocate nothing
   const int v = plan_shape(plan);
-  if (variant_fits(plan, v)) {
+  if (v == kDirectShape || variant_fits(plan, v)) {
     const int rc = ensure_trial_offsets(plan, v, nullptr);
     if (rc != MDSM_OK) return rc;
   }

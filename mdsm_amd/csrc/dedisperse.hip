@@ -15,7 +15,8 @@
 // ds_read2st64).  These adds are bound by LDS reads, not by HBM, so the
 // storage formats trade LDS bytes per add.  The register-window tiles (the
 // defaults of every storage type) read a word once per wave instead of once
-// per trial and are bound by instruction issue.  The word-per-add formats:
+// per trial and are bound by instruction issue; calls of few outputs use no
+// tiles at all (direct kernel).  The word-per-add formats:
 //   F32  4 B per add: one float per LDS word, staged by direct buffer->LDS
 //        loads (buffer_load_dword ... lds) that use no data VGPRs.
 //   F16  2 B per add: LDS words hold pairs of consecutive samples in two
@@ -1881,6 +1882,105 @@ void batch_flat_kernel(const BeamDesc *__restrict__ beams,
   run_item<Tile>(beams, it, cbr, lds);
 }
 
+// ------------------------------------------------------------ direct kernel
+// Few outputs (launch_dedisperse's shape 0): tiles would leave most of the
+// chip idle while each of them walks all channels behind barriers.  A wave
+// takes 256 samples of one trial, four consecutive ones per lane, straight
+// from the rows: 16 channels' loads in flight (one access per lane and
+// channel, at any alignment), summed in channel order.  The four waves of a
+// workgroup take four consecutive trials, whose rows overlap in L1.  The table
+// is the delay table transposed, [trial][channel], 16 channels per scalar
+// load.  Lanes past the row's last whole group repeat that group (they store
+// the same values again).
+typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef _Float16 half4u __attribute__((ext_vector_type(4), aligned(2)));
+struct __attribute__((packed)) byte4u {
+  uint32_t v;
+};
+
+template <int MODE>
+__global__ __launch_bounds__(256) void dedisp_direct_kernel(const void *__restrict__ in, uint64_t ld,
+                                                            const int32_t *__restrict__ dtab,
+                                                            uint32_t nchans, uint32_t cpad, uint32_t nsamp,
+                                                            uint32_t ndms, float *__restrict__ out) {
+  typedef int32_t i32x16 __attribute__((ext_vector_type(16)));
+  typedef __attribute__((address_space(4))) const i32x16 const_i32x16;
+  const uint32_t lane = threadIdx.x & 63u;
+  // XCD x (workgroup IDs are dealt round-robin) takes time blocks x (mod 8),
+  // each with all its trials one after the other: their rows stay in its L2
+  const uint32_t ndg = (ndms + 3u) / 4u, k = blockIdx.x >> 3;
+  const uint32_t tb = (k / ndg) * 8u + (blockIdx.x & 7u);
+  const uint32_t d = uniform((k % ndg) * 4u + (threadIdx.x >> 6));
+  if (d >= ndms || tb * 256u >= nsamp) return;
+  const uint32_t t = min((tb * 64u + lane) * 4u, nsamp - 4u);
+  constexpr uint32_t SZ = MODE == MDSM_F32 ? 4u : (MODE == MDSM_U8 ? 1u : 2u);
+  const const_i32x16 *tab = (const const_i32x16 *)(uintptr_t)(dtab + (uint64_t)d * cpad);
+  const char *row = reinterpret_cast<const char *>(in);  // of the channel
+  const uint64_t step = ld * SZ;
+  const uint32_t off = t * SZ;
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+  uint32_t sum[4] = {0u, 0u, 0u, 0u};
+  auto run16 = [&](uint32_t n, i32x16 o) {
+    float4u f[16];
+    half4u h[16];
+    uint32_t u[16];
+#pragma unroll
+    for (int c = 0; c < 16; ++c) {
+      // (channels past the last one repeat it and are not added)
+      const char *q = row + (uint64_t)(uint32_t)o[c] * SZ + off;
+      if constexpr (MODE == MDSM_F32) f[c] = *reinterpret_cast<const float4u *>(q);
+      else if constexpr (MODE == MDSM_U8) u[c] = reinterpret_cast<const byte4u *>(q)->v;
+      else h[c] = *reinterpret_cast<const half4u *>(q);
+      if ((uint32_t)c + 1u < n) row += step;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < 16; ++c) {
+      if ((uint32_t)c < n) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if constexpr (MODE == MDSM_F32) {
+            acc[e] += f[c][e];
+          } else if constexpr (MODE == MDSM_F16) {
+            acc[e] += (float)h[c][e];
+          } else if constexpr (MODE == MDSM_U8) {
+            sum[e] += (u[c] >> (8 * e)) & 0xFFu;
+          } else if (c % 2 == 0) {  // channel pairs: one FP16 rounding (a last channel alone adds 0)
+            const _Float16 z = (uint32_t)c + 1u < n ? h[c + 1][e] : (_Float16)0.0f;
+            acc[e] += (float)(_Float16)(h[c][e] + z);
+          }
+        }
+      }
+    }
+  };
+  uint32_t c = 0;
+  for (; c + 16u <= nchans; c += 16u) {
+    const i32x16 o = *tab++;
+    run16(16u, o);
+    if (c + 16u < nchans) row += step;
+  }
+  if (c < nchans) {
+    const i32x16 o = *tab;
+    run16(nchans - c, o);
+  }
+  float4u v;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    v[e] = MODE == MDSM_U8 ? (float)((double)sum[e] * (8.0 / 255.0) + (double)nchans * -4.0) : acc[e];
+  *reinterpret_cast<float4u *>(out + (uint64_t)d * nsamp + t) = v;
+}
+
+// [trial][cpad] from [channel][trial]; entries past the last channel repeat it
+__global__ __launch_bounds__(256) void direct_table_kernel(const int32_t *__restrict__ table,
+                                                           uint32_t nchans, uint32_t cpad, uint32_t ndms,
+                                                           uint64_t total, int32_t *__restrict__ dtab) {
+  const uint64_t e = (uint64_t)blockIdx.x * 256u + threadIdx.x;
+  if (e >= total) return;
+  const uint32_t d = (uint32_t)(e % ndms), c = (uint32_t)(e / ndms);
+  dtab[(uint64_t)d * cpad + c] = table[(uint64_t)min(c, nchans - 1u) * ndms + d];
+}
+inline uint32_t direct_pad(uint32_t nchans) { return (nchans + 15u) & ~15u; }
+
 // ------------------------------------------------------------ variant table
 // Variant v: F32 tile (MW, K, CB) and packed tiles (MW, K2, CB) with the same
 // TD = 4*MW and similar time extent.
@@ -2089,12 +2189,20 @@ double tile_rounds(int dtype, int shape, double tiles) {
 }
 
 // The shape an untuned plan launches for its tile variant `nominal`.
+//   Direct kernel: a window tile walks all channels at 0.48 to 0.54 us per
+//   channel however few tiles there are, the direct kernel adds 7.5 (F32), 6
+//   (F16, pair sums) or 10.5 T/s (U8), which meets that at 2.2 to 4.3 million
+//   outputs (256 channels x 64 trials x 8192 samples F32: 19 against 132 us;
+//   512 x 256 x 12000: 205 against 257; x 16384: 274 against 257).
 //   Eight waves instead of 16, or a pair-sum shape of smaller tiles instead of
 //   the pair windows: by the tiles' rounds (32 trials x 600000 samples x 512
 //   channels F32: 399 against 598 us; 856 channels x 1222 trials x 15994
 //   samples U8, 260 tiles of 16 waves: 540 against 766 us).
 // `fits` holds the shapes that take the survey.
 int untuned_shape(int dtype, int nominal, const std::vector<bool> &fits, uint32_t ndms, uint32_t nsamp) {
+  const uint64_t direct_outputs = dtype == MDSM_F32 ? 3100000u : dtype == MDSM_F16 ? 2500000u
+                                  : dtype == MDSM_U8 ? 4300000u : 2200000u;
+  if (nsamp >= 256u && (uint64_t)ndms * nsamp <= direct_outputs) return kDirectShape;
   auto cost = [&](int shape) {
     const TileShape sh = variant_shape(dtype, shape);
     return tile_rounds(dtype, shape, ((double)((ndms + sh.td() - 1) / sh.td())) * ((nsamp + sh.tt() - 1) / sh.tt()));
@@ -2169,6 +2277,7 @@ uint32_t stage_channels(int dtype, int variant, uint32_t rw) {
 }
 
 uint64_t trial_offset_words(int dtype, int variant, uint32_t nchans, uint32_t ndms, uint32_t cbr) {
+  if (variant == kDirectShape) return (uint64_t)ndms * direct_pad(nchans);
   uint64_t n = 0;
   with_tile(dtype, variant, [&](auto *tp) {
     using Tile = std::remove_pointer_t<decltype(tp)>;
@@ -2188,6 +2297,13 @@ uint64_t trial_offset_words(int dtype, int variant, uint32_t nchans, uint32_t nd
 
 int launch_trial_offsets(int dtype, int variant, const int32_t *table, uint32_t nchans,
                          uint32_t ndms, uint32_t rw, uint32_t cbr, int32_t *reltab, hipStream_t s) {
+  if (variant == kDirectShape) {
+    const uint64_t total = (uint64_t)ndms * direct_pad(nchans);
+    hipLaunchKernelGGL(direct_table_kernel, dim3((uint32_t)((total + 255u) / 256u)), dim3(256), 0, s, table,
+                       nchans, direct_pad(nchans), ndms, total, reltab);
+    MDSM_HIP(hipGetLastError());
+    return MDSM_OK;
+  }
   MDSM_REQUIRE(rw > 0 && cbr > 0, MDSM_ERR_ARG, "tile variant %d cannot stage this survey", variant);
   return with_tile(dtype, variant, [&](auto *tp) -> int {
     using Tile = std::remove_pointer_t<decltype(tp)>;
@@ -2221,6 +2337,19 @@ int launch_trial_offsets(int dtype, int variant, const int32_t *table, uint32_t 
 int launch_dedisperse(int dtype, int variant, const void *in, uint64_t ld, const int32_t *table,
                       const int32_t *reltab, uint32_t nchans, uint32_t nsamp, uint32_t ndms,
                       uint32_t rw, float *out, hipStream_t s) {
+  if (variant == kDirectShape) {
+    MDSM_REQUIRE(reltab, MDSM_ERR_STATE, "delay table missing");
+    const dim3 grid(((nsamp + 255u) / 256u + 7u) / 8u * 8u * ((ndms + 3u) / 4u));
+    const uint32_t cpad = direct_pad(nchans);
+    switch (dtype) {
+      case MDSM_F32: hipLaunchKernelGGL(dedisp_direct_kernel<MDSM_F32>, grid, dim3(256), 0, s, in, ld, reltab, nchans, cpad, nsamp, ndms, out); break;
+      case MDSM_F16: hipLaunchKernelGGL(dedisp_direct_kernel<MDSM_F16>, grid, dim3(256), 0, s, in, ld, reltab, nchans, cpad, nsamp, ndms, out); break;
+      case MDSM_U8: hipLaunchKernelGGL(dedisp_direct_kernel<MDSM_U8>, grid, dim3(256), 0, s, in, ld, reltab, nchans, cpad, nsamp, ndms, out); break;
+      default: hipLaunchKernelGGL(dedisp_direct_kernel<MDSM_F16_PAIRS>, grid, dim3(256), 0, s, in, ld, reltab, nchans, cpad, nsamp, ndms, out); break;
+    }
+    MDSM_HIP(hipGetLastError());
+    return MDSM_OK;
+  }
   MDSM_REQUIRE(rw > 0, MDSM_ERR_ARG,
                "delay spread too large for tile variant %d (choose another variant)", variant);
   MDSM_REQUIRE(reltab, MDSM_ERR_STATE, "trial offset table missing for tile variant %d", variant);

@@ -79,7 +79,9 @@ int fallback_variant(int dtype, int n);
 // Launch shapes: the public tile variants 1..num_variants, two more that
 // untuned plans and batches choose by size (narrow_variant: the eight-wave form
 // of a 16-wave variant, 0 if it has none; its DM tiles of half the trials also
-// take surveys that a variant set by number cannot stage).
+// take surveys that a variant set by number cannot stage), and kDirectShape, the kernel
+// without tiles for few outputs (its table is the transposed delay table).
+constexpr int kDirectShape = 0;
 int num_shapes(int dtype);
 int narrow_variant(int dtype, int variant);
 // Estimated time of a number of tiles of a register-window or pair-sum shape.
