@@ -43,14 +43,54 @@ struct mdsm_batch_s {
 };
 
 // Adjacent time tiles per XCD group (the item order is described at
-// decode_item in dedisperse.hip).  Measured on the 32-beam batch: 4 cuts the
-// input fetched from beyond L2 from 35.7x to 19.9x the input bytes (2:
-// 23.3x; 8 overflows L2: 34.6x) and runs 0-2 % faster than 1; MDSM_TGROUP
-// (1..16) overrides it.
-static uint32_t batch_tgroup() {
+// decode_item in dedisperse.hip).  Measured on the 32-beam batch (time tiles
+// of 512 samples): 4 cuts the input fetched from beyond L2 from 35.7x to
+// 19.9x the input bytes (2: 23.3x; 8 overflows L2: 34.6x) and runs 0-2 %
+// faster than 1.  An XCD gets whole groups, so a beam of few time tiles leaves
+// some XCDs with more of them than others (41 tiles in groups of 4: 8 or 4
+// per XCD, in groups of 3: 6 or 3): of the groups up to 4, the one whose
+// busiest XCD has the fewest tiles, the largest of equals.  With the rotation
+// below: 4 beams of 0.4 to 2.6e5 samples F16 115.7 -> 108.7 ms, 3 beams through
+// a pipeline 5.91 -> 5.28 ms; two beams of up to 65536 samples 1157 -> 638 us.
+// MDSM_TGROUP (1..16) overrides it.
+static uint32_t batch_tgroup(uint32_t n_ttiles) {
   const char *e = getenv("MDSM_TGROUP");
-  const int a = e ? atoi(e) : 4;
-  return a >= 1 && a <= 16 ? (uint32_t)a : 4u;
+  const int a = e ? atoi(e) : 0;
+  if (a >= 1 && a <= 16) return (uint32_t)a;
+  uint32_t best = 1, busiest = UINT32_MAX;
+  for (uint32_t g = 1; g <= 4; ++g) {
+    const uint32_t most = (n_ttiles + 8u * g - 1u) / (8u * g) * g;
+    if (most <= busiest) {
+      best = g;
+      busiest = most;
+    }
+  }
+  return best;
+}
+
+// The slot rotation that keeps the XCDs' loads level over the beams: load[x]
+// is what XCD x has so far, and time-tile slot s of this beam (tiles n of it)
+// goes to XCD (s - rot) mod 8.
+static uint32_t batch_rotation(double (&load)[8], uint32_t n_ttiles, uint32_t tgroup, double per_tile) {
+  double slot[8] = {};
+  const uint32_t span = 8u * tgroup;
+  for (uint32_t s = 0; s < 8u; ++s) {
+    const uint32_t left = n_ttiles % span, from = s * tgroup;
+    slot[s] = per_tile * ((double)(n_ttiles / span * tgroup) +
+                          (double)(left > from ? std::min(left - from, tgroup) : 0u));
+  }
+  uint32_t best = 0;
+  double least = 0.0;
+  for (uint32_t r = 0; r < 8u; ++r) {
+    double most = 0.0;
+    for (uint32_t x = 0; x < 8u; ++x) most = std::max(most, load[x] + slot[(x + r) & 7u]);
+    if (r == 0 || most < least) {
+      best = r;
+      least = most;
+    }
+  }
+  for (uint32_t x = 0; x < 8u; ++x) load[x] += slot[(x + best) & 7u];
+  return best;
 }
 
 // A tile shape can run the batch when every beam's delay spread has an LDS
@@ -79,13 +119,15 @@ static int batch_variant(const mdsm_batch_s *b) {
   return pref;
 }
 
-// The shape a launch uses: the variant that was set or tuned, or the eight-wave
-// form of the default by the rounds of all beams' tiles (as untuned_shape).
+// The shape a launch uses: the variant that was set or tuned, or the default
+// or one of its smaller forms by the rounds of all beams' tiles (as
+// untuned_shape).
 static int batch_shape(const mdsm_batch_s *b) {
   const int v = batch_variant(b);
-  const int narrow = narrow_variant(b->dtype, v);
-  if (!narrow || !batch_fits(b, narrow)) return v;
-  if (b->variant) return batch_fits(b, v) ? v : narrow;
+  if (b->variant) {
+    const int narrow = batch_fits(b, v) ? 0 : narrow_variant(b->dtype, v);
+    return narrow && batch_fits(b, narrow) ? narrow : v;
+  }
   auto cost = [&](int shape) {
     const TileShape sh = variant_shape(b->dtype, shape);
     double tiles = 0.0, work = 0.0;
@@ -94,9 +136,12 @@ static int batch_shape(const mdsm_batch_s *b) {
       tiles += n;
       work += n * s.nchans;
     }
-    return tile_rounds(b->dtype, shape, tiles) * (work / tiles);
+    return tile_rounds(b->dtype, shape, tiles, b->beams.size() == 1) * (work / tiles);
   };
-  return cost(narrow) < cost(v) ? narrow : v;
+  int best = v;
+  for (int n = 0, shape; (shape = smaller_shape(b->dtype, v, n)) != 0; ++n)
+    if (batch_fits(b, shape) && cost(shape) < cost(best)) best = shape;
+  return best;
 }
 
 static void free_batch(mdsm_batch_s *b) {
@@ -308,6 +353,7 @@ extern "C" int mdsm_batch_bind(mdsm_batch batch, const void *const *d_in, const 
     batch->d_rel[i][v] = d;
   }
   MDSM_HIP(hipStreamSynchronize(nullptr));
+  double load[8] = {};  // work per XCD
   for (uint32_t k = 0; k < nb; ++k) {
     const uint32_t i = batch->order[k];
     const auto &s = batch->beams[i];
@@ -334,7 +380,9 @@ extern "C" int mdsm_batch_bind(mdsm_batch batch, const void *const *d_in, const 
     d.n_ttiles = (s.nsamp + sh.tt() - 1) / sh.tt();
     d.n_dtiles = (s.ndms + sh.td() - 1) / sh.td();
     d.item_begin = (uint32_t)items;
-    d.tgroup = batch_tgroup();
+    d.tgroup = batch_tgroup(d.n_ttiles);
+    d.rot = batch_rotation(load, d.n_ttiles, d.tgroup, (double)d.n_dtiles * s.nchans);
+    d.pad = 0;
     // items are numbered XCD-major: 8 slots per group of 8 * tgroup time tiles
     const uint32_t span = 8u * d.tgroup;
     items += (uint64_t)(d.n_ttiles + span - 1u) / span * span * d.n_dtiles;

@@ -1788,9 +1788,9 @@ __global__ __launch_bounds__(256) void trial_offset_kernel(const int32_t *__rest
 
 // Multi-beam item numbering (both launch shapes): a beam's items are
 // XCD-major, 8 A * ceil(n_ttiles / (8 A)) * n_dtiles of them starting at a
-// multiple of 8, A = tgroup; item g belongs to XCD slot s = g % 8, and with
-// k = (g - begin) / 8, j = k / (A n_dtiles), r = k % (A n_dtiles) it is DM
-// tile r / A of time tile 8 A j + A s + r % A: each XCD takes groups of A
+// multiple of 8, A = tgroup; item g belongs to XCD g % 8, and with slot s =
+// (g + rot) % 8, k = (g - begin) / 8, j = k / (A n_dtiles), r = k % (A
+// n_dtiles) it is DM tile r / A of time tile 8 A j + A s + r % A: each XCD takes groups of A
 // adjacent time tiles and runs a DM tile for all A of them back to back, so
 // their shifted windows overlap in its L2 (A = 1: time tile 8 j + s, DM
 // tile r).  Padding items with a time tile past the beam's end do nothing.
@@ -1816,7 +1816,7 @@ __device__ __forceinline__ BeamItem decode_item(const BeamDesc *__restrict__ bea
   BeamItem it;
   it.bd = bd;
   it.dt = r / A;
-  it.tt = 8u * A * j + A * (local & 7u) + (r - it.dt * A);
+  it.tt = 8u * A * j + A * ((local + bd->rot) & 7u) + (r - it.dt * A);
   it.valid = it.tt < bd->n_ttiles;
   return it;
 }
@@ -2163,13 +2163,21 @@ int narrow_variant(int dtype, int variant) {
   }
 }
 
+// The shapes of smaller tiles that may replace a default one (n = 0, 1, ..; 0:
+// no more).
+int smaller_shape(int dtype, int nominal, int n) {
+  if (n == 0) return narrow_variant(dtype, nominal);
+  return n == 1 && nominal == 22 ? (dtype == MDSM_U8 ? 21 : 20) : 0;
+}
+
 // Estimated time of a launch's tiles, for the shapes that untuned launches
 // choose between: every CU runs one (16 waves) or two workgroups of a shape at
 // a time, so tiles take whole rounds of 256 or 512, each at the shape's full
-// rate; a last round of up to 256 of two per CU, three quarters of one.  T
-// adds/s measured at 512 to 1024 channels, 1920 trials x 81920 samples; eight
+// rate; a last round of up to 256 of two per CU, three quarters of one.  Tiles of
+// several beams (not equal) end at different times: half a round over the
+// mean instead.  T adds/s measured at 512 to 1024 channels, 1920 trials x 81920 samples; eight
 // waves per workgroup 1.04 to 1.36 times as long per add.
-double tile_rounds(int dtype, int shape, double tiles) {
+double tile_rounds(int dtype, int shape, double tiles, bool equal) {
   const int nv = num_variants(dtype);
   const bool pair_windows = shape == 22 || (shape == nv + 1 && (dtype == MDSM_U8 || dtype == MDSM_F16_PAIRS));
   const double wide = dtype == MDSM_F32 ? 39.0 : (pair_windows ? 42.0 : 36.5);
@@ -2185,6 +2193,7 @@ double tile_rounds(int dtype, int shape, double tiles) {
   const TileShape sh = variant_shape(dtype, shape);
   double rounds = ceil(tiles / slots);
   if (slots > 256.0 && tiles <= slots * rounds - 256.0) rounds -= 0.25;
+  if (!equal && rounds > 1.0) rounds = tiles / slots + 0.5;
   return rounds * slots * sh.td() * sh.tt() / rate;
 }
 
@@ -2205,13 +2214,10 @@ int untuned_shape(int dtype, int nominal, const std::vector<bool> &fits, uint32_
   if (nsamp >= 256u && (uint64_t)ndms * nsamp <= direct_outputs) return kDirectShape;
   auto cost = [&](int shape) {
     const TileShape sh = variant_shape(dtype, shape);
-    return tile_rounds(dtype, shape, ((double)((ndms + sh.td() - 1) / sh.td())) * ((nsamp + sh.tt() - 1) / sh.tt()));
+    return tile_rounds(dtype, shape, ((double)((ndms + sh.td() - 1) / sh.td())) * ((nsamp + sh.tt() - 1) / sh.tt()), true);
   };
   int best = nominal;
-  const int narrow = narrow_variant(dtype, nominal);
-  if (!narrow) return nominal;
-  const int small = nominal == 22 ? (dtype == MDSM_U8 ? 21 : 20) : narrow;
-  for (int shape : {narrow, small})
+  for (int n = 0, shape; (shape = smaller_shape(dtype, nominal, n)) != 0; ++n)
     if (fits[shape] && cost(shape) < cost(best)) best = shape;
   return best;
 }

@@ -84,8 +84,10 @@ int fallback_variant(int dtype, int n);
 constexpr int kDirectShape = 0;
 int num_shapes(int dtype);
 int narrow_variant(int dtype, int variant);
-// Estimated time of a number of tiles of a register-window or pair-sum shape.
-double tile_rounds(int dtype, int shape, double tiles);
+// Shapes of smaller tiles in place of a default one, and the estimated time of
+// a number of tiles of one of these.
+int smaller_shape(int dtype, int nominal, int n);
+double tile_rounds(int dtype, int shape, double tiles, bool equal);
 // The shape an untuned plan launches where its tile variant is `nominal`.
 int untuned_shape(int dtype, int nominal, const std::vector<bool> &fits, uint32_t ndms, uint32_t nsamp);
 // Channels staged per LDS block for a tile variant and row width (0: does not fit).
@@ -114,6 +116,7 @@ struct BeamDesc {
   uint32_t n_ttiles, n_dtiles;
   uint32_t item_begin;  // first work item of this beam in the queue order
   uint32_t tgroup;      // adjacent time tiles per XCD group (1: every 8th time tile)
+  uint32_t rot, pad;    // XCD x takes time-tile slot (x + rot) % 8
 };
 
 int launch_batch_flat(int dtype, int variant, const BeamDesc *d_beams, uint32_t nbeams,
