@@ -210,10 +210,11 @@ extern "C" int mdsm_pipeline_candidates(mdsm_pipeline p, uint32_t beam, mdsm_can
   const uint32_t kept = std::min(cnt, p->dp.cand_cap);
   const uint32_t k = std::min(kept, cap);
   if (k) {
-    std::vector<mdsm_cand_t> all(kept);
-    MDSM_HIP(hipMemcpy(all.data(), p->d_cands[beam], kept * sizeof(mdsm_cand_t), hipMemcpyDeviceToHost));
-    mdsm_sort_candidates(all.data(), kept);
-    std::copy(all.begin(), all.begin() + k, host);
+    std::vector<mdsm_cand_t> all(k < kept ? kept : 0u);  // sorted before the cut
+    mdsm_cand_t *dst = k < kept ? all.data() : host;
+    MDSM_HIP(hipMemcpy(dst, p->d_cands[beam], kept * sizeof(mdsm_cand_t), hipMemcpyDeviceToHost));
+    mdsm_sort_candidates(dst, kept);
+    if (dst != host) std::copy(all.begin(), all.begin() + k, host);
   }
   if (cnt > p->dp.cand_cap || cnt > cap) {
     set_error("beam %u: %u candidates exceed the capacity", beam, cnt);
