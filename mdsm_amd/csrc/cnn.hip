@@ -1,8 +1,8 @@
 // cnn.hip -- BF16 MFMA kernels of the event-triage CNN (forward, backward,
 // optimiser).
 //
-// The 3x3 convolutions run as implicit products on
-// v_mfma_f32_16x16x16_bf16 with BF16 operands and FP32 accumulation, each
+// The 3x3 convolutions run as implicit products on v_mfma_f32_16x16x32_bf16
+// and v_mfma_f32_16x16x16_bf16 with BF16 operands and FP32 accumulation, each
 // fused with what follows or precedes it (forward with bias, ReLU and pool;
 // the first layer's weight gradient with the pool's backward), reading NHWC
 // activations without an im2col buffer.  The two linear layers run through
@@ -23,6 +23,8 @@
 // cross-entropy, Adam, NCHW -> NHWC input transpose, parameter layouts.  BF16 conversion is round-to-nearest-even.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "cnn_internal.h"
 
 namespace mdsm {
@@ -30,6 +32,7 @@ namespace cnn {
 namespace {
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int BM = 64, BN = 64, BK = 32, PITCH = BK + 4, NT = 256;
@@ -204,47 +207,65 @@ struct Pixel {
 };
 
 __device__ __forceinline__ bf16x4 load4(const uint16_t *p) { return *reinterpret_cast<const bf16x4 *>(p); }
+__device__ __forceinline__ uint4 load8(const uint16_t *p) { return *reinterpret_cast<const uint4 *>(p); }
+__device__ __forceinline__ f32x4 mfma32(uint4 a, uint4 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
 
 // 3x3 convolution (pad 1) + bias + ReLU + 2x2 max pool in one pass, NHWC BF16
-// in and out, FP32 accumulation on v_mfma_f32_16x16x16_bf16 over
-// k = (ky*3 + kx)*CI + ci in order.
+// in and out, FP32 accumulation over k = (ky*3 + kx)*CI + ci in order, on
+// v_mfma_f32_16x16x32_bf16 (CI = 2, k to 18: v_mfma_f32_16x16x16_bf16).
 //   A (16 x 16): rows are 4 pooled pixels x the 4 positions of their window,
 //   so a lane's four results of one output channel (D rows 4*(lane/16)+r) are
 //   one pool window and bias, ReLU and maximum need no exchange; a lane's
-//   operand is one 8-byte load of 4 channels (two 4-byte loads for CI = 2),
+//   operand is one 16-byte load of 8 channels (two 4-byte loads for CI = 2),
 //   straight from the activations (each is read 9 times, from L1/L2).
 //   B: the layer's weights, held in registers for the wave's whole run of
 //   tiles; NB output-channel tiles per wave.
 // a[pooled][CO] = BF16 of the maximum, idx = argmax (0..3, first maximum) | 4
 // when the maximum is positive.  Storing the FP32 pre-activations and pooling
 // them in a second pass moved 8 bytes per pixel and channel: 256 snippets of
-// 64 x 256, three layers: 320 + 117 + 57 us, now 46 + 44 + 41.  Bound by the
-// activation loads (9 per element, L1 and L2).
+// 64 x 256, three layers: 320 + 117 + 57 us, now 46 + 33 + 29 (45 and 41 with
+// 16-deep steps and 8-byte loads).  Bound by the activation loads (9 per
+// element, L1 and L2).
 template <int CI, int CO, int NB>
 __global__ __launch_bounds__(NT) void conv_pool_kernel(const uint16_t *__restrict__ x,
                                                        const uint16_t *__restrict__ wt,
                                                        const float *__restrict__ bias, int64_t P, int H,
                                                        int W, int run, uint16_t *__restrict__ a,
                                                        uint8_t *__restrict__ idx) {
-  constexpr int KC = (9 * CI + 15) / 16;  // 16-deep steps
+  constexpr int DEPTH = CI == 2 ? 16 : 32;             // k values per step, DEPTH / 4 per lane
+  constexpr int KC = (9 * CI + DEPTH - 1) / DEPTH;
+  using Operand = std::conditional_t<CI == 2, bf16x4, uint4>;
   const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
   const int Ho = H / 2, Wo = W / 2;
   const int n0 = blockIdx.y * NB * 16;
-  bf16x4 bw[KC][NB];
+  Operand bw[KC][NB];
 #pragma unroll
   for (int c = 0; c < KC; ++c)
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
-      const uint16_t *q = wt + (int64_t)(n0 + 16 * j + n) * (9 * CI) + 16 * c + 4 * g;
+      const int k = DEPTH * c + DEPTH / 4 * g;
+      const uint16_t *q = wt + (int64_t)(n0 + 16 * j + n) * (9 * CI) + k;
       if constexpr (CI == 2) {  // rows of 18, 4-byte aligned
-        const int k = 16 * c + 4 * g;
         const uint32_t lo = k < 18 ? *reinterpret_cast<const uint32_t *>(q) : 0u;
         const uint32_t hi = k + 2 < 18 ? *reinterpret_cast<const uint32_t *>(q + 2) : 0u;
         bw[c][j] = __builtin_bit_cast(bf16x4, ((uint64_t)hi << 32) | lo);
       } else {
-        bw[c][j] = load4(q);
+        bw[c][j] = k < 9 * CI ? load8(q) : make_uint4(0u, 0u, 0u, 0u);
       }
     }
+  // CI = 16: a step holds two taps, the lanes of g < 2 the first; this lane's
+  // tap of each step (9 past the last: outside everywhere)
+  int dy[KC], dx[KC];
+  if constexpr (CI != 2) {
+#pragma unroll
+    for (int c = 0; c < KC; ++c) {
+      const int t = CI == 16 ? 2 * c + (g >> 1) : c * 32 / CI;
+      dy[c] = t < 9 ? t / 3 - 1 : H;
+      dx[c] = t % 3 - 1;
+    }
+  }
   float bs[NB];
 #pragma unroll
   for (int j = 0; j < NB; ++j) bs[j] = bias[n0 + 16 * j + n];
@@ -258,11 +279,6 @@ __global__ __launch_bounds__(NT) void conv_pool_kernel(const uint16_t *__restric
   for (; p < pend; p += 4) {
     const int h = 2 * px.h + ((n >> 1) & 1), w = 2 * px.w + (n & 1);
     const uint16_t *q = x + ((px.b * H + h) * W + w) * CI;
-    auto tap = [&](int t, bool &ok) {  // address of the tap's pixel, itself when outside
-      const int ky = t / 3, kx = t - 3 * ky;
-      ok = (ky != 0 || h > 0) && (ky != 2 || h < H - 1) && (kx != 0 || w > 0) && (kx != 2 || w < W - 1);
-      return q + (ok ? ((ky - 1) * W + (kx - 1)) * CI : 0);
-    };
     f32x4 acc[NB];
 #pragma unroll
     for (int j = 0; j < NB; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -288,20 +304,19 @@ __global__ __launch_bounds__(NT) void conv_pool_kernel(const uint16_t *__restric
         acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a1, bw[1][j], acc[j], 0, 0, 0);
       }
     } else {
-      bf16x4 av[KC];
+      uint4 av[KC];
 #pragma unroll
       for (int c = 0; c < KC; ++c) {
-        bool ok;
-        const uint16_t *s = tap(c * 16 / CI, ok);
-        av[c] = load4(s + c * 16 % CI + 4 * g);
-        if (!ok) av[c] = bf16x4{0, 0, 0, 0};
+        const int hh = h + dy[c], ww = w + dx[c];
+        const bool ok = (unsigned)hh < (unsigned)H && (unsigned)ww < (unsigned)W;
+        av[c] = load8(q + (ok ? (dy[c] * W + dx[c]) * CI : 0) + (8 * g) % CI);
+        if (!ok) av[c] = make_uint4(0u, 0u, 0u, 0u);
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int c = 0; c < KC; ++c)
 #pragma unroll
-        for (int j = 0; j < NB; ++j)
-          acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av[c], bw[c][j], acc[j], 0, 0, 0);
+        for (int j = 0; j < NB; ++j) acc[j] = mfma32(av[c], bw[c][j], acc[j]);
     }
     if (p + g < P) {
 #pragma unroll
@@ -332,20 +347,29 @@ __global__ __launch_bounds__(NT) void conv_pool_kernel(const uint16_t *__restric
 // w[co][tap][ci], FP32.  As the forward kernel, with 16 consecutive pixels as
 // rows; wf: the weights as [ci][(ky*3 + kx)*CO + co] (weights_flip_kernel).
 // Bound by its gradient loads; every input-channel tile in one wave reads
-// them once (64 -> 32 channels, 256 snippets: 98 us, 158 with a wave per
-// tile; 32 -> 16: 78 us, 148 as an im2col product).
+// them once.  256 snippets: 64 -> 32 channels 43 us (98 with 8-byte loads and
+// the weights in 144 registers of every wave instead of 36 KB of LDS), 32 -> 16
+// 48 us (78 with 8-byte loads, 148 as an im2col product).
 template <int CO, int CI, int NB>
 __global__ __launch_bounds__(NT) void conv_dx_kernel(const uint16_t *__restrict__ dz,
                                                      const uint16_t *__restrict__ wf, int64_t P, int H,
                                                      int W, int run, float *__restrict__ dx) {
-  constexpr int KC = 9 * CO / 16;
+  constexpr int KC = 9 * CO / 32;
+  constexpr bool LW = KC * NB > 18;  // weights in LDS
   const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
   const int n0 = blockIdx.y * NB * 16;
-  bf16x4 bw[KC][NB];
+  __shared__ uint4 ws[LW ? KC * NB * 64 : 1];
+  uint4 bw[LW ? 1 : KC][NB];
+  auto weight = [&](int c, int j) { return load8(wf + (int64_t)(n0 + 16 * j + n) * (9 * CO) + 32 * c + 8 * g); };
+  if constexpr (LW) {
+    for (int i = threadIdx.x >> 6; i < KC * NB; i += NT / 64) ws[i * 64 + lane] = weight(i / NB, i % NB);
+    __syncthreads();
+  } else {
 #pragma unroll
-  for (int c = 0; c < KC; ++c)
+    for (int c = 0; c < KC; ++c)
 #pragma unroll
-    for (int j = 0; j < NB; ++j) bw[c][j] = load4(wf + (int64_t)(n0 + 16 * j + n) * (9 * CO) + 16 * c + 4 * g);
+      for (int j = 0; j < NB; ++j) bw[c][j] = weight(c, j);
+  }
   const int64_t wave = (int64_t)blockIdx.x * (NT / 64) + (threadIdx.x >> 6);
   int64_t p = wave * run * 16;
   const int64_t pend = p + (int64_t)run * 16 < P ? p + (int64_t)run * 16 : P;
@@ -357,27 +381,21 @@ __global__ __launch_bounds__(NT) void conv_dx_kernel(const uint16_t *__restrict_
     f32x4 acc[NB];
 #pragma unroll
     for (int j = 0; j < NB; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // the loads of HALF steps are issued together ahead of their products
-    constexpr int HALF = KC > 18 ? KC / 2 : KC;
+    uint4 av[KC];
 #pragma unroll
-    for (int c0 = 0; c0 < KC; c0 += HALF) {
-      bf16x4 av[HALF];
-#pragma unroll
-      for (int c = 0; c < HALF; ++c) {
-        const int t = (c0 + c) / (CO / 16), cc = (c0 + c) % (CO / 16);
-        const int ky = t / 3, kx = t - 3 * ky;  // reads (h - ky + 1, w - kx + 1)
-        const bool ok = (ky != 2 || px.h > 0) && (ky != 0 || px.h < H - 1) && (kx != 2 || px.w > 0) &&
-                        (kx != 0 || px.w < W - 1);
-        av[c] = load4(q + (ok ? ((1 - ky) * W + (1 - kx)) * CO : 0) + 16 * cc + 4 * g);
-        if (!ok) av[c] = bf16x4{0, 0, 0, 0};
-      }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int c = 0; c < HALF; ++c)
-#pragma unroll
-        for (int j = 0; j < NB; ++j)
-          acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av[c], bw[c0 + c][j], acc[j], 0, 0, 0);
+    for (int c = 0; c < KC; ++c) {
+      const int t = c / (CO / 32), cc = c % (CO / 32);
+      const int ky = t / 3, kx = t - 3 * ky;  // reads (h - ky + 1, w - kx + 1)
+      const bool ok = (ky != 2 || px.h > 0) && (ky != 0 || px.h < H - 1) && (kx != 2 || px.w > 0) &&
+                      (kx != 0 || px.w < W - 1);
+      av[c] = load8(q + (ok ? ((1 - ky) * W + (1 - kx)) * CO : 0) + 32 * cc + 8 * g);
+      if (!ok) av[c] = make_uint4(0u, 0u, 0u, 0u);
     }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < KC; ++c)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) acc[j] = mfma32(av[c], LW ? ws[(c * NB + j) * 64 + lane] : bw[LW ? 0 : c][j], acc[j]);
 #pragma unroll
     for (int j = 0; j < NB; ++j)
 #pragma unroll
@@ -839,8 +857,8 @@ int conv_pool(int layer, const uint16_t *x, int64_t B, int H, int W, const uint1
     case 1: hipLaunchKernelGGL((conv_pool_kernel<16, 32, 2>), dim3(gx, 1), dim3(NT), 0, s, x, w, bias, P, H, W, run, a, idx); break;
     default:
       // all four output tiles in one wave read the activations once (256
-      // snippets of 64 x 256: 41 us, 53 with two waves of two tiles); with
-      // few tiles the second wave is worth more (24 snippets: 12 against 13)
+      // snippets of 64 x 256: 29 us, more with two waves of two tiles); with
+      // few tiles the second wave is worth more (24 snippets: 7 us)
       if (tiles >= 8192)
         hipLaunchKernelGGL((conv_pool_kernel<32, 64, 4>), dim3(gx, 1), dim3(NT), 0, s, x, w, bias, P, H, W, run, a, idx);
       else
