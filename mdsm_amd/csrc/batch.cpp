@@ -139,7 +139,7 @@ static int batch_shape(const mdsm_batch_s *b) {
     return tile_rounds(b->dtype, shape, tiles, b->beams.size() == 1) * (work / tiles);
   };
   int best = v;
-  for (int n = 0, shape; (shape = smaller_shape(b->dtype, v, n)) != 0; ++n)
+  for (int n = 0, shape; (shape = other_shape(b->dtype, v, n)) != 0; ++n)
     if (batch_fits(b, shape) && cost(shape) < cost(best)) best = shape;
   return best;
 }

@@ -2163,11 +2163,20 @@ int narrow_variant(int dtype, int variant) {
   }
 }
 
-// The shapes of smaller tiles that may replace a default one (n = 0, 1, ..; 0:
-// no more).
-int smaller_shape(int dtype, int nominal, int n) {
-  if (n == 0) return narrow_variant(dtype, nominal);
-  return n == 1 && nominal == 22 ? (dtype == MDSM_U8 ? 21 : 20) : 0;
+// The shapes that may replace a default one where its tiles pad too much (n =
+// 0, 1, ..; 0: no more): those of smaller or, after 20 and 21, fewer tiles.
+int other_shape(int dtype, int nominal, int n) {
+  const int nv = num_variants(dtype);
+  if (dtype == MDSM_U8) {
+    static const int after22[] = {23, 21, 0}, after21[] = {2, 24, 0}, after2[] = {24, 0};
+    return nominal == 22 ? after22[n] : (nominal == 21 ? after21[n] : (nominal == 2 ? after2[n] : 0));
+  }
+  if (dtype == MDSM_F16_PAIRS) {
+    static const int after22[] = {23, 20, 0}, after20[] = {21, 16, 15, 0};
+    if (nominal == 22) return after22[n];
+    return nominal == 20 ? after20[n] : (nominal == 21 ? after20[n + 1] : (nominal == 16 ? after20[n + 2] : 0));
+  }
+  return n == 0 && nominal == 12 ? nv + 1 : 0;
 }
 
 // Estimated time of a launch's tiles, for the shapes that untuned launches
@@ -2180,12 +2189,15 @@ int smaller_shape(int dtype, int nominal, int n) {
 double tile_rounds(int dtype, int shape, double tiles, bool equal) {
   const int nv = num_variants(dtype);
   const bool pair_windows = shape == 22 || (shape == nv + 1 && (dtype == MDSM_U8 || dtype == MDSM_F16_PAIRS));
-  const double wide = dtype == MDSM_F32 ? 39.0 : (pair_windows ? 42.0 : 36.5);
+  const double wide = dtype == MDSM_F32 ? 39.0 : (pair_windows ? 42.0 : (dtype == MDSM_U8 ? 34.5 : 36.5));
   double rate, slots = 512.0;
   if (shape > nv) {
     rate = wide / (pair_windows ? 1.36 : (dtype == MDSM_F32 ? 1.17 : 1.04));
-  } else if (shape == 20 || shape == 21) {
-    rate = dtype == MDSM_U8 ? 36.5 : 37.5;
+  } else if (shape == 20 || shape == 21 || shape == 16) {
+    rate = dtype == MDSM_U8 ? 36.5 : (shape == 20 ? 37.5 : (shape == 21 ? 33.0 : 31.0));
+  } else if (dtype == MDSM_F16_PAIRS && shape == 15) {
+    rate = 25.0;  // bound by LDS reads, few of its workgroups fill a CU
+    slots = 256.0;
   } else {
     rate = wide;
     slots = 256.0;
@@ -2203,8 +2215,9 @@ double tile_rounds(int dtype, int shape, double tiles, bool equal) {
 //   (F16, pair sums) or 10.5 T/s (U8), which meets that at 2.2 to 4.3 million
 //   outputs (256 channels x 64 trials x 8192 samples F32: 19 against 132 us;
 //   512 x 256 x 12000: 205 against 257; x 16384: 274 against 257).
-//   Eight waves instead of 16, or a pair-sum shape of smaller tiles instead of
-//   the pair windows: by the tiles' rounds (32 trials x 600000 samples x 512
+//   Eight waves instead of 16, or a shape that pads the trials less: by the
+//   tiles' rounds (46 trials x 218486 samples x 295 channels F16_PAIRS, delay
+//   differences for 40 trials: 264 us in two such tiles, 205 in one of 48; 32 trials x 600000 samples x 512
 //   channels F32: 399 against 598 us; 856 channels x 1222 trials x 15994
 //   samples U8, 260 tiles of 16 waves: 540 against 766 us).
 // `fits` holds the shapes that take the survey.
@@ -2217,7 +2230,7 @@ int untuned_shape(int dtype, int nominal, const std::vector<bool> &fits, uint32_
     return tile_rounds(dtype, shape, ((double)((ndms + sh.td() - 1) / sh.td())) * ((nsamp + sh.tt() - 1) / sh.tt()), true);
   };
   int best = nominal;
-  for (int n = 0, shape; (shape = smaller_shape(dtype, nominal, n)) != 0; ++n)
+  for (int n = 0, shape; (shape = other_shape(dtype, nominal, n)) != 0; ++n)
     if (fits[shape] && cost(shape) < cost(best)) best = shape;
   return best;
 }

@@ -84,9 +84,9 @@ int fallback_variant(int dtype, int n);
 constexpr int kDirectShape = 0;
 int num_shapes(int dtype);
 int narrow_variant(int dtype, int variant);
-// Shapes of smaller tiles in place of a default one, and the estimated time of
+// Shapes that may replace a default one, and the estimated time of
 // a number of tiles of one of these.
-int smaller_shape(int dtype, int nominal, int n);
+int other_shape(int dtype, int nominal, int n);
 double tile_rounds(int dtype, int shape, double tiles, bool equal);
 // The shape an untuned plan launches where its tile variant is `nominal`.
 int untuned_shape(int dtype, int nominal, const std::vector<bool> &fits, uint32_t ndms, uint32_t nsamp);
