@@ -207,6 +207,13 @@ struct Pixel {
 };
 
 __device__ __forceinline__ bf16x4 load4(const uint16_t *p) { return *reinterpret_cast<const bf16x4 *>(p); }
+// Four pixels of one channel per lane from pixel-major LDS rows: in each group
+// of 16 lanes, lane j names 4 channels (j % 4) of pixel j / 4 and lane n gets
+// channel n of the four pixels.
+__device__ __forceinline__ bf16x4 load_transposed(const uint16_t *p) {
+  typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_bf16x4 *)p);
+}
 __device__ __forceinline__ uint4 load8(const uint16_t *p) { return *reinterpret_cast<const uint4 *>(p); }
 __device__ __forceinline__ f32x4 mfma32(uint4 a, uint4 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
@@ -421,15 +428,16 @@ __global__ void weights_flip_kernel(const uint16_t *__restrict__ w, int CI, int 
 // the reduction, so both operands need 4 consecutive pixels of one channel
 // per lane while the activations are stored channel by channel of a pixel.
 // A workgroup stages WR rows x WC columns of dz and of x (with a border) in
-// LDS and its lanes gather the pixels with 2-byte reads; the three taps of a
-// kernel row share one window of 6 pixels.  The pixel pitch is 8 bytes more
-// than the channels take, which spreads the four 16-lane groups (4 pixels
-// apart) over the banks.  A wave owns CT output-channel tiles x 9*CI/16
+// LDS and its lanes read them transposed (ds_read_b64_tr_b16).  The pixel pitch
+// is 8 bytes more than the channels take, which spreads a group's four pixels
+// over the banks.  A wave owns CT output-channel tiles x 9*CI/16
 // column tiles (72 accumulator registers); with CO > 16 CT the waves split the
 // output channels, and otherwise the workgroup's pixels (their sums are added
 // in LDS).  Each workgroup writes one partial; sum_rows_kernel adds them.
-// Bound by the 2-byte LDS reads: 256 snippets 73 + 5 us (32 channels) and 46
-// + 13 us (64), 377 and 187 as split im2col products.
+// An item's loads are in registers while the products of the one before run.
+// 256 snippets: 35 + 5 us (32 channels) and 30 + 13 us (64); 73 and 46 with the
+// loads between the barriers and 2-byte LDS reads (transposed reads alone: 70
+// and 42), 377 and 187 as split im2col products.
 constexpr int WR = 2, WC = 64;
 template <int CI, int CO, int CT>
 __global__ __launch_bounds__(NT) void conv_dw_kernel(const uint16_t *__restrict__ dz,
@@ -450,49 +458,60 @@ __global__ __launch_bounds__(NT) void conv_dw_kernel(const uint16_t *__restrict_
     for (int j = 0; j < NTILE; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int nh = (H + WR - 1) / WR, nw = (W + WC - 1) / WC;
   const int64_t items = B * nh * nw;
-  for (int64_t it = blockIdx.x; it < items; it += gridDim.x) {
+  constexpr int NZ = WR * WC * (CO / 4), NX = (WR + 2) * XW * (CI / 4);  // 8-byte pieces of an item
+  constexpr int RZ = (NZ + NT - 1) / NT, RX = (NX + NT - 1) / NT;
+  uint2 vz[RZ], vx[RX];
+  auto fetch = [&](int64_t it) {
     const int iw = (int)(it % nw);
     const int64_t r0 = it / nw;
-    const int ih = (int)(r0 % nh);
+    const int h0 = (int)(r0 % nh) * WR, w0 = iw * WC;
     const int64_t b = r0 / nh;
-    const int h0 = ih * WR, w0 = iw * WC;
-    __syncthreads();
-    for (int i = threadIdx.x; i < WR * WC * (CO / 4); i += NT) {
-      const int c = i % (CO / 4), q = i / (CO / 4), ww = q % WC, hh = q / WC;
-      uint2 v = make_uint2(0u, 0u);
-      if (h0 + hh < H && w0 + ww < W)
-        v = *reinterpret_cast<const uint2 *>(dz + ((b * H + h0 + hh) * W + w0 + ww) * CO + 4 * c);
-      *reinterpret_cast<uint2 *>(sz + (hh * WC + ww) * PZ + 4 * c) = v;
+#pragma unroll
+    for (int r = 0; r < RZ; ++r) {
+      const int i = threadIdx.x + r * NT, c = i % (CO / 4), q = i / (CO / 4), hs = h0 + q / WC, wsrc = w0 + q % WC;
+      vz[r] = make_uint2(0u, 0u);
+      if (i < NZ && hs < H && wsrc < W)
+        vz[r] = *reinterpret_cast<const uint2 *>(dz + ((b * H + hs) * W + wsrc) * CO + 4 * c);
     }
-    for (int i = threadIdx.x; i < (WR + 2) * XW * (CI / 4); i += NT) {
-      const int c = i % (CI / 4), q = i / (CI / 4), ww = q % XW, hh = q / XW;
-      const int hs = h0 + hh - 1, wsrc = w0 + ww - 1;
-      uint2 v = make_uint2(0u, 0u);
-      if (hs >= 0 && hs < H && wsrc >= 0 && wsrc < W)
-        v = *reinterpret_cast<const uint2 *>(x + ((b * H + hs) * W + wsrc) * CI + 4 * c);
-      *reinterpret_cast<uint2 *>(sx + (hh * XW + ww) * PX + 4 * c) = v;
+#pragma unroll
+    for (int r = 0; r < RX; ++r) {
+      const int i = threadIdx.x + r * NT, c = i % (CI / 4), q = i / (CI / 4);
+      const int hs = h0 + q / XW - 1, wsrc = w0 + q % XW - 1;
+      vx[r] = make_uint2(0u, 0u);
+      if (i < NX && hs >= 0 && hs < H && wsrc >= 0 && wsrc < W)
+        vx[r] = *reinterpret_cast<const uint2 *>(x + ((b * H + hs) * W + wsrc) * CI + 4 * c);
+    }
+  };
+  if (blockIdx.x < items) fetch(blockIdx.x);
+  for (int64_t it = blockIdx.x; it < items; it += gridDim.x) {
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < RZ; ++r) {
+      const int i = threadIdx.x + r * NT, c = i % (CO / 4), q = i / (CO / 4);
+      if (i < NZ) *reinterpret_cast<uint2 *>(sz + q * PZ + 4 * c) = vz[r];
+    }
+#pragma unroll
+    for (int r = 0; r < RX; ++r) {
+      const int i = threadIdx.x + r * NT, c = i % (CI / 4), q = i / (CI / 4);
+      if (i < NX) *reinterpret_cast<uint2 *>(sx + q * PX + 4 * c) = vx[r];
     }
     __syncthreads();
+    if (it + gridDim.x < items) fetch(it + gridDim.x);  // under this item's products
     for (int ks = kw; ks < WR * WC / 16; ks += KS) {
       const int hh = ks / (WC / 16), wb = (ks % (WC / 16)) * 16 + 4 * g;  // this lane's first pixel
       bf16x4 av[CT];
 #pragma unroll
       for (int i = 0; i < CT; ++i) {
-        const uint16_t *q = sz + (hh * WC + wb) * PZ + (ws * CT + i) * 16 + n;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) av[i][e] = (short)q[e * PZ];
+        av[i] = load_transposed(sz + (hh * WC + wb + n / 4) * PZ + (ws * CT + i) * 16 + 4 * (n & 3));
       }
 #pragma unroll
       for (int ky = 0; ky < 3; ++ky)
 #pragma unroll
         for (int cc = 0; cc < CI / 16; ++cc) {
-          const uint16_t *q = sx + ((hh + ky) * XW + wb) * PX + 16 * cc + n;
-          short v[6];
-#pragma unroll
-          for (int e = 0; e < 6; ++e) v[e] = (short)q[e * PX];
+          const uint16_t *q = sx + ((hh + ky) * XW + wb + n / 4) * PX + 16 * cc + 4 * (n & 3);
 #pragma unroll
           for (int kx = 0; kx < 3; ++kx) {
-            const bf16x4 bv = {v[kx], v[kx + 1], v[kx + 2], v[kx + 3]};
+            const bf16x4 bv = load_transposed(q + kx * PX);
             const int j = (ky * 3 + kx) * (CI / 16) + cc;
 #pragma unroll
             for (int i = 0; i < CT; ++i)
