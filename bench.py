@@ -40,8 +40,8 @@ from mdsm_amd import abi  # noqa: E402
 
 HBM_PEAK = 8.0e12        # MI355X HBM3E, bytes/s
 LDS_PEAK = 256 * 128 * 2.4e9  # bytes/s: 128 B per clock per CU, 256 CUs at 2.4 GHz
-VALU_ADD_PEAK = 39.3e12  # FP32 vector adds/s, one per lane per clock (157.3 TFLOP/s counts
-                         # packed FMA as 4 flops; packed FP32 is not used here)
+VALU_ADD_PEAK = 78.6e12  # FP32 vector adds/s: 128 lanes per clock per CU (157.3 TFLOP/s of FMA);
+                         # a loop of plain v_add_f32 reaches 64e12
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic_batch_fp16.json")
 FCH1, BAND, TSAMP = 1500.0, 300.0, 64e-6
 
@@ -801,6 +801,7 @@ def main():
         else:
             log(f"no traffic profile of tile variant {v16} (profiled: {sorted(tr.get('by_variant', {}))}): "
                 "roofline.traffic left null")
+    lds_add = 1.2 if v16 == 12 and hdt == abi.F16 else 2.0
     line = {
         "metric": {abi.F16: "dedispersed DM x samples per second (batched, FP16 storage)",
                    abi.F16_PAIRS: "dedispersed DM x samples per second (batched, FP16 storage, channel-pair sums)",
@@ -826,10 +827,11 @@ def main():
                      "algorithmic_bytes_per_launch": B16, "measured_copy_gbs": copy_gbs},
         "valu": {"adds_per_s": total_adds / (ms16 / 1e3), "peak_adds_per_s": VALU_ADD_PEAK,
                  "frac": total_adds / (ms16 / 1e3) / VALU_ADD_PEAK},
-        # algorithmic LDS reads of the FP16 tiles: half a 4-byte word (one
-        # 16-bit sample) per add
-        "lds": {"achieved": 2.0 * total_adds / (ms16 / 1e3), "peak": LDS_PEAK, "unit": "B/s",
-                "frac": 2.0 * total_adds / (ms16 / 1e3) / LDS_PEAK, "bytes_per_add": 2},
+        # algorithmic LDS reads per add: the register windows (variant 12) read
+        # at least 24 words for the 80 adds of a lane and channel, the other
+        # FP16 tiles half a word (one 16-bit sample) per add
+        "lds": {"achieved": lds_add * total_adds / (ms16 / 1e3), "peak": LDS_PEAK, "unit": "B/s",
+                "frac": lds_add * total_adds / (ms16 / 1e3) / LDS_PEAK, "bytes_per_add": lds_add},
         "batched_u8": u8,
         "batched_fp16_pairs": pairs,
         "batched_fp16_pairs_vs_plain_fp32": (pairs["dm_samples_per_s"] / plain["dm_samples_per_s"])
