@@ -133,8 +133,8 @@ int mdsm_plan_device_table(mdsm_plan plan, const int32_t **table);
  * or exact u16) once per delay difference of its two channels; those take
  * a survey only when that
  * difference is >= 0 and spans at most 3 values (19: 4) in every DM tile of
- * the shape, and a shape that does not take the survey makes
- * mdsm_dedisperse fail with MDSM_ERR_ARG (the autotuners skip it).  Every
+ * the shape (22: or of its half-width form), and a shape that does not take
+ * the survey makes mdsm_dedisperse fail with MDSM_ERR_ARG (the autotuners skip it).  Every
  * shape of a storage type gives the same results.  Setting a variant builds
  * its trial-offset table (one allocation and one kernel, synchronous); a
  * variant first used by mdsm_dedisperse without being set builds it there,
@@ -144,15 +144,19 @@ int mdsm_plan_get_variant(mdsm_plan plan, int *variant);
 int mdsm_tile_variants(int in_dtype, int *count);
 /* The untuned default tile shape of a storage type.  A plan or batch uses
  * it when it takes the survey; otherwise MDSM_F16_PAIRS and MDSM_U8 fall
- * back to shapes 15 and 2 (which take every survey whose delay spread they
- * can stage), and any type to the first shape that can. */
+ * back through pair-sum shapes of fewer trials to shapes 15 and 2 (which take
+ * every survey whose delay spread they can stage), and any type to the first
+ * shape that can.  An untuned plan or batch may launch a smaller form of that
+ * shape, or for few outputs a kernel without tiles, with the same results;
+ * mdsm_plan_get_variant names the shape it stands for. */
 int mdsm_tile_preferred(int in_dtype, int *variant);
 /* Channels a tile shape stages per LDS block for this plan's delay spread;
  * 0 when the shape cannot stage it. */
 int mdsm_plan_variant_channels(mdsm_plan plan, int variant, uint32_t *channels);
 /* Time each tile variant on the given buffers (best of three launches after
  * a warm-up) and keep the fastest; the storage type's default variant is
- * kept when it is within 2 % of the fastest. */
+ * kept when it is within 2 % of the fastest, and the plan stays untuned when
+ * what it launches then is faster than all of them. */
 int mdsm_plan_autotune(mdsm_plan plan, const void *d_in, uint64_t ld, float *d_out, void *stream,
                        int *best_variant, float *best_ms);
 

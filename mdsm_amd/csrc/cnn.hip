@@ -206,7 +206,6 @@ struct Pixel {
   }
 };
 
-__device__ __forceinline__ bf16x4 load4(const uint16_t *p) { return *reinterpret_cast<const bf16x4 *>(p); }
 // Four pixels of one channel per lane from pixel-major LDS rows: in each group
 // of 16 lanes, lane j names 4 channels (j % 4) of pixel j / 4 and lane n gets
 // channel n of the four pixels.
