@@ -11,6 +11,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <mutex>
 #include <random>
 #include <vector>
 
@@ -70,6 +71,7 @@ struct mdsm_cnn_s {
   int last_batch = 0;
   int step = 0;
   std::vector<void *> allocs;
+  std::mutex read;  // held from canon's kernel to its download
 };
 
 namespace {
@@ -193,7 +195,8 @@ extern "C" int mdsm_cnn_set_params(mdsm_cnn n, const float *host) {
 }
 
 // (the layouts are exchanged on the device: one pass and one copy instead of
-// a copy, an index map and a gather on the host)
+// a copy, an index map and a gather on the host; threads reading one network
+// take turns at its staging buffer)
 static int get_canonical(mdsm_cnn n, const float *dsrc, float *host) {
   MDSM_REQUIRE(n && host, MDSM_ERR_ARG, "null argument");
   const Layout &L = n->L;
@@ -209,6 +212,7 @@ static int get_canonical(mdsm_cnn n, const float *dsrc, float *host) {
   c.hid = HID;
   c.pix = (n->H / 8) * (n->W / 8);
   c.chan = CH[3];
+  const std::lock_guard<std::mutex> lock(n->read);
   MDSM_HIP(hipDeviceSynchronize());
   const int rc = cnn::to_canonical(dsrc, c, n->canon, nullptr);
   if (rc != MDSM_OK) return rc;
