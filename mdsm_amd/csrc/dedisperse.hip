@@ -1855,13 +1855,15 @@ void batch_kernel(const BeamDesc *__restrict__ beams,
                                                     uint32_t nbeams, uint32_t total_items,
                                                     uint32_t cbr, uint32_t *__restrict__ counter) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
-  __shared__ uint32_t item_s;
+  // the item goes through the tile's first word: a tile may take all of a
+  // CU's LDS, and any word beside it would make that launch fail
+  uint32_t *const item_s = reinterpret_cast<uint32_t *>(lds);
   const uint32_t slot = blockIdx.x & 7u;
   while (true) {
-    if (threadIdx.x == 0) item_s = atomicAdd(counter + slot, 1u) * 8u + slot;
+    if (threadIdx.x == 0) *item_s = atomicAdd(counter + slot, 1u) * 8u + slot;
     __syncthreads();
     // wave-uniform: the descriptor lookup and every tile parameter stay scalar
-    const uint32_t item = uniform(item_s);
+    const uint32_t item = uniform(*item_s);
     __syncthreads();
     if (item >= total_items) break;
     const BeamItem it = decode_item(beams, nbeams, item);
@@ -2096,8 +2098,7 @@ int with_tile(int dtype, int variant, Fn &&fn) {
 // CU, take its 160 KB in one workgroup of 16 waves or two of eight.
 template <typename Tile>
 constexpr uint64_t tile_lds() {
-  // (256 bytes spare for static LDS)
-  if constexpr (IsWindow<Tile>::value) return (Tile::WAVES == 8 ? 80 : 160) * 1024 - 256;
+  if constexpr (IsWindow<Tile>::value) return (Tile::WAVES == 8 ? 80 : 160) * 1024;
   else return 64 * 1024;
 }
 
