@@ -126,9 +126,10 @@ typedef unsigned short ushort4u __attribute__((ext_vector_type(4), aligned(4)));
 // Each thread takes NORM_Q groups of four consecutive samples, a workgroup
 // NORM_Q * 1024 of them.  HBM-bound: one element per load and store moved
 // 4.1 TB/s (1024 channels x 144321 samples to F16, 214 us), four 6.4 TB/s
-// (139 us).  Rows
-// that do not start on 4-byte boundaries (F16 rows of odd length, U8 rows of
-// a length that is no multiple of 4) are stored element by element.
+// (139 us).  Rows that do not start on 4-byte boundaries (F16 rows of odd
+// length, U8 rows of a length that is no multiple of 4) are stored element by
+// element, neighbouring lanes at neighbouring elements (1024 rows of 2^17
+// samples to odd F16 rows 141 us, 240 with four of a lane's elements in turn).
 constexpr int NORM_Q = 2;
 template <int DT, bool WIDE>
 __global__ __launch_bounds__(NT) void normalise_kernel(const float *__restrict__ raw, uint64_t ld,
@@ -146,6 +147,26 @@ __global__ __launch_bounds__(NT) void normalise_kernel(const float *__restrict__
   auto f16 = [](double v) { return __half_as_ushort(__float2half_rn((float)v)); };
   for (uint64_t base = (uint64_t)blockIdx.x * (NT * 4 * NORM_Q); base < n;
        base += (uint64_t)gridDim.x * (NT * 4 * NORM_Q)) {
+    auto one = [&](uint64_t t, float x) {
+      const double v = ((double)x - m) * inv;
+      if (DT == MDSM_F32) o32[t] = (float)v;
+      else if (DT == MDSM_F16) o16[t] = f16(v);
+      else o8[t] = quant_u8(v);
+    };
+    if constexpr (!WIDE) {
+      float x[4 * NORM_Q];
+#pragma unroll
+      for (int k = 0; k < 4 * NORM_Q; ++k) {
+        const uint64_t t = base + (uint64_t)(k * NT + threadIdx.x);
+        if (t < n) x[k] = row[t];
+      }
+#pragma unroll
+      for (int k = 0; k < 4 * NORM_Q; ++k) {
+        const uint64_t t = base + (uint64_t)(k * NT + threadIdx.x);
+        if (t < n) one(t, x[k]);
+      }
+      continue;
+    }
     float4u x[NORM_Q];
 #pragma unroll
     for (int k = 0; k < NORM_Q; ++k) {
@@ -155,7 +176,7 @@ __global__ __launch_bounds__(NT) void normalise_kernel(const float *__restrict__
 #pragma unroll
     for (int k = 0; k < NORM_Q; ++k) {
       const uint64_t t = base + (uint64_t)(k * NT + threadIdx.x) * 4u;
-      if (WIDE && t + 4u <= n) {
+      if (t + 4u <= n) {
         double v[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = ((double)x[k][e] - m) * inv;
@@ -167,12 +188,7 @@ __global__ __launch_bounds__(NT) void normalise_kernel(const float *__restrict__
           *reinterpret_cast<uint32_t *>(o8 + t) = (uint32_t)quant_u8(v[0]) | (uint32_t)quant_u8(v[1]) << 8 |
                                                   (uint32_t)quant_u8(v[2]) << 16 | (uint32_t)quant_u8(v[3]) << 24;
       } else {
-        for (uint64_t e = t; e < n && e < t + 4u; ++e) {
-          const double v = ((double)row[e] - m) * inv;
-          if (DT == MDSM_F32) o32[e] = (float)v;
-          else if (DT == MDSM_F16) o16[e] = f16(v);
-          else o8[e] = quant_u8(v);
-        }
+        for (uint64_t e = t; e < n && e < t + 4u; ++e) one(e, row[e]);
       }
     }
   }
