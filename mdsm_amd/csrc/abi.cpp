@@ -313,7 +313,7 @@ static int plan_shape(const mdsm_plan_s *p) {
   if (!variant_fits(p, v)) return v;  // refused there
   std::vector<bool> fits(p->row_words.size());
   for (int i = 1; i < (int)fits.size(); ++i) fits[i] = variant_fits(p, i);
-  return untuned_shape(p->dtype, v, fits, p->s.ndms, p->s.nsamp);
+  return untuned_shape(p->dtype, v, fits, p->s.nchans, p->s.ndms, p->s.nsamp);
 }
 
 extern "C" int mdsm_plan_create(const mdsm_survey_t *s, int in_dtype, mdsm_plan *plan) {

@@ -1908,11 +1908,13 @@ __global__ __launch_bounds__(256) void dedisp_direct_kernel(const void *__restri
   typedef int32_t i32x16 __attribute__((ext_vector_type(16)));
   typedef __attribute__((address_space(4))) const i32x16 const_i32x16;
   const uint32_t lane = threadIdx.x & 63u;
-  // XCD x (workgroup IDs are dealt round-robin) takes time blocks x (mod 8),
-  // each with all its trials one after the other: their rows stay in its L2
-  const uint32_t ndg = (ndms + 3u) / 4u, k = blockIdx.x >> 3;
-  const uint32_t tb = (k / ndg) * 8u + (blockIdx.x & 7u);
-  const uint32_t d = uniform((k % ndg) * 4u + (threadIdx.x >> 6));
+  // the pairs (time block, four trials) in that order, an eighth of them to
+  // each XCD (workgroup IDs are dealt round-robin): its time blocks run through
+  // all their trials one after the other, whose rows stay in its L2, and however
+  // few time blocks there are, no XCD idles
+  const uint32_t ndg = (ndms + 3u) / 4u, item = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  const uint32_t tb = item / ndg;
+  const uint32_t d = uniform((item - tb * ndg) * 4u + (threadIdx.x >> 6));
   if (d >= ndms || tb * 256u >= nsamp) return;
   const uint32_t t = min((tb * 64u + lane) * 4u, nsamp - 4u);
   constexpr uint32_t SZ = MODE == MDSM_F32 ? 4u : (MODE == MDSM_U8 ? 1u : 2u);
@@ -1982,6 +1984,13 @@ __global__ __launch_bounds__(256) void direct_table_kernel(const int32_t *__rest
   dtab[(uint64_t)d * cpad + c] = table[(uint64_t)min(c, nchans - 1u) * ndms + d];
 }
 inline uint32_t direct_pad(uint32_t nchans) { return (nchans + 15u) & ~15u; }
+// Workgroups: 256 samples of four trials each, a multiple of 8 of them.
+inline uint64_t direct_grid(uint32_t ndms, uint32_t nsamp) {
+  const uint64_t items = (((uint64_t)nsamp + 255u) / 256u) * (((uint64_t)ndms + 3u) / 4u);
+  return (items + 7u) / 8u * 8u;
+}
+// Rows of four samples or more (a lane's), whose grid IDs have 31 bits.
+inline bool direct_takes(uint32_t ndms, uint32_t nsamp) { return nsamp >= 4u && direct_grid(ndms, nsamp) < (1ull << 31); }
 
 // ------------------------------------------------------------ variant table
 // Variant v: F32 tile (MW, K, CB) and packed tiles (MW, K2, CB) with the same
@@ -2210,29 +2219,36 @@ double tile_rounds(int dtype, int shape, double tiles, bool equal) {
   return rounds * slots * sh.td() * sh.tt() / rate;
 }
 
-// The shape an untuned plan launches for its tile variant `nominal`.
-//   Direct kernel: a window tile walks all channels at 0.48 to 0.54 us per
-//   channel however few tiles there are, the direct kernel adds 7.5 (F32), 6
-//   (F16, pair sums) or 10.5 T/s (U8), which meets that at 2.2 to 4.3 million
-//   outputs (256 channels x 64 trials x 8192 samples F32: 19 against 132 us;
-//   512 x 256 x 12000: 205 against 257; x 16384: 274 against 257).
+// The shape an untuned plan launches for its tile variant `nominal`: the least
+// estimate.
+//   Direct kernel: 7.5 (F32), 6 (F16), 10.5 (U8) or 5.5 T adds/s (pair sums)
+//   over rows padded to 256 samples, 4 us to start and 0.6 us per million
+//   outputs stored; tiles 9 us to start and what their rounds take, 0.4 us per
+//   channel at least however few there are (256 channels x 64 trials x 8192
+//   samples F32: 19 against 132 us; 512 x 256 x 12000: 205 against 257; x 16384:
+//   274 against 257; 646 x 890 x 22 F16: 31 against 300).
 //   Eight waves instead of 16, or a shape that pads the trials less: by the
 //   tiles' rounds (46 trials x 218486 samples x 295 channels F16_PAIRS, delay
 //   differences for 40 trials: 264 us in two such tiles, 205 in one of 48; 32 trials x 600000 samples x 512
 //   channels F32: 399 against 598 us; 856 channels x 1222 trials x 15994
 //   samples U8, 260 tiles of 16 waves: 540 against 766 us).
 // `fits` holds the shapes that take the survey.
-int untuned_shape(int dtype, int nominal, const std::vector<bool> &fits, uint32_t ndms, uint32_t nsamp) {
-  const uint64_t direct_outputs = dtype == MDSM_F32 ? 3100000u : dtype == MDSM_F16 ? 2500000u
-                                  : dtype == MDSM_U8 ? 4300000u : 2200000u;
-  if (nsamp >= 256u && (uint64_t)ndms * nsamp <= direct_outputs) return kDirectShape;
+int untuned_shape(int dtype, int nominal, const std::vector<bool> &fits, uint32_t nchans, uint32_t ndms,
+                  uint32_t nsamp) {
+  // us per channel
   auto cost = [&](int shape) {
     const TileShape sh = variant_shape(dtype, shape);
-    return tile_rounds(dtype, shape, ((double)((ndms + sh.td() - 1) / sh.td())) * ((nsamp + sh.tt() - 1) / sh.tt()), true);
+    return 1e-6 * tile_rounds(dtype, shape, ((double)((ndms + sh.td() - 1) / sh.td())) * ((nsamp + sh.tt() - 1) / sh.tt()), true);
   };
   int best = nominal;
   for (int n = 0, shape; (shape = other_shape(dtype, nominal, n)) != 0; ++n)
     if (fits[shape] && cost(shape) < cost(best)) best = shape;
+  if (direct_takes(ndms, nsamp)) {
+    const double rate = dtype == MDSM_F32 ? 7.5 : dtype == MDSM_F16 ? 6.0 : dtype == MDSM_U8 ? 10.5 : 5.5;
+    const double padded = (double)ndms * ((nsamp + 255u) / 256u * 256u);
+    const double direct = 4.0 + 0.6e-6 * ((double)ndms * nsamp) + 1e-6 * nchans * padded / rate;
+    if (direct < 9.0 + nchans * std::max(0.4, cost(best))) return kDirectShape;
+  }
   return best;
 }
 
@@ -2359,7 +2375,8 @@ int launch_dedisperse(int dtype, int variant, const void *in, uint64_t ld, const
                       uint32_t rw, float *out, hipStream_t s) {
   if (variant == kDirectShape) {
     MDSM_REQUIRE(reltab, MDSM_ERR_STATE, "delay table missing");
-    const dim3 grid(((nsamp + 255u) / 256u + 7u) / 8u * 8u * ((ndms + 3u) / 4u));
+    MDSM_REQUIRE(direct_takes(ndms, nsamp), MDSM_ERR_ARG, "rows too short or too many for the kernel without tiles");
+    const dim3 grid((uint32_t)direct_grid(ndms, nsamp));
     const uint32_t cpad = direct_pad(nchans);
     switch (dtype) {
       case MDSM_F32: hipLaunchKernelGGL(dedisp_direct_kernel<MDSM_F32>, grid, dim3(256), 0, s, in, ld, reltab, nchans, cpad, nsamp, ndms, out); break;

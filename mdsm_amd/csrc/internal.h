@@ -89,7 +89,8 @@ int narrow_variant(int dtype, int variant);
 int other_shape(int dtype, int nominal, int n);
 double tile_rounds(int dtype, int shape, double tiles, bool equal);
 // The shape an untuned plan launches where its tile variant is `nominal`.
-int untuned_shape(int dtype, int nominal, const std::vector<bool> &fits, uint32_t ndms, uint32_t nsamp);
+int untuned_shape(int dtype, int nominal, const std::vector<bool> &fits, uint32_t nchans, uint32_t ndms,
+                  uint32_t nsamp);
 // Channels staged per LDS block for a tile variant and row width (0: does not fit).
 uint32_t stage_channels(int dtype, int variant, uint32_t row_words);
 // Words of a variant's trial-offset table, and the kernel that fills it
