@@ -120,8 +120,8 @@ static int batch_variant(const mdsm_batch_s *b) {
 }
 
 // The shape a launch uses: the variant that was set or tuned, or the default
-// or one of its smaller forms by the rounds of all beams' tiles (as
-// untuned_shape).
+// or one of its alternatives, whichever has the least estimate for all beams'
+// tiles (as untuned_shape).
 static int batch_shape(const mdsm_batch_s *b) {
   const int v = batch_variant(b);
   if (b->variant) {
@@ -130,17 +130,18 @@ static int batch_shape(const mdsm_batch_s *b) {
   }
   auto cost = [&](int shape) {
     const TileShape sh = variant_shape(b->dtype, shape);
-    double tiles = 0.0, work = 0.0;
+    double tiles = 0.0, work = 0.0, outputs = 0.0;
     for (const auto &s : b->beams) {
       const double n = (double)((s.nsamp + sh.tt() - 1) / sh.tt()) * ((s.ndms + sh.td() - 1) / sh.td());
       tiles += n;
       work += n * s.nchans;
+      outputs += (double)s.ndms * s.nsamp;
     }
-    return tile_rounds(b->dtype, shape, tiles, b->beams.size() == 1) * (work / tiles);
+    return launch_estimate(b->dtype, shape, tiles, b->beams.size() == 1, work / tiles, outputs);
   };
   int best = v;
   for (int n = 0, shape; (shape = other_shape(b->dtype, v, n)) != 0; ++n)
-    if (batch_fits(b, shape) && cost(shape) < cost(best)) best = shape;
+    if (batch_fits(b, shape) && (b->dtype != MDSM_F16 || shape != 15) && cost(shape) < cost(best)) best = shape;
   return best;
 }
 

@@ -2173,8 +2173,8 @@ int narrow_variant(int dtype, int variant) {
   }
 }
 
-// The shapes that may replace a default one where its tiles pad too much (n =
-// 0, 1, ..; 0: no more): those of smaller or, after 20 and 21, fewer tiles.
+// The shapes that may replace a default one where its tiles pad too much or
+// its workgroups wait for their stores (n = 0, 1, ..; 0: no more).
 int other_shape(int dtype, int nominal, int n) {
   const int nv = num_variants(dtype);
   if (dtype == MDSM_U8) {
@@ -2186,68 +2186,98 @@ int other_shape(int dtype, int nominal, int n) {
     if (nominal == 22) return after22[n];
     return nominal == 20 ? after20[n] : (nominal == 21 ? after20[n + 1] : (nominal == 16 ? after20[n + 2] : 0));
   }
-  return n == 0 && nominal == 12 ? nv + 1 : 0;
+  if (nominal != 12) return 0;
+  return n == 0 ? nv + 1 : (n == 1 ? (dtype == MDSM_F32 ? 8 : 15) : 0);
 }
 
-// Estimated time of a launch's tiles, for the shapes that untuned launches
-// choose between: every CU runs one (16 waves) or two workgroups of a shape at
-// a time, so tiles take whole rounds of 256 or 512, each at the shape's full
-// rate; a last round of up to 256 of two per CU, three quarters of one.  Tiles of
-// several beams (not equal) end at different times: half a round over the
-// mean instead.  T adds/s measured at 512 to 1024 channels, 1920 trials x 81920 samples; eight
-// waves per workgroup 1.04 to 1.36 times as long per add.
-double tile_rounds(int dtype, int shape, double tiles, bool equal) {
+// Estimated time (us) of a launch of `tiles` tiles over nchans channels, for
+// the shapes that untuned launches choose between: the rounds of adds, and what
+// goes on beside them.
+//   Adds: every CU runs one (16 waves) or two workgroups of a shape at a time,
+//   so tiles take whole rounds of 256 or 512, each at the shape's full rate; a
+//   last round of up to 256 of two per CU, three quarters of one.  Tiles of
+//   several beams (not equal) end at different times: half a round over the
+//   mean instead.  T adds/s measured at 512 to 1024 channels, 1920 trials x
+//   81920 samples; eight waves per workgroup 1.04 to 1.36 times as long per add,
+//   and 0.87 of all that where rows come from the caches (12 to 96 channels);
+//   0.4 us per channel at least however few tiles there are.  The word-per-add
+//   shapes fit no rounds: 16 (F32) or 25 T adds/s, 0.6 or 0.5 us at least.
+//   Beside them: a window tile's workgroups fill their CUs alone, so nothing
+//   adds while they store: 0.7 us per million outputs, 6 at least, against 0.47
+//   (4) of the pair-sum shapes and 0.5 (3.5) of the word-per-add ones.  At few
+//   channels that decides: 64 channels x 4000 trials x 50000 samples 388 us in
+//   shape 20 against 427 in 22 (F16_PAIRS), 393 in 21 against 426 (U8); 96
+//   channels 548 against 559 and 546 against 555.
+double launch_estimate(int dtype, int shape, double tiles, bool equal, double nchans, double outputs) {
   const int nv = num_variants(dtype);
-  const bool pair_windows = shape == 22 || (shape == nv + 1 && (dtype == MDSM_U8 || dtype == MDSM_F16_PAIRS));
-  const double wide = dtype == MDSM_F32 ? 39.0 : (pair_windows ? 42.0 : (dtype == MDSM_U8 ? 34.5 : 36.5));
-  double rate, slots = 512.0;
-  if (shape > nv) {
-    rate = wide / (pair_windows ? 1.36 : (dtype == MDSM_F32 ? 1.17 : 1.04));
-  } else if (shape == 20 || shape == 21 || shape == 16) {
-    rate = dtype == MDSM_U8 ? 36.5 : (shape == 20 ? 37.5 : (shape == 21 ? 33.0 : 31.0));
-  } else if (dtype == MDSM_F16_PAIRS && shape == 15) {
-    rate = 25.0;  // bound by LDS reads, few of its workgroups fill a CU
-    slots = 256.0;
-  } else {
-    rate = wide;
-    slots = 256.0;
-  }
   const TileShape sh = variant_shape(dtype, shape);
-  double rounds = ceil(tiles / slots);
-  if (slots > 256.0 && tiles <= slots * rounds - 256.0) rounds -= 0.25;
-  if (!equal && rounds > 1.0) rounds = tiles / slots + 0.5;
-  return rounds * slots * sh.td() * sh.tt() / rate;
+  const double work = (double)sh.td() * sh.tt();
+  const bool word = (dtype == MDSM_F32 && shape == 8) || (dtype == MDSM_F16 && shape == 15) ||
+                    (dtype == MDSM_F16_PAIRS && shape == 15);
+  const bool pair_sums = (dtype == MDSM_U8 || dtype == MDSM_F16_PAIRS) && shape >= 16 && shape <= 21;
+  double per_channel;
+  if (word) {
+    per_channel = dtype == MDSM_F32 ? std::max(0.6, 1e-6 * tiles * work / 16.0)
+                                    : std::max(0.5, 1e-6 * tiles * work / 25.0);
+  } else {
+    const bool pair_windows = shape == 22 || (shape == nv + 1 && (dtype == MDSM_U8 || dtype == MDSM_F16_PAIRS));
+    const double wide = dtype == MDSM_F32 ? 39.0 : (pair_windows ? 42.0 : (dtype == MDSM_U8 ? 34.5 : 36.5));
+    double rate = wide, slots = 256.0;
+    if (shape > nv) {
+      rate = wide / (pair_windows ? 1.36 : (dtype == MDSM_F32 ? 1.17 : 1.04));
+      slots = 512.0;
+    } else if (pair_sums) {
+      rate = dtype == MDSM_U8 ? 36.5 : (shape == 20 ? 37.5 : (shape == 21 ? 33.0 : 31.0));
+      slots = 512.0;
+    }
+    double rounds = ceil(tiles / slots);
+    if (slots > 256.0 && tiles <= slots * rounds - 256.0) rounds -= 0.25;
+    if (!equal && rounds > 1.0) rounds = tiles / slots + 0.5;
+    per_channel = std::max(0.4, 0.87e-6 * rounds * slots * work / rate);
+  }
+  const double start = word ? 3.5 : (pair_sums ? 4.0 : 6.0), store = word ? 0.5 : (pair_sums ? 0.47 : 0.7);
+  return 3.0 + std::max(start, store * 1e-6 * outputs) + nchans * per_channel;
 }
 
 // The shape an untuned plan launches for its tile variant `nominal`: the least
 // estimate.
-//   Direct kernel: 7.5 (F32), 6 (F16), 10.5 (U8) or 5.5 T adds/s (pair sums)
-//   over rows padded to 256 samples, 4 us to start and 0.6 us per million
-//   outputs stored; tiles 9 us to start and what their rounds take, 0.4 us per
-//   channel at least however few there are (256 channels x 64 trials x 8192
-//   samples F32: 19 against 132 us; 512 x 256 x 12000: 205 against 257; x 16384:
-//   274 against 257; 646 x 890 x 22 F16: 31 against 300).
-//   Eight waves instead of 16, or a shape that pads the trials less: by the
-//   tiles' rounds (46 trials x 218486 samples x 295 channels F16_PAIRS, delay
-//   differences for 40 trials: 264 us in two such tiles, 205 in one of 48; 32 trials x 600000 samples x 512
+//   Eight waves instead of 16, or a shape that pads the trials less (46 trials x
+//   218486 samples x 295 channels F16_PAIRS, delay differences for 40 trials:
+//   264 us in two such tiles, 205 in one of 48; 32 trials x 600000 samples x 512
 //   channels F32: 399 against 598 us; 856 channels x 1222 trials x 15994
 //   samples U8, 260 tiles of 16 waves: 540 against 766 us).
+//   F16's shape 15 where fewer than 40 channels meet fewer than 128 window tiles,
+//   which leave half of the CUs idle, and is not weighed otherwise (16 channels x
+//   200 trials x 20000 samples: 13 us against 16).
+//   Direct kernel, up to 5.3 million outputs of rows padded to 256 samples: 7.5
+//   (F32), 6 (F16), 11.5 (U8) or 5.5 T adds/s (pair sums), 4 us to start and 0.8
+//   us per million outputs stored (256 channels x 64 trials x 8192 samples F32:
+//   19 against 132 us; 512 x 256 x 12000: 205 against 257; x 16384: 274 against
+//   257; 646 x 890 x 22 F16: 31 against 300).  More outputs of few trials read
+//   their rows from HBM for every four of them (421 channels x 6 trials x 10^6
+//   samples F16_PAIRS: 621 us against 540).
 // `fits` holds the shapes that take the survey.
 int untuned_shape(int dtype, int nominal, const std::vector<bool> &fits, uint32_t nchans, uint32_t ndms,
                   uint32_t nsamp) {
-  // us per channel
-  auto cost = [&](int shape) {
+  const double outputs = (double)ndms * nsamp;
+  auto tiles = [&](int shape) {
     const TileShape sh = variant_shape(dtype, shape);
-    return 1e-6 * tile_rounds(dtype, shape, ((double)((ndms + sh.td() - 1) / sh.td())) * ((nsamp + sh.tt() - 1) / sh.tt()), true);
+    return ((double)((ndms + sh.td() - 1) / sh.td())) * ((nsamp + sh.tt() - 1) / sh.tt());
   };
+  auto cost = [&](int shape) { return launch_estimate(dtype, shape, tiles(shape), true, nchans, outputs); };
   int best = nominal;
-  for (int n = 0, shape; (shape = other_shape(dtype, nominal, n)) != 0; ++n)
-    if (fits[shape] && cost(shape) < cost(best)) best = shape;
-  if (direct_takes(ndms, nsamp)) {
-    const double rate = dtype == MDSM_F32 ? 7.5 : dtype == MDSM_F16 ? 6.0 : dtype == MDSM_U8 ? 10.5 : 5.5;
-    const double padded = (double)ndms * ((nsamp + 255u) / 256u * 256u);
-    const double direct = 4.0 + 0.6e-6 * ((double)ndms * nsamp) + 1e-6 * nchans * padded / rate;
-    if (direct < 9.0 + nchans * std::max(0.4, cost(best))) return kDirectShape;
+  for (int n = 0, shape; (shape = other_shape(dtype, nominal, n)) != 0; ++n) {
+    if (!fits[shape]) continue;
+    if (dtype == MDSM_F16 && shape == 15) {
+      if (nchans < 40u && tiles(nominal) < 128.0) best = shape;
+    } else if (cost(shape) < cost(best)) {
+      best = shape;
+    }
+  }
+  const double padded = (double)ndms * ((nsamp + 255u) / 256u * 256u);
+  if (direct_takes(ndms, nsamp) && padded <= 5.3e6) {
+    const double rate = dtype == MDSM_F32 ? 7.5 : dtype == MDSM_F16 ? 6.0 : dtype == MDSM_U8 ? 11.5 : 5.5;
+    if (4.0 + 0.8e-6 * outputs + 1e-6 * nchans * padded / rate < cost(best)) return kDirectShape;
   }
   return best;
 }

@@ -84,10 +84,10 @@ int fallback_variant(int dtype, int n);
 constexpr int kDirectShape = 0;
 int num_shapes(int dtype);
 int narrow_variant(int dtype, int variant);
-// Shapes that may replace a default one, and the estimated time of
-// a number of tiles of one of these.
+// Shapes that may replace a default one, and the estimated time of a launch of
+// one of these (us).
 int other_shape(int dtype, int nominal, int n);
-double tile_rounds(int dtype, int shape, double tiles, bool equal);
+double launch_estimate(int dtype, int shape, double tiles, bool equal, double nchans, double outputs);
 // The shape an untuned plan launches where its tile variant is `nominal`.
 int untuned_shape(int dtype, int nominal, const std::vector<bool> &fits, uint32_t nchans, uint32_t ndms,
                   uint32_t nsamp);
