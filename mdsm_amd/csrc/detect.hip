@@ -78,6 +78,28 @@ __device__ __forceinline__ void chain_sums(const float *__restrict__ row, uint64
   a = 0.0;
   q = 0.0;
   uint64_t j = threadIdx.x;
+  // one or two elements per lane: no loops to set up (2^20 samples in blocks of
+  // 16 36 us, 39 through the loops; in blocks of 257 4.4 and 4.7)
+  if (n <= NT) {
+    if (j < n) {
+      const double d = (double)row[j];
+      a = a + d;
+      q = q + d * d;
+    }
+    return;
+  }
+  if (n <= 2u * NT) {
+    const float v0 = row[j], v1 = j + NT < n ? row[j + NT] : 0.0f;
+    const double d0 = (double)v0;
+    a = a + d0;
+    q = q + d0 * d0;
+    if (j + NT < n) {
+      const double d = (double)v1;
+      a = a + d;
+      q = q + d * d;
+    }
+    return;
+  }
   for (; j + (U - 1) * NT < n; j += U * NT) {
     float v[U];
 #pragma unroll
