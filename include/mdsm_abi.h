@@ -133,9 +133,9 @@ int mdsm_plan_device_table(mdsm_plan plan, const int32_t **table);
  * or exact u16) once per delay difference of its two channels; those take
  * a survey only when that
  * difference is >= 0 and spans at most 3 values (19: 4) in every DM tile of
- * the shape (22: or of its half-width form), and a shape that does not take
- * the survey makes mdsm_dedisperse fail with MDSM_ERR_ARG (the autotuners skip it).  Every
- * shape of a storage type gives the same results.  Setting a variant builds
+ * the shape (22: 64, 32 or 40 trials, 21: 40 or 48), and a number none of whose
+ * shapes takes the survey makes mdsm_dedisperse fail with MDSM_ERR_ARG (the
+ * autotuners skip it).  Every shape of a storage type gives the same results.  Setting a variant builds
  * its trial-offset table (one allocation and one kernel, synchronous); a
  * variant first used by mdsm_dedisperse without being set builds it there,
  * once. */

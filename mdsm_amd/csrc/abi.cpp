@@ -302,17 +302,14 @@ static int default_variant(const mdsm_plan_s *p) {
 
 static int plan_variant(const mdsm_plan_s *p) { return p->variant ? p->variant : default_variant(p); }
 
-// What a dedisperse call launches: the variant that was set or tuned, or the
-// form of the default variant that suits the survey's size.
-static int plan_shape(const mdsm_plan_s *p) {
-  if (p->variant) {
-    const int narrow = variant_fits(p, p->variant) ? 0 : narrow_variant(p->dtype, p->variant);
-    return narrow && variant_fits(p, narrow) ? narrow : p->variant;
-  }
-  const int v = default_variant(p);
-  if (!variant_fits(p, v)) return v;  // refused there
+// What a dedisperse call launches: the variant that was set or tuned where it
+// takes the survey, or the shape that suits the survey's size.
+static int plan_shape(const mdsm_plan_s *p, int variant) {
   std::vector<bool> fits(p->row_words.size());
   for (int i = 1; i < (int)fits.size(); ++i) fits[i] = variant_fits(p, i);
+  if (variant) return numbered_shape(p->dtype, variant, fits);
+  const int v = default_variant(p);
+  if (!fits[v]) return v;  // refused there
   return untuned_shape(p->dtype, v, fits, p->s.nchans, p->s.ndms, p->s.nsamp);
 }
 
@@ -395,7 +392,7 @@ extern "C" int mdsm_plan_set_variant(mdsm_plan plan, int variant) {
   plan->variant = variant;
   // build the variant's trial-offset table now, so that dedisperse calls
   // (and graphs captured from them) allocate nothing
-  const int v = plan_shape(plan);
+  const int v = plan_shape(plan, variant);
   if (v == kDirectShape || variant_fits(plan, v)) {
     const int rc = ensure_trial_offsets(plan, v, nullptr);
     if (rc != MDSM_OK) return rc;
@@ -415,8 +412,7 @@ extern "C" int mdsm_plan_variant_channels(mdsm_plan plan, int variant, uint32_t 
   MDSM_REQUIRE(plan && channels, MDSM_ERR_ARG, "null argument");
   MDSM_REQUIRE(variant >= 1 && variant <= num_variants(plan->dtype), MDSM_ERR_ARG,
                "variant %d out of range", variant);
-  int v = variant;
-  if (!variant_fits(plan, v) && narrow_variant(plan->dtype, v)) v = narrow_variant(plan->dtype, v);
+  const int v = plan_shape(plan, variant);
   *channels = variant_fits(plan, v) ? stage_channels(plan->dtype, v, plan->row_words[v]) : 0u;
   return MDSM_OK;
 }
@@ -438,7 +434,7 @@ extern "C" int mdsm_dedisperse(mdsm_plan plan, const void *d_in, uint64_t ld, fl
                input_alignment(plan->dtype));
   MDSM_REQUIRE(ld / input_alignment(plan->dtype) < (1ull << 29), MDSM_ERR_ARG,
                "input rows must be shorter than 2 GiB");
-  const int v = plan_shape(plan);
+  const int v = plan_shape(plan, plan->variant);
   const int rc = ensure_trial_offsets(plan, v, as_stream(stream));
   if (rc != MDSM_OK) return rc;
   return launch_dedisperse(plan->dtype, v, d_in, ld, plan->d_table, plan->d_rel[v], plan->s.nchans,
@@ -460,7 +456,7 @@ int plan_time_variants(mdsm_plan plan, const void *d_in, uint64_t ld, float *d_o
   t.assign(nv + 1, -1.0f);
   for (int v = 0; v <= nv; ++v) {
     plan->variant = v;
-    if (v == 0 && plan_shape(plan) == plan_variant(plan)) continue;  // timed by its number
+    if (v == 0 && plan_shape(plan, 0) == plan_variant(plan)) continue;  // timed by its number
     if (mdsm_dedisperse(plan, d_in, ld, d_out, s) != MDSM_OK) continue;  // warm-up / LDS fit
     float vms = -1.0f;
     for (int rep = 0; rep < 3; ++rep) {

@@ -107,8 +107,7 @@ static bool batch_fits(const mdsm_batch_s *b, int v) {
 
 // Untuned default: the preferred tile shape when it fits every beam, else the
 // storage type's fallback shape, else the first shape that does.
-static int batch_variant(const mdsm_batch_s *b) {
-  if (b->variant) return b->variant;
+static int batch_default(const mdsm_batch_s *b) {
   auto fits = [&](int v) { return batch_fits(b, v); };
   const int pref = preferred_variant(b->dtype);
   if (fits(pref)) return pref;
@@ -119,29 +118,29 @@ static int batch_variant(const mdsm_batch_s *b) {
   return pref;
 }
 
-// The shape a launch uses: the variant that was set or tuned, or the default
-// or one of its alternatives, whichever has the least estimate for all beams'
-// tiles (as untuned_shape).
-static int batch_shape(const mdsm_batch_s *b) {
-  const int v = batch_variant(b);
-  if (b->variant) {
-    const int narrow = batch_fits(b, v) ? 0 : narrow_variant(b->dtype, v);
-    return narrow && batch_fits(b, narrow) ? narrow : v;
-  }
+static int batch_variant(const mdsm_batch_s *b) { return b->variant ? b->variant : batch_default(b); }
+
+// The shape a launch uses: the variant that was set or tuned where it takes the
+// beams, or the default or one of its alternatives, whichever has the least
+// estimate for all beams' tiles (as untuned_shape).
+static int batch_shape(const mdsm_batch_s *b, int variant) {
   auto cost = [&](int shape) {
-    const TileShape sh = variant_shape(b->dtype, shape);
     double tiles = 0.0, work = 0.0, outputs = 0.0;
     for (const auto &s : b->beams) {
-      const double n = (double)((s.nsamp + sh.tt() - 1) / sh.tt()) * ((s.ndms + sh.td() - 1) / sh.td());
+      const double n = tile_count(b->dtype, shape, s.ndms, s.nsamp);
       tiles += n;
       work += n * s.nchans;
       outputs += (double)s.ndms * s.nsamp;
     }
     return launch_estimate(b->dtype, shape, tiles, b->beams.size() == 1, work / tiles, outputs);
   };
+  std::vector<bool> fits(num_shapes(b->dtype) + 1);
+  for (int i = 1; i < (int)fits.size(); ++i) fits[i] = batch_fits(b, i);
+  if (variant) return numbered_shape(b->dtype, variant, fits);
+  const int v = batch_default(b);
   int best = v;
   for (int n = 0, shape; (shape = other_shape(b->dtype, v, n)) != 0; ++n)
-    if (batch_fits(b, shape) && (b->dtype != MDSM_F16 || shape != 15) && cost(shape) < cost(best)) best = shape;
+    if (fits[shape] && (b->dtype != MDSM_F16 || shape != 15) && cost(shape) < cost(best)) best = shape;
   return best;
 }
 
@@ -328,7 +327,7 @@ extern "C" int mdsm_batch_bind(mdsm_batch batch, const void *const *d_in, const 
                                float *const *d_out) {
   MDSM_REQUIRE(batch && d_in && ld && d_out, MDSM_ERR_ARG, "null argument");
   const uint32_t nb = (uint32_t)batch->beams.size();
-  const int v = batch_shape(batch);
+  const int v = batch_shape(batch, batch->variant);
   const TileShape sh = variant_shape(batch->dtype, v);
   batch->h_desc.resize(nb);
   uint64_t items = 0;

@@ -2173,6 +2173,22 @@ int narrow_variant(int dtype, int variant) {
   }
 }
 
+// What took a number's surveys before the register windows had it: a survey that
+// neither of their forms takes runs there (F32: shape 1's smaller tiles; 22: 40
+// trials, 21: 48 trials of pair sums).
+static int stand_in(int dtype, int variant) {
+  if (dtype == MDSM_F32) return variant == 12 ? 1 : 0;
+  if (dtype == MDSM_U8 || dtype == MDSM_F16_PAIRS) return variant == 22 ? 21 : (variant == 21 ? 20 : 0);
+  return 0;
+}
+
+int numbered_shape(int dtype, int variant, const std::vector<bool> &fits) {
+  if (fits[variant]) return variant;
+  for (const int other : {narrow_variant(dtype, variant), stand_in(dtype, variant)})
+    if (other && fits[other]) return other;
+  return variant;
+}
+
 // The shapes that may replace a default one where its tiles pad too much or
 // its workgroups wait for their stores (n = 0, 1, ..; 0: no more).
 int other_shape(int dtype, int nominal, int n) {
@@ -2188,6 +2204,11 @@ int other_shape(int dtype, int nominal, int n) {
   }
   if (nominal != 12) return 0;
   return n == 0 ? nv + 1 : (n == 1 ? (dtype == MDSM_F32 ? 8 : 15) : 0);
+}
+
+double tile_count(int dtype, int shape, uint32_t ndms, uint32_t nsamp) {
+  const TileShape sh = variant_shape(dtype, shape);
+  return (double)((ndms + sh.td() - 1) / sh.td()) * ((nsamp + sh.tt() - 1) / sh.tt());
 }
 
 // Estimated time (us) of a launch of `tiles` tiles over nchans channels, for
@@ -2260,10 +2281,7 @@ double launch_estimate(int dtype, int shape, double tiles, bool equal, double nc
 int untuned_shape(int dtype, int nominal, const std::vector<bool> &fits, uint32_t nchans, uint32_t ndms,
                   uint32_t nsamp) {
   const double outputs = (double)ndms * nsamp;
-  auto tiles = [&](int shape) {
-    const TileShape sh = variant_shape(dtype, shape);
-    return ((double)((ndms + sh.td() - 1) / sh.td())) * ((nsamp + sh.tt() - 1) / sh.tt());
-  };
+  auto tiles = [&](int shape) { return tile_count(dtype, shape, ndms, nsamp); };
   auto cost = [&](int shape) { return launch_estimate(dtype, shape, tiles(shape), true, nchans, outputs); };
   int best = nominal;
   for (int n = 0, shape; (shape = other_shape(dtype, nominal, n)) != 0; ++n) {

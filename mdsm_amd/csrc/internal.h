@@ -76,17 +76,23 @@ int preferred_variant(int dtype);
 // The shapes an untuned plan tries, n = 0, 1, .. (0: no more), when the
 // preferred one does not take the survey; after them the first one that does.
 int fallback_variant(int dtype, int n);
-// Launch shapes: the public tile variants 1..num_variants, two more that
-// untuned plans and batches choose by size (narrow_variant: the eight-wave form
-// of a 16-wave variant, 0 if it has none; its DM tiles of half the trials also
-// take surveys that a variant set by number cannot stage), and kDirectShape, the kernel
-// without tiles for few outputs (its table is the transposed delay table).
+// Launch shapes: the public tile variants 1..num_variants; the eight-wave forms
+// that the numbers of the 16-wave register windows stand for too
+// (narrow_variant, 0: none); and kDirectShape, the kernel without tiles for few
+// outputs, which only untuned plans launch (its table is the transposed delay
+// table).
 constexpr int kDirectShape = 0;
 int num_shapes(int dtype);
 int narrow_variant(int dtype, int variant);
-// Shapes that may replace a default one, and the estimated time of a launch of
-// one of these (us).
+// What a variant set by number launches: its shape, the eight-wave form, or a
+// shape that takes every survey which the number took before it, the first
+// that takes the survey (`fits`, by shape); else the variant itself, which is
+// refused.
+int numbered_shape(int dtype, int variant, const std::vector<bool> &fits);
+// Shapes that may replace a default one, a shape's tiles for a survey, and the
+// estimated time of a launch of a number of them (us).
 int other_shape(int dtype, int nominal, int n);
+double tile_count(int dtype, int shape, uint32_t ndms, uint32_t nsamp);
 double launch_estimate(int dtype, int shape, double tiles, bool equal, double nchans, double outputs);
 // The shape an untuned plan launches where its tile variant is `nominal`.
 int untuned_shape(int dtype, int nominal, const std::vector<bool> &fits, uint32_t nchans, uint32_t ndms,
