@@ -135,10 +135,14 @@ int mdsm_plan_device_table(mdsm_plan plan, const int32_t **table);
  * difference is >= 0 and spans at most 3 values (19: 4) in every DM tile of
  * the shape (22: 64, 32 or 40 trials, 21: 40 or 48), and a number none of whose
  * shapes takes the survey makes mdsm_dedisperse fail with MDSM_ERR_ARG (the
- * autotuners skip it).  Every shape of a storage type gives the same results.  Setting a variant builds
+ * autotuners skip it).  Shapes 12 (MDSM_F32, MDSM_F16), 2 (MDSM_U8) and 22 come
+ * in DM tiles of 64 and of 32 trials and launch the form that suits the survey.
+ * Every shape of a storage type gives the same results.  Setting a variant builds
  * its trial-offset table (one allocation and one kernel, synchronous); a
  * variant first used by mdsm_dedisperse without being set builds it there,
- * once. */
+ * once.  mdsm_plan_get_variant returns the number that was set or tuned (0 after
+ * an autotune that kept the untuned launch), or the shape that a plan without
+ * one stands for. */
 int mdsm_plan_set_variant(mdsm_plan plan, int variant);
 int mdsm_plan_get_variant(mdsm_plan plan, int *variant);
 int mdsm_tile_variants(int in_dtype, int *count);
@@ -146,17 +150,19 @@ int mdsm_tile_variants(int in_dtype, int *count);
  * it when it takes the survey; otherwise MDSM_F16_PAIRS and MDSM_U8 fall
  * back through pair-sum shapes of fewer trials to shapes 15 and 2 (which take
  * every survey whose delay spread they can stage), and any type to the first
- * shape that can.  An untuned plan or batch may launch a smaller form of that
- * shape, or for few outputs a kernel without tiles, with the same results;
- * mdsm_plan_get_variant names the shape it stands for. */
+ * shape that can.  An untuned plan or batch may launch another shape that suits
+ * its sizes better, and a plan of few outputs a kernel without tiles, which has
+ * no number, with the same results. */
 int mdsm_tile_preferred(int in_dtype, int *variant);
 /* Channels a tile shape stages per LDS block for this plan's delay spread;
  * 0 when the shape cannot stage it. */
 int mdsm_plan_variant_channels(mdsm_plan plan, int variant, uint32_t *channels);
 /* Time each tile variant on the given buffers (best of three launches after
  * a warm-up) and keep the fastest; the storage type's default variant is
- * kept when it is within 2 % of the fastest, and the plan stays untuned when
- * what it launches then is faster than all of them. */
+ * kept when it is within 2 % of the fastest, and the plan stays untuned where
+ * the kernel without tiles is faster than all of them.  Setting *best_variant
+ * (0: the untuned launch) on a plan of the same survey launches what took
+ * *best_ms. */
 int mdsm_plan_autotune(mdsm_plan plan, const void *d_in, uint64_t ld, float *d_out, void *stream,
                        int *best_variant, float *best_ms);
 
@@ -353,10 +359,11 @@ int mdsm_batch_set_variant(mdsm_batch batch, int variant);
  * tile shape on every beam truncated to 2^16 samples (reading d_in[i], ld[i]
  * into a scratch output it allocates), each shape's batch time estimated as
  * the sum of its beams' times scaled to their full length; then the three
- * least estimates among the shapes that fit every beam are timed as one
- * whole launch each into d_out, and the fastest is kept (the next bind uses
- * it; the buffers are left unbound).  best_variant receives the batch's
- * variant afterwards, best_ms its launch time. */
+ * least estimates among the shapes that fit every beam, and the number of what
+ * the untuned batch launches, are timed as one whole launch each into d_out, and
+ * the fastest is kept (the next bind uses it; the buffers are left unbound).
+ * best_variant receives the batch's variant afterwards, best_ms its launch
+ * time. */
 int mdsm_batch_autotune(mdsm_batch batch, const void *const *d_in, const uint64_t *ld,
                         float *const *d_out, void *stream, int *best_variant, float *best_ms);
 /* Launch shape (takes effect at the next bind): FLAT (default) launches one

@@ -248,6 +248,7 @@ struct mdsm_plan_s {
   std::vector<int32_t> h_table;
   int32_t *d_table = nullptr;
   int variant = 0;  // 0 until set or tuned; then 1..num_variants
+  bool kept_untuned = false;  // tuned, and the untuned launch was the fastest
   std::vector<uint32_t> row_words;  // per variant (index 1..)
   std::vector<int32_t *> d_rel;     // trial-offset table per variant, built on first use
 };
@@ -302,15 +303,25 @@ static int default_variant(const mdsm_plan_s *p) {
 
 static int plan_variant(const mdsm_plan_s *p) { return p->variant ? p->variant : default_variant(p); }
 
-// What a dedisperse call launches: the variant that was set or tuned where it
-// takes the survey, or the shape that suits the survey's size.
-static int plan_shape(const mdsm_plan_s *p, int variant) {
+// What a dedisperse call launches: the form of the variant that was set or
+// tuned, or the shape, that suits the survey's size (*own: see numbered_shape).
+static int plan_shape(const mdsm_plan_s *p, int variant, bool *own) {
   std::vector<bool> fits(p->row_words.size());
   for (int i = 1; i < (int)fits.size(); ++i) fits[i] = variant_fits(p, i);
-  if (variant) return numbered_shape(p->dtype, variant, fits);
+  if (variant)
+    return numbered_shape(p->dtype, variant, fits, [&](int shape) {
+      return launch_estimate(p->dtype, shape, tile_count(p->dtype, shape, p->s.ndms, p->s.nsamp), true, p->s.nchans,
+                             p->s.nchans, (double)p->s.ndms * p->s.nsamp);
+    }, own);
+  *own = true;
   const int v = default_variant(p);
   if (!fits[v]) return v;  // refused there
   return untuned_shape(p->dtype, v, fits, p->s.nchans, p->s.ndms, p->s.nsamp);
+}
+
+static int plan_shape(const mdsm_plan_s *p, int variant) {
+  bool own;
+  return plan_shape(p, variant, &own);
 }
 
 extern "C" int mdsm_plan_create(const mdsm_survey_t *s, int in_dtype, mdsm_plan *plan) {
@@ -390,6 +401,7 @@ extern "C" int mdsm_plan_set_variant(mdsm_plan plan, int variant) {
   MDSM_REQUIRE(variant >= 0 && variant <= num_variants(plan->dtype), MDSM_ERR_ARG,
                "variant %d out of range", variant);
   plan->variant = variant;
+  plan->kept_untuned = false;
   // build the variant's trial-offset table now, so that dedisperse calls
   // (and graphs captured from them) allocate nothing
   const int v = plan_shape(plan, variant);
@@ -419,7 +431,7 @@ extern "C" int mdsm_plan_variant_channels(mdsm_plan plan, int variant, uint32_t 
 
 extern "C" int mdsm_plan_get_variant(mdsm_plan plan, int *variant) {
   MDSM_REQUIRE(plan && variant, MDSM_ERR_ARG, "null argument");
-  *variant = plan_variant(plan);
+  *variant = plan->kept_untuned ? 0 : plan_variant(plan);
   return MDSM_OK;
 }
 
@@ -445,7 +457,8 @@ extern "C" int mdsm_dedisperse(mdsm_plan plan, const void *d_in, uint64_t ld, fl
 namespace mdsm {
 
 // Time every tile variant of a plan on the given buffers: one warm-up launch,
-// then the best of three timed launches; t[v] < 0 where a variant does not fit.
+// then the best of three timed launches; t[v] < 0 where no form of a variant
+// fits.  t[0]: the untuned plan, where it launches what no number stands for.
 int plan_time_variants(mdsm_plan plan, const void *d_in, uint64_t ld, float *d_out,
                        hipStream_t s, std::vector<float> &t) {
   hipEvent_t e0, e1;
@@ -456,7 +469,9 @@ int plan_time_variants(mdsm_plan plan, const void *d_in, uint64_t ld, float *d_o
   t.assign(nv + 1, -1.0f);
   for (int v = 0; v <= nv; ++v) {
     plan->variant = v;
-    if (v == 0 && plan_shape(plan, 0) == plan_variant(plan)) continue;  // timed by its number
+    bool own;
+    const int shape = plan_shape(plan, v, &own);
+    if (!own || (v == 0 && shape != kDirectShape)) continue;  // timed by its own number
     if (mdsm_dedisperse(plan, d_in, ld, d_out, s) != MDSM_OK) continue;  // warm-up / LDS fit
     float vms = -1.0f;
     for (int rep = 0; rep < 3; ++rep) {
@@ -499,11 +514,10 @@ extern "C" int mdsm_plan_autotune(mdsm_plan plan, const void *d_in, uint64_t ld,
   if (rc != MDSM_OK) return rc;
   const int best = pick_variant(plan->dtype, t);
   MDSM_REQUIRE(best > 0, MDSM_ERR_ARG, "no tile variant fits this survey");
-  // t[0]: the untuned plan, where it launches no numbered shape
-  const bool untuned = t[0] >= 0.0f && t[0] <= t[best];
-  plan->variant = untuned ? 0 : best;
-  if (best_variant) *best_variant = plan_variant(plan);
-  if (best_ms) *best_ms = t[untuned ? 0 : best];
+  plan->kept_untuned = t[0] >= 0.0f && t[0] <= t[best];
+  plan->variant = plan->kept_untuned ? 0 : best;
+  if (best_variant) *best_variant = plan->variant;
+  if (best_ms) *best_ms = t[plan->variant];
   return MDSM_OK;
 }
 

@@ -120,23 +120,25 @@ static int batch_default(const mdsm_batch_s *b) {
 
 static int batch_variant(const mdsm_batch_s *b) { return b->variant ? b->variant : batch_default(b); }
 
-// The shape a launch uses: the variant that was set or tuned where it takes the
-// beams, or the default or one of its alternatives, whichever has the least
-// estimate for all beams' tiles (as untuned_shape).
-static int batch_shape(const mdsm_batch_s *b, int variant) {
+// The shape a launch uses: the form of the variant that was set or tuned, or
+// the default or one of its alternatives, whichever has the least estimate for
+// all beams' tiles (as untuned_shape; *own: see numbered_shape).
+static int batch_shape(const mdsm_batch_s *b, int variant, bool *own) {
   auto cost = [&](int shape) {
-    double tiles = 0.0, work = 0.0, outputs = 0.0;
+    double tiles = 0.0, work = 0.0, most = 0.0, outputs = 0.0;
     for (const auto &s : b->beams) {
       const double n = tile_count(b->dtype, shape, s.ndms, s.nsamp);
       tiles += n;
       work += n * s.nchans;
+      most = std::max(most, (double)s.nchans);
       outputs += (double)s.ndms * s.nsamp;
     }
-    return launch_estimate(b->dtype, shape, tiles, b->beams.size() == 1, work / tiles, outputs);
+    return launch_estimate(b->dtype, shape, tiles, b->beams.size() == 1, work / tiles, most, outputs);
   };
   std::vector<bool> fits(num_shapes(b->dtype) + 1);
   for (int i = 1; i < (int)fits.size(); ++i) fits[i] = batch_fits(b, i);
-  if (variant) return numbered_shape(b->dtype, variant, fits);
+  if (variant) return numbered_shape(b->dtype, variant, fits, cost, own);
+  *own = true;
   const int v = batch_default(b);
   int best = v;
   for (int n = 0, shape; (shape = other_shape(b->dtype, v, n)) != 0; ++n)
@@ -241,7 +243,8 @@ extern "C" int mdsm_batch_set_variant(mdsm_batch batch, int variant) {
 // from the caller's input into a scratch output allocated here, and a
 // shape's batch time is estimated as the sum of its beams' times scaled to
 // their full length; the three least estimates among the shapes that fit
-// every beam are then timed as one whole launch each, and the fastest kept.
+// every beam, and the number of the untuned launch, are then timed as one
+// whole launch each, and the fastest kept.
 extern "C" int mdsm_batch_autotune(mdsm_batch batch, const void *const *d_in, const uint64_t *ld,
                                    float *const *d_out_full, void *stream, int *best_variant,
                                    float *best_ms) {
@@ -263,6 +266,13 @@ extern "C" int mdsm_batch_autotune(mdsm_batch batch, const void *const *d_in, co
   std::vector<double> est(nv + 1, 0.0);
   std::vector<bool> ok(nv + 1, true);
   ok[0] = false;
+  // what each number launches here; -1 where it takes not all beams
+  std::vector<int> shape_of(nv + 1);
+  for (int v = 0; v <= nv; ++v) {
+    bool own;
+    const int shape = batch_shape(batch, v, &own);
+    shape_of[v] = own && batch_fits(batch, shape) ? shape : -1;
+  }
   int rc = MDSM_OK;
   for (uint32_t i = 0; i < nb && rc == MDSM_OK; ++i) {
     mdsm_survey_t probe = batch->beams[i];
@@ -275,7 +285,7 @@ extern "C" int mdsm_batch_autotune(mdsm_batch batch, const void *const *d_in, co
     mdsm_plan_destroy(p);
     const double scale = (double)batch->beams[i].nsamp / (double)probe.nsamp;
     for (int v = 1; v <= nv; ++v) {
-      if (t.size() <= (size_t)v || t[v] < 0.0f || !batch_fits(batch, v)) ok[v] = false;
+      if (t.size() <= (size_t)v || t[v] < 0.0f || shape_of[v] < 0) ok[v] = false;
       else est[v] += scale * t[v];
     }
   }
@@ -289,6 +299,11 @@ extern "C" int mdsm_batch_autotune(mdsm_batch batch, const void *const *d_in, co
     if (ok[u]) cand.push_back(u);
   std::sort(cand.begin(), cand.end(), [&](int a, int b) { return est[a] < est[b]; });
   if (cand.size() > 3) cand.resize(3);
+  for (int u = 1; u <= nv; ++u)
+    if (shape_of[u] >= 0 && shape_of[u] == shape_of[0]) {
+      if (std::find(cand.begin(), cand.end(), u) == cand.end()) cand.push_back(u);
+      break;
+    }
   const int keep_variant = batch->variant;
   hipStream_t s = as_stream(stream);
   hipEvent_t e0, e1;
@@ -327,7 +342,8 @@ extern "C" int mdsm_batch_bind(mdsm_batch batch, const void *const *d_in, const 
                                float *const *d_out) {
   MDSM_REQUIRE(batch && d_in && ld && d_out, MDSM_ERR_ARG, "null argument");
   const uint32_t nb = (uint32_t)batch->beams.size();
-  const int v = batch_shape(batch, batch->variant);
+  bool own;
+  const int v = batch_shape(batch, batch->variant, &own);
   const TileShape sh = variant_shape(batch->dtype, v);
   batch->h_desc.resize(nb);
   uint64_t items = 0;

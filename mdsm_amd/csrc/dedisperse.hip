@@ -2182,11 +2182,14 @@ static int stand_in(int dtype, int variant) {
   return 0;
 }
 
-int numbered_shape(int dtype, int variant, const std::vector<bool> &fits) {
+int numbered_shape(int dtype, int variant, const std::vector<bool> &fits, const std::function<double(int)> &cost,
+                   bool *own) {
+  const int narrow = narrow_variant(dtype, variant), other = stand_in(dtype, variant);
+  *own = true;
+  if (narrow && fits[narrow] && (!fits[variant] || cost(narrow) < cost(variant))) return narrow;
   if (fits[variant]) return variant;
-  for (const int other : {narrow_variant(dtype, variant), stand_in(dtype, variant)})
-    if (other && fits[other]) return other;
-  return variant;
+  *own = false;
+  return other && fits[other] ? other : variant;
 }
 
 // The shapes that may replace a default one where its tiles pad too much or
@@ -2211,14 +2214,15 @@ double tile_count(int dtype, int shape, uint32_t ndms, uint32_t nsamp) {
   return (double)((ndms + sh.td() - 1) / sh.td()) * ((nsamp + sh.tt() - 1) / sh.tt());
 }
 
-// Estimated time (us) of a launch of `tiles` tiles over nchans channels, for
-// the shapes that untuned launches choose between: the rounds of adds, and what
+// Estimated time (us) of a launch of `tiles` tiles over nchans channels (in the
+// mean of the tiles, `most` in the beam that has most), for the shapes that untuned launches choose between: the rounds of adds, and what
 // goes on beside them.
 //   Adds: every CU runs one (16 waves) or two workgroups of a shape at a time,
 //   so tiles take whole rounds of 256 or 512, each at the shape's full rate; a
-//   last round of up to 256 of two per CU, three quarters of one.  Tiles of
+//   last round of up to 256 of two per CU, three quarters of one (F32 nine
+//   tenths: 256 tiles of 32 trials 204 us, of 64 187, 320 channels).  Tiles of
 //   several beams (not equal) end at different times: half a round over the
-//   mean instead.  T adds/s measured at 512 to 1024 channels, 1920 trials x
+//   mean instead, and no less than the beam of most channels alone.  T adds/s measured at 512 to 1024 channels, 1920 trials x
 //   81920 samples; eight waves per workgroup 1.04 to 1.36 times as long per add,
 //   and 0.87 of all that where rows come from the caches (12 to 96 channels);
 //   0.4 us per channel at least however few tiles there are.  The word-per-add
@@ -2229,17 +2233,18 @@ double tile_count(int dtype, int shape, uint32_t ndms, uint32_t nsamp) {
 //   channels that decides: 64 channels x 4000 trials x 50000 samples 388 us in
 //   shape 20 against 427 in 22 (F16_PAIRS), 393 in 21 against 426 (U8); 96
 //   channels 548 against 559 and 546 against 555.
-double launch_estimate(int dtype, int shape, double tiles, bool equal, double nchans, double outputs) {
+double launch_estimate(int dtype, int shape, double tiles, bool equal, double nchans, double most, double outputs) {
   const int nv = num_variants(dtype);
   const TileShape sh = variant_shape(dtype, shape);
   const double work = (double)sh.td() * sh.tt();
   const bool word = (dtype == MDSM_F32 && shape == 8) || (dtype == MDSM_F16 && shape == 15) ||
                     (dtype == MDSM_F16_PAIRS && shape == 15);
   const bool pair_sums = (dtype == MDSM_U8 || dtype == MDSM_F16_PAIRS) && shape >= 16 && shape <= 21;
-  double per_channel;
+  // time of one round's adds and of all of them
+  double round, adds;
   if (word) {
-    per_channel = dtype == MDSM_F32 ? std::max(0.6, 1e-6 * tiles * work / 16.0)
-                                    : std::max(0.5, 1e-6 * tiles * work / 25.0);
+    round = dtype == MDSM_F32 ? 0.6 : 0.5;
+    adds = std::max(round * most, 1e-6 * tiles * work / (dtype == MDSM_F32 ? 16.0 : 25.0) * nchans);
   } else {
     const bool pair_windows = shape == 22 || (shape == nv + 1 && (dtype == MDSM_U8 || dtype == MDSM_F16_PAIRS));
     const double wide = dtype == MDSM_F32 ? 39.0 : (pair_windows ? 42.0 : (dtype == MDSM_U8 ? 34.5 : 36.5));
@@ -2251,13 +2256,20 @@ double launch_estimate(int dtype, int shape, double tiles, bool equal, double nc
       rate = dtype == MDSM_U8 ? 36.5 : (shape == 20 ? 37.5 : (shape == 21 ? 33.0 : 31.0));
       slots = 512.0;
     }
+    // one workgroup alone on its CU, of two that share it
+    const double lone = slots > 256.0 ? (dtype == MDSM_F32 ? 0.9 : 0.75) : 1.0;
     double rounds = ceil(tiles / slots);
-    if (slots > 256.0 && tiles <= slots * rounds - 256.0) rounds -= 0.25;
-    if (!equal && rounds > 1.0) rounds = tiles / slots + 0.5;
-    per_channel = std::max(0.4, 0.87e-6 * rounds * slots * work / rate);
+    if (tiles <= slots * rounds - 256.0) rounds -= 1.0 - lone;
+    round = 0.87e-6 * slots * work / rate;
+    if (!equal) {
+      const double mean = tiles / slots + 0.5;
+      adds = round * std::max(lone * most, (rounds > 1.0 ? mean : std::min(mean, rounds)) * nchans);
+    } else {
+      adds = std::max(0.4, rounds * round) * nchans;
+    }
   }
   const double start = word ? 3.5 : (pair_sums ? 4.0 : 6.0), store = word ? 0.5 : (pair_sums ? 0.47 : 0.7);
-  return 3.0 + std::max(start, store * 1e-6 * outputs) + nchans * per_channel;
+  return 3.0 + std::max(start, store * 1e-6 * outputs) + adds;
 }
 
 // The shape an untuned plan launches for its tile variant `nominal`: the least
@@ -2282,7 +2294,7 @@ int untuned_shape(int dtype, int nominal, const std::vector<bool> &fits, uint32_
                   uint32_t nsamp) {
   const double outputs = (double)ndms * nsamp;
   auto tiles = [&](int shape) { return tile_count(dtype, shape, ndms, nsamp); };
-  auto cost = [&](int shape) { return launch_estimate(dtype, shape, tiles(shape), true, nchans, outputs); };
+  auto cost = [&](int shape) { return launch_estimate(dtype, shape, tiles(shape), true, nchans, nchans, outputs); };
   int best = nominal;
   for (int n = 0, shape; (shape = other_shape(dtype, nominal, n)) != 0; ++n) {
     if (!fits[shape]) continue;

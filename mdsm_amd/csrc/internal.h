@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <functional>
 #include <vector>
 
 #include "mdsm_abi.h"
@@ -84,16 +85,17 @@ int fallback_variant(int dtype, int n);
 constexpr int kDirectShape = 0;
 int num_shapes(int dtype);
 int narrow_variant(int dtype, int variant);
-// What a variant set by number launches: its shape, the eight-wave form, or a
-// shape that takes every survey which the number took before it, the first
-// that takes the survey (`fits`, by shape); else the variant itself, which is
-// refused.
-int numbered_shape(int dtype, int variant, const std::vector<bool> &fits);
+// What a variant set by number launches: of its forms that take the survey
+// (`fits`, by shape) the one of less cost, as untuned launches choose; else
+// (*own: false) a shape that takes every survey which the number took before
+// it, or the variant itself, which is refused.
+int numbered_shape(int dtype, int variant, const std::vector<bool> &fits, const std::function<double(int)> &cost,
+                   bool *own);
 // Shapes that may replace a default one, a shape's tiles for a survey, and the
 // estimated time of a launch of a number of them (us).
 int other_shape(int dtype, int nominal, int n);
 double tile_count(int dtype, int shape, uint32_t ndms, uint32_t nsamp);
-double launch_estimate(int dtype, int shape, double tiles, bool equal, double nchans, double outputs);
+double launch_estimate(int dtype, int shape, double tiles, bool equal, double nchans, double most, double outputs);
 // The shape an untuned plan launches where its tile variant is `nominal`.
 int untuned_shape(int dtype, int nominal, const std::vector<bool> &fits, uint32_t nchans, uint32_t ndms,
                   uint32_t nsamp);
