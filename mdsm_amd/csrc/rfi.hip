@@ -109,14 +109,14 @@ __global__ __launch_bounds__(RFI_NT) void channel_flag_kernel(const float *__res
 }
 
 // A workgroup per `per` (at most 64) consecutive blocks of a channel: every
-// wave reads all their flags, one per lane, and the whole workgroup fills the
-// flagged blocks one after the other.  Bound by launching where nearly no block
-// is flagged (131072 blocks of 1024: 33 us with a workgroup each, 4.5 us in
-// groups of 16) and by stores where many are, so a workgroup's blocks hold
-// about 16384 samples: all of 4 rows of 2^22 samples in blocks of 65536 take 12
-// us (one wave per 64 blocks, whatever their length: 1647).  While fewer than
-// 1024 workgroups are left, groups shrink to one block (2^20 samples of one row
-// 3.4 us, 4.9 in groups of 16).
+// wave reads all their flags, one per lane; the whole workgroup fills the
+// flagged blocks one after the other, or each wave every fourth of them where a
+// block is shorter than a workgroup.  Bound by launching where nearly no block
+// is flagged (131072 blocks of 1024: 33 us with a workgroup each, 3.5 us in
+// groups of 64) and by stores where many are, so groups shrink until there are
+// 2048 workgroups or one per block: all of 4 rows of 2^22 samples in blocks of
+// 65536 take 12 us (one wave per 64 blocks, whatever their length: 1647), 2^20
+// samples of one row in blocks of 1024 3.4 us (4.9 in groups of 16).
 __global__ __launch_bounds__(RFI_NT) void channel_clip_kernel(float *__restrict__ x, uint64_t ld,
                                                               uint64_t col0, uint64_t n,
                                                               const double *__restrict__ fitted,
@@ -126,13 +126,16 @@ __global__ __launch_bounds__(RFI_NT) void channel_clip_kernel(float *__restrict_
   const uint64_t b0 = (uint64_t)blockIdx.x * per;
   unsigned long long set =
       __ballot(lane < per && b0 + lane < nb && flags[(uint64_t)c * nb + b0 + lane] != 0);
+  const bool split = cb < RFI_NT;
+  if (split) set &= 0x1111111111111111ull << (threadIdx.x >> 6);
   if (set == 0ull) return;
+  const uint32_t from = split ? lane : threadIdx.x, step = split ? 64u : RFI_NT;
   const float bp = __double2float_rz(fitted[c]);
   float *row = x + (uint64_t)c * ld + col0;
   while (set) {
     const uint64_t start = (b0 + (uint64_t)(__ffsll((long long)set) - 1)) * cb;
     const uint64_t end = start + cb <= n ? start + cb : n;
-    for (uint64_t s = start + threadIdx.x; s < end; s += RFI_NT) row[s] = bp;
+    for (uint64_t s = start + from; s < end; s += step) row[s] = bp;
     set &= set - 1ull;
   }
 }
@@ -203,8 +206,7 @@ int launch_channel_flag(const float *x, uint64_t ld, uint32_t nchans, uint64_t c
 int launch_channel_clip(float *x, uint64_t ld, uint32_t nchans, uint64_t col0, uint64_t n,
                         const double *fitted, uint32_t cb, const uint8_t *flags, hipStream_t s) {
   const uint32_t nb = (uint32_t)((n + cb - 1) / cb);
-  const uint64_t spread = std::max<uint64_t>(1u, (uint64_t)nb * nchans / 1024u);
-  const uint32_t per = (uint32_t)std::min<uint64_t>(spread, std::min(64u, std::max(1u, 16384u / cb)));
+  const uint32_t per = (uint32_t)std::min<uint64_t>(64u, std::max<uint64_t>(1u, (uint64_t)nb * nchans / 2048u));
   hipLaunchKernelGGL(channel_clip_kernel, dim3((uint32_t)(((uint64_t)nb + per - 1) / per), nchans), dim3(RFI_NT), 0,
                      s, x, ld, col0, n, fitted, cb, nb, per, flags);
   MDSM_HIP(hipGetLastError());
