@@ -142,7 +142,7 @@ static int batch_shape(const mdsm_batch_s *b, int variant, bool *own) {
   const int v = batch_default(b);
   int best = v;
   for (int n = 0, shape; (shape = other_shape(b->dtype, v, n)) != 0; ++n)
-    if (fits[shape] && (b->dtype != MDSM_F16 || shape != 15) && cost(shape) < cost(best)) best = shape;
+    if (fits[shape] && cost(shape) < kBetter * cost(best)) best = shape;
   return best;
 }
 

@@ -1908,14 +1908,22 @@ __global__ __launch_bounds__(256) void dedisp_direct_kernel(const void *__restri
   typedef int32_t i32x16 __attribute__((ext_vector_type(16)));
   typedef __attribute__((address_space(4))) const i32x16 const_i32x16;
   const uint32_t lane = threadIdx.x & 63u;
-  // the pairs (time block, four trials) in that order, an eighth of them to
-  // each XCD (workgroup IDs are dealt round-robin): its time blocks run through
-  // all their trials one after the other, whose rows stay in its L2, and however
-  // few time blocks there are, no XCD idles
-  const uint32_t ndg = (ndms + 3u) / 4u, item = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  // An eighth (give or take one) of the time blocks to each XCD (workgroup IDs
+  // are dealt round-robin), which runs through all their trials one after the
+  // other, so that their rows stay in its L2; of the pairs (time block, four
+  // trials) in that order where an XCD's blocks are more than it can hold at a
+  // time (256 workgroups), so that few time blocks of many trials leave no XCD
+  // idle (15 trials x 5 blocks split: 78 us instead of 57; 8000 x 1 not split: 2.2
+  // ms instead of 0.3).
+  const uint32_t ndg = (ndms + 3u) / 4u, ntb = (nsamp + 255u) / 256u, x = blockIdx.x & 7u;
+  const uint32_t unit = (ntb + 7u) / 8u * ndg <= 256u ? ndg : 1u, units = unit > 1u ? ntb : ntb * ndg;
+  const uint32_t first = (units / 8u * x + units % 8u * x / 8u) * unit;
+  const uint32_t past = (units / 8u * (x + 1u) + units % 8u * (x + 1u) / 8u) * unit;
+  const uint32_t item = first + (blockIdx.x >> 3);
+  if (item >= past) return;
   const uint32_t tb = item / ndg;
   const uint32_t d = uniform((item - tb * ndg) * 4u + (threadIdx.x >> 6));
-  if (d >= ndms || tb * 256u >= nsamp) return;
+  if (d >= ndms) return;
   const uint32_t t = min((tb * 64u + lane) * 4u, nsamp - 4u);
   constexpr uint32_t SZ = MODE == MDSM_F32 ? 4u : (MODE == MDSM_U8 ? 1u : 2u);
   const const_i32x16 *tab = (const const_i32x16 *)(uintptr_t)(dtab + (uint64_t)d * cpad);
@@ -1984,10 +1992,12 @@ __global__ __launch_bounds__(256) void direct_table_kernel(const int32_t *__rest
   dtab[(uint64_t)d * cpad + c] = table[(uint64_t)min(c, nchans - 1u) * ndms + d];
 }
 inline uint32_t direct_pad(uint32_t nchans) { return (nchans + 15u) & ~15u; }
-// Workgroups: 256 samples of four trials each, a multiple of 8 of them.
+// Workgroups (256 samples of four trials each), as many to each XCD as its
+// share can be.
 inline uint64_t direct_grid(uint32_t ndms, uint32_t nsamp) {
-  const uint64_t items = (((uint64_t)nsamp + 255u) / 256u) * (((uint64_t)ndms + 3u) / 4u);
-  return (items + 7u) / 8u * 8u;
+  const uint64_t ntb = ((uint64_t)nsamp + 255u) / 256u, ndg = ((uint64_t)ndms + 3u) / 4u;
+  const uint64_t whole = (ntb + 7u) / 8u * ndg;
+  return 8u * (whole <= 256u ? whole : (ntb * ndg + 7u) / 8u);
 }
 // Rows of four samples or more (a lane's), whose grid IDs have 31 bits.
 inline bool direct_takes(uint32_t ndms, uint32_t nsamp) { return nsamp >= 4u && direct_grid(ndms, nsamp) < (1ull << 31); }
@@ -2186,7 +2196,7 @@ int numbered_shape(int dtype, int variant, const std::vector<bool> &fits, const 
                    bool *own) {
   const int narrow = narrow_variant(dtype, variant), other = stand_in(dtype, variant);
   *own = true;
-  if (narrow && fits[narrow] && (!fits[variant] || cost(narrow) < cost(variant))) return narrow;
+  if (narrow && fits[narrow] && (!fits[variant] || cost(narrow) < kBetter * cost(variant))) return narrow;
   if (fits[variant]) return variant;
   *own = false;
   return other && fits[other] ? other : variant;
@@ -2205,8 +2215,7 @@ int other_shape(int dtype, int nominal, int n) {
     if (nominal == 22) return after22[n];
     return nominal == 20 ? after20[n] : (nominal == 21 ? after20[n + 1] : (nominal == 16 ? after20[n + 2] : 0));
   }
-  if (nominal != 12) return 0;
-  return n == 0 ? nv + 1 : (n == 1 ? (dtype == MDSM_F32 ? 8 : 15) : 0);
+  return n == 0 && nominal == 12 ? nv + 1 : 0;
 }
 
 double tile_count(int dtype, int shape, uint32_t ndms, uint32_t nsamp) {
@@ -2222,17 +2231,19 @@ double tile_count(int dtype, int shape, uint32_t ndms, uint32_t nsamp) {
 //   last round of up to 256 of two per CU, three quarters of one (F32 nine
 //   tenths: 256 tiles of 32 trials 204 us, of 64 187, 320 channels).  Tiles of
 //   several beams (not equal) end at different times: half a round over the
-//   mean instead, and no less than the beam of most channels alone.  T adds/s measured at 512 to 1024 channels, 1920 trials x
-//   81920 samples; eight waves per workgroup 1.04 to 1.36 times as long per add,
-//   and 0.87 of all that where rows come from the caches (12 to 96 channels);
-//   0.4 us per channel at least however few tiles there are.  The word-per-add
-//   shapes fit no rounds: 16 (F32) or 25 T adds/s, 0.6 or 0.5 us at least.
+//   mean instead, and no less than the beam of most channels alone.  T adds/s
+//   of the windows measured at 512 to 1024 channels, 1920 trials x 81920 samples,
+//   and 0.87 of their time where rows come from the caches (32 to 320 channels);
+//   eight waves per workgroup 1.04 to 1.5 times as long per add; 0.4 us per
+//   channel at least however few tiles there are.  The word-per-add shapes fit no
+//   rounds: 16 (F32) or 25 T adds/s, 0.6 or 0.5 us at least.
 //   Beside them: a window tile's workgroups fill their CUs alone, so nothing
-//   adds while they store: 0.7 us per million outputs, 6 at least, against 0.47
-//   (4) of the pair-sum shapes and 0.5 (3.5) of the word-per-add ones.  At few
+//   adds while they store: 0.8 us per million outputs, 7 to 9 at least, 0.7 (F32
+//   0.85) and 4 to 7.5 of two eight-wave ones per CU, 0.35 (4) of the pair-sum
+//   shapes, 0.5 (3.5) of the word-per-add ones.  At few
 //   channels that decides: 64 channels x 4000 trials x 50000 samples 388 us in
-//   shape 20 against 427 in 22 (F16_PAIRS), 393 in 21 against 426 (U8); 96
-//   channels 548 against 559 and 546 against 555.
+//   shape 20 against 427 in 22 (F16_PAIRS), 393 in 21 against 426 (U8); 32 x 160
+//   x 256000 F16 60 us in eight waves against 81.
 double launch_estimate(int dtype, int shape, double tiles, bool equal, double nchans, double most, double outputs) {
   const int nv = num_variants(dtype);
   const TileShape sh = variant_shape(dtype, shape);
@@ -2240,27 +2251,31 @@ double launch_estimate(int dtype, int shape, double tiles, bool equal, double nc
   const bool word = (dtype == MDSM_F32 && shape == 8) || (dtype == MDSM_F16 && shape == 15) ||
                     (dtype == MDSM_F16_PAIRS && shape == 15);
   const bool pair_sums = (dtype == MDSM_U8 || dtype == MDSM_F16_PAIRS) && shape >= 16 && shape <= 21;
-  // time of one round's adds and of all of them
-  double round, adds;
+  // time of one round's adds and of all of them, and beside them
+  double round, adds, start = 3.5, store = 0.5;
   if (word) {
     round = dtype == MDSM_F32 ? 0.6 : 0.5;
     adds = std::max(round * most, 1e-6 * tiles * work / (dtype == MDSM_F32 ? 16.0 : 25.0) * nchans);
   } else {
     const bool pair_windows = shape == 22 || (shape == nv + 1 && (dtype == MDSM_U8 || dtype == MDSM_F16_PAIRS));
     const double wide = dtype == MDSM_F32 ? 39.0 : (pair_windows ? 42.0 : (dtype == MDSM_U8 ? 34.5 : 36.5));
-    double rate = wide, slots = 256.0;
+    double rate = wide / 0.87, slots = 256.0;
+    start = pair_windows ? 9.0 : (dtype == MDSM_F32 ? 7.0 : 8.5), store = 0.8;
     if (shape > nv) {
-      rate = wide / (pair_windows ? 1.36 : (dtype == MDSM_F32 ? 1.17 : 1.04));
+      rate /= pair_windows ? 1.5 : (dtype == MDSM_F32 ? 1.17 : 1.04);
       slots = 512.0;
+      start -= dtype == MDSM_F32 ? 3.0 : (pair_windows ? 1.5 : 2.0);
+      if (!pair_windows) store = dtype == MDSM_F32 ? 0.85 : 0.7;
     } else if (pair_sums) {
-      rate = dtype == MDSM_U8 ? 36.5 : (shape == 20 ? 37.5 : (shape == 21 ? 33.0 : 31.0));
+      rate = dtype == MDSM_U8 ? 40.5 : (shape == 20 ? 39.5 : (shape == 21 ? 34.5 : 32.5));
       slots = 512.0;
+      start = 4.0, store = 0.35;
     }
     // one workgroup alone on its CU, of two that share it
     const double lone = slots > 256.0 ? (dtype == MDSM_F32 ? 0.9 : 0.75) : 1.0;
     double rounds = ceil(tiles / slots);
     if (tiles <= slots * rounds - 256.0) rounds -= 1.0 - lone;
-    round = 0.87e-6 * slots * work / rate;
+    round = 1e-6 * slots * work / rate;
     if (!equal) {
       const double mean = tiles / slots + 0.5;
       adds = round * std::max(lone * most, (rounds > 1.0 ? mean : std::min(mean, rounds)) * nchans);
@@ -2268,7 +2283,6 @@ double launch_estimate(int dtype, int shape, double tiles, bool equal, double nc
       adds = std::max(0.4, rounds * round) * nchans;
     }
   }
-  const double start = word ? 3.5 : (pair_sums ? 4.0 : 6.0), store = word ? 0.5 : (pair_sums ? 0.47 : 0.7);
   return 3.0 + std::max(start, store * 1e-6 * outputs) + adds;
 }
 
@@ -2279,16 +2293,20 @@ double launch_estimate(int dtype, int shape, double tiles, bool equal, double nc
 //   264 us in two such tiles, 205 in one of 48; 32 trials x 600000 samples x 512
 //   channels F32: 399 against 598 us; 856 channels x 1222 trials x 15994
 //   samples U8, 260 tiles of 16 waves: 540 against 766 us).
-//   F16's shape 15 where fewer than 40 channels meet fewer than 128 window tiles,
-//   which leave half of the CUs idle, and is not weighed otherwise (16 channels x
-//   200 trials x 20000 samples: 13 us against 16).
-//   Direct kernel, up to 5.3 million outputs of rows padded to 256 samples: 7.5
-//   (F32), 6 (F16), 11.5 (U8) or 5.5 T adds/s (pair sums), 4 us to start and 0.8
-//   us per million outputs stored (256 channels x 64 trials x 8192 samples F32:
-//   19 against 132 us; 512 x 256 x 12000: 205 against 257; x 16384: 274 against
-//   257; 646 x 890 x 22 F16: 31 against 300).  More outputs of few trials read
-//   their rows from HBM for every four of them (421 channels x 6 trials x 10^6
-//   samples F16_PAIRS: 621 us against 540).
+//   (by 1 % at least: 514 channels x 700 trials x 19652 samples U8, 234 against
+//   236 us by the estimate, 260 against 222 in truth).
+//   The word-per-add shapes for F16 rows of fewer than 4 samples, and where few
+//   channels (13 of F32, 40 of F16) meet fewer than 128 window tiles, which leave
+//   half of the CUs idle (16 channels x 200 trials x 20000 samples F16: 13 us
+//   against 16); with more tiles their short rows store slower (3 channels x 6820
+//   trials x 311399 samples F32: 3.0 ms against 2.2).
+//   Direct kernel, up to 5.3 million outputs of rows padded to 256 samples (2.3
+//   to 4.3 of less than 32 trials): 8.5 (F32), 6.6 (F16), 12 (U8) or 6.4 T adds/s
+//   (pair sums), 4 us to start and 0.8 us per million outputs stored (256 channels
+//   x 64 trials x 8192 samples F32: 18 against 132 us; 512 x 256 x 12000: 205
+//   against 257; 646 x 890 x 22 F16: 31 against 300).  More outputs of few trials
+//   read their rows from HBM for every four of them (421 channels x 6 trials x
+//   10^6 samples F16_PAIRS: 621 us against 540).
 // `fits` holds the shapes that take the survey.
 int untuned_shape(int dtype, int nominal, const std::vector<bool> &fits, uint32_t nchans, uint32_t ndms,
                   uint32_t nsamp) {
@@ -2296,19 +2314,18 @@ int untuned_shape(int dtype, int nominal, const std::vector<bool> &fits, uint32_
   auto tiles = [&](int shape) { return tile_count(dtype, shape, ndms, nsamp); };
   auto cost = [&](int shape) { return launch_estimate(dtype, shape, tiles(shape), true, nchans, nchans, outputs); };
   int best = nominal;
-  for (int n = 0, shape; (shape = other_shape(dtype, nominal, n)) != 0; ++n) {
-    if (!fits[shape]) continue;
-    if (dtype == MDSM_F16 && shape == 15) {
-      if (nchans < 40u && tiles(nominal) < 128.0) best = shape;
-    } else if (cost(shape) < cost(best)) {
-      best = shape;
-    }
+  for (int n = 0, shape; (shape = other_shape(dtype, nominal, n)) != 0; ++n)
+    if (fits[shape] && cost(shape) < kBetter * cost(best)) best = shape;
+  if ((dtype == MDSM_F32 || dtype == MDSM_F16) && nominal == 12) {
+    const int word = dtype == MDSM_F32 ? 8 : 15;
+    const bool few = tiles(nominal) < 128.0 && nchans < (dtype == MDSM_F32 ? 13u : 40u);
+    if (fits[word] && (few || (dtype == MDSM_F16 && nsamp < 4u))) best = word;
   }
+  const double rate = dtype == MDSM_F32 ? 8.5 : dtype == MDSM_F16 ? 6.6 : dtype == MDSM_U8 ? 12.0 : 6.4;
   const double padded = (double)ndms * ((nsamp + 255u) / 256u * 256u);
-  if (direct_takes(ndms, nsamp) && padded <= 5.3e6) {
-    const double rate = dtype == MDSM_F32 ? 7.5 : dtype == MDSM_F16 ? 6.0 : dtype == MDSM_U8 ? 11.5 : 5.5;
-    if (4.0 + 0.8e-6 * outputs + 1e-6 * nchans * padded / rate < cost(best)) return kDirectShape;
-  }
+  const double direct = 4.0 + 0.8e-6 * outputs + 1e-6 * nchans * padded / rate;
+  const double limit = ndms >= 32u ? 5.3e6 : 0.36e6 * rate;
+  if (direct_takes(ndms, nsamp) && padded <= limit && direct < cost(best)) return kDirectShape;
   return best;
 }
 

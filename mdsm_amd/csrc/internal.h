@@ -91,6 +91,8 @@ int narrow_variant(int dtype, int variant);
 // it, or the variant itself, which is refused.
 int numbered_shape(int dtype, int variant, const std::vector<bool> &fits, const std::function<double(int)> &cost,
                    bool *own);
+// What another shape's estimate has to fall to, to be launched instead.
+constexpr double kBetter = 0.99;
 // Shapes that may replace a default one, a shape's tiles for a survey, and the
 // estimated time of a launch of a number of them (us).
 int other_shape(int dtype, int nominal, int n);

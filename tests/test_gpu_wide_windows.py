@@ -1,9 +1,9 @@
 """GPU parity of the 16-wave register windows, which surveys of whole rounds of
-their tiles (64 trials x 1280 samples, 256 at a time) take: around a DM tile,
-around a channel block (12 of F32 and of pair sums, 16 of F16 and U8) and its
-double, as plans and in both launch forms of a batch; and of the shape that an
-untuned plan falls back to on a delay spread that no window holds, with more
-outputs than the kernel without tiles takes.  Against the oracle bit for bit."""
+their tiles (64 trials x 1280 samples, 256 at a time) take: around a DM tile
+and around channel blocks (12 of F32 and of pair sums, 16 of F16 and U8), as
+plans and in both launch forms of a batch; and of the shape that an untuned
+plan falls back to on a delay spread that no window holds, with more outputs
+than the kernel without tiles takes.  Against the oracle bit for bit."""
 import numpy as np
 import pytest
 
@@ -27,10 +27,17 @@ def data(dtype, C, ld, t, N):
     return x, (O.dedisperse_f16_pairs if dtype == abi.F16_PAIRS else O.dedisperse_f16)(x, t, N)
 
 
-@pytest.mark.parametrize("C,M,N", [(1, 63, TILES - 3), (11, 64, TILES), (12, 63, TILES - 1279), (13, 64, TILES - 1),
-                                   (16, 64, TILES - 3), (17, 127, TILES - 640), (24, 128, TILES - 3), (33, 64, TILES - 5)])
-@pytest.mark.parametrize("dtype,number,block", [(abi.F32, 12, 12), (abi.F16, 12, 16), (abi.U8, 2, 16), (abi.U8, 22, 12),
-                                                (abi.F16_PAIRS, 22, 12)])
+# whole rounds of 200 or 256 tiles, at channel counts (around multiples of the
+# block) where 64 trials per tile are the faster form
+CASES = [(abi.F32, 12, 12, C, M, 200 * 1280 - 3) for C, M in ((36, 63), (37, 64), (47, 64))]
+CASES += [(d, v, 16, C, M, N) for d, v in ((abi.F16, 12), (abi.U8, 2))
+          for C, M, N in ((128, 63, TILES - 3), (129, 64, TILES), (143, 64, TILES - 1279), (128, 128, TILES - 5))]
+CASES += [(d, 22, 12, C, M, N) for d in (abi.U8, abi.F16_PAIRS)
+          for C, M, N in ((1, 63, TILES - 3), (11, 64, TILES), (12, 63, TILES - 1279), (13, 64, TILES - 1),
+                          (24, 128, TILES - 3), (25, 127, TILES - 640))]
+
+
+@pytest.mark.parametrize("dtype,number,block,C,M,N", CASES)
 def test_wide_windows_bitexact(dtype, number, block, C, M, N):
     s = abi.Survey.make(1500.0, -300.0 / C, C, 64e-6, 0.0, 0.015, M, N)
     t, S = abi.delay_table(s)
