@@ -448,7 +448,6 @@ struct WindowCode {
   }
 };
 
-//
 // A workgroup is NW waves: 16 (64 trials, all 160 KB of a CU's LDS) stage and
 // widen a row for twice the trials and meet at half the barriers per add of 8
 // (32 trials, 80 KB): F32 40.5 against 34.6 T adds/s, F16 37.7 against 36.5,
@@ -611,7 +610,7 @@ template <typename T>
 struct IsWindow : std::false_type {};
 template <int MODE, int NW>
 struct IsWindow<WindowTile<MODE, NW>> : std::true_type {};
-// Threads per workgroup: four waves, or the window tiles' eight.
+// Threads per workgroup: four waves, or the window tiles' 16 or eight.
 template <typename T>
 constexpr int tile_threads() {
   if constexpr (IsWindow<T>::value) return T::THREADS;

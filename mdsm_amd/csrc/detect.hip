@@ -383,7 +383,8 @@ __device__ __forceinline__ float from_next_lane(float x) {
 // E >= |x| over a level's window of w samples, the FP32 sum lies within
 // 6 * 2^-24 w E of the FP64 one, and the FP64 test needs
 // S >= w m + thresh sd sqrt(w) (1 - 2^-40), whose FP32 form is off by less
-// than 8 * 2^-24 of its terms; slack covers both twice over.  The compare is
+// than 8 * 2^-24 of its terms; slack covers the sum's rounding 1.33 times and
+// the terms' twice.  The compare is
 // written so that a NaN or an overflow on either side passes.
 __device__ __forceinline__ bool screen_runs(const float (&x)[DW_R], double m, double sd, int nwidths,
                                             float thresh) {
@@ -437,8 +438,8 @@ __device__ __forceinline__ bool screen_runs(const float (&x)[DW_R], double m, do
 // issue at twice the rate, one DPP move instead of two), so it pays while
 // most waves hold no candidate: launch_detect takes it from a threshold of
 // 4 on (noise passes in about one wave in ten there, in one of 10^5 at 6);
-// at 3 nearly every wave does.  4096 rows of 2^17 samples at 6 sigma: 400 us
-// (5.4 TB/s read), 617 us with FP64 levels and 4-byte loads everywhere.  One
+// at 3 nearly every wave does.  4096 rows of 2^17 samples at 6 sigma: 320 us
+// (6.7 TB/s read), 617 us with FP64 levels and 4-byte loads everywhere.  One
 // reservation per wave instead of one per sample position matters where
 // candidates are many: at 3 sigma (4.2 million) 6.4 ms, 35 ms before.
 template <bool SCREEN>
